@@ -98,32 +98,148 @@ template <> struct Geo<float> {
   static __device__ __forceinline__ float w(const P& a) { return __uint_as_float(a.w); }
 };
 
+// FP64 elementary functions of the pair passes, which are bound by their
+// instructions (and next by L1 lookups, two an entry).  The library's
+// versions carry the special cases of their whole domains (denormals,
+// large-argument reduction, division fix-up) into every list entry: the RGL
+// force pass took about 230 vector instructions an entry with them and takes
+// 112 with these, 60.7 -> 43.9 us a launch on 97,092 atoms (density pass
+// 50.7 -> 34.2 us).  These take the arguments the passes produce, without
+// branches; polynomials are interpolations at Chebyshev nodes (their own
+// error below 4e-17 relative), the last operation of each is the one that
+// rounds.  Largest errors in ulps: rcp 0.50, sqrt 0.50, 1/sqrt 0.99, exp
+// 1.13, sin 1.9, cos 1.3 below 1.4 (absolute 1.7e-16 at pi/2), pow 2.0; the
+// forces of a Cu crystal and of a gas against long double are no further off
+// than before (3.25e-15 -> 3.23e-15, 3.15e-15 -> 2.88e-15).
+namespace f64 {
+// a constant in scalar registers: left to itself the compiler keeps the
+// polynomials' coefficients in vector registers and copies each one before
+// the fused multiply-add that overwrites it
+__device__ __forceinline__ double sc(double c) {
+  asm("" : "+s"(c));
+  return c;
+}
+// 1/x, |x| normal: the hardware estimate (within 3e-8) and one third-order
+// step (x = 0 or infinite gives NaN, where 1/x gives infinity or 0)
+__device__ __forceinline__ double rcp(double x) {
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
+}
+// r = sqrt(d2), ir = 1/sqrt(d2) for normal d2 > 0 (d2 = 0: NaN, as inf * 0 of
+// the quotients it takes part in): the hardware estimate with one third-order
+// step, then one correction of r against d2
+__device__ __forceinline__ void sqrt_rsqrt(double d2, double& r, double& ir) {
+  const double y = __builtin_amdgcn_rsq(d2);
+  const double e = fma(-(d2 * y), y, 1.0);
+  ir = fma(y * e, fma(e, 0.375, 0.5), y);
+  const double s = d2 * ir;
+  r = fma(fma(-s, s, d2), 0.5 * ir, s);
+}
+// 2^n (1 + r + r^2 ...): e**r for |r| <= ln2/2 by degree 11, scaled
+__device__ __forceinline__ double exp_tail(double r, double n) {
+  double q = sc(0x1.af2391d7f5e6cp-26);
+  q = fma(q, r, sc(0x1.288060f149570p-22));
+  q = fma(q, r, sc(0x1.71de17d5ef6f3p-19));
+  q = fma(q, r, sc(0x1.a019c98e708e7p-16));
+  q = fma(q, r, sc(0x1.a01a01a4b5f72p-13));
+  q = fma(q, r, sc(0x1.6c16c173948e7p-10));
+  q = fma(q, r, sc(0x1.1111111110e68p-7));
+  q = fma(q, r, sc(0x1.5555555554cb0p-5));
+  q = fma(q, r, sc(0x1.5555555555555p-3));
+  q = fma(q, r, 0.5);
+  return __builtin_amdgcn_ldexp(1.0 + fma(r * r, q, r), (int)n);
+}
+// exp(x), x = n ln2 + r, for |x| < 1e15; underflow to 0 and overflow to
+// infinity come from the scaling
+__device__ __forceinline__ double exp(double x) {
+  const double n = rint(x * 0x1.71547652b82fep+0);
+  return exp_tail(fma(-n, 0x1.a39ef35793c76p-33, fma(-n, 0x1.62e42fee00000p-1, x)), n);
+}
+// exp(x + xl), |xl| << |x|
+__device__ __forceinline__ double exp(double x, double xl) {
+  const double n = rint(x * 0x1.71547652b82fep+0);
+  return exp_tail(fma(-n, 0x1.62e42fee00000p-1, x) + fma(-n, 0x1.a39ef35793c76p-33, xl), n);
+}
+// sine and cosine of y in [0, pi/2]
+__device__ __forceinline__ double cos_q1(double y) {
+  const double z = y * y;
+  double p = sc(-0x1.5eeafc14774b8p-53);
+  p = fma(p, z, sc(0x1.ae5a5d377edf5p-45));
+  p = fma(p, z, sc(-0x1.9396fdb46f278p-37));
+  p = fma(p, z, sc(0x1.1eed8ea6c7954p-29));
+  p = fma(p, z, sc(-0x1.27e4fb771a86dp-22));
+  p = fma(p, z, sc(0x1.a01a01a019783p-16));
+  p = fma(p, z, sc(-0x1.6c16c16c16c13p-10));
+  p = fma(p, z, sc(0x1.5555555555555p-5));
+  p = fma(p, z, -0.5);
+  return fma(p, z, 1.0);
+}
+__device__ __forceinline__ double sin_q1(double y) {
+  const double z = y * y;
+  double p = sc(0x1.89a4866f527ebp-49);
+  p = fma(p, z, sc(-0x1.ae5138c1216b3p-41));
+  p = fma(p, z, sc(0x1.6124015b5ee3ap-33));
+  p = fma(p, z, sc(-0x1.ae6455a1d7087p-26));
+  p = fma(p, z, sc(0x1.71de3a5456716p-19));
+  p = fma(p, z, sc(-0x1.a01a01a018aadp-13));
+  p = fma(p, z, sc(0x1.1111111111107p-7));
+  p = fma(p, z, sc(-0x1.5555555555555p-3));
+  return fma(y * z, p, y);
+}
+// x**y for finite x > 0: log x = 2 atanh((m-1)/(m+1)) + e ln2 as a two-part
+// sum (its second part holds the quotient's remainder and the cubic and
+// higher terms), then y log x in two parts
+__device__ __forceinline__ double pow_pos(double x, double y) {
+  double m = __builtin_amdgcn_frexp_mant(x);
+  int e = __builtin_amdgcn_frexp_exp(x);
+  const bool lo = m < 0x1.6a09e667f3bcdp-1;
+  m = lo ? m + m : m;
+  const double k = (double)(lo ? e - 1 : e);
+  const double num = m - 1.0, den = m + 1.0, dl = m - (den - 1.0);
+  const double id = rcp(den);
+  const double s = num * id;
+  const double sl = fma(-s, dl, fma(-s, den, num)) * id;
+  const double w = s * s;
+  double p = 0x1.0c1263e1bac13p-3;
+  p = fma(p, w, 0x1.0fbd2bafa02d6p-3);
+  p = fma(p, w, 0x1.3b1c42e3df02cp-3);
+  p = fma(p, w, 0x1.745cf8c4c7bcap-3);
+  p = fma(p, w, 0x1.c71c7201f207cp-3);
+  p = fma(p, w, 0x1.2492492476765p-2);
+  p = fma(p, w, 0x1.9999999999a3ap-2);
+  p = fma(p, w, 0x1.5555555555555p-1);
+  const double a = k * 0x1.62e42fee00000p-1, b = s + s;
+  const double hi = a + b;
+  const double l = (b - (hi - a)) + fma(k, 0x1.a39ef35793c76p-33, fma(s * w, p, sl + sl));
+  const double ph = y * hi;
+  return exp(ph, fma(y, l, fma(y, hi, -ph)));
+}
+// x**y for finite x, the zero and negative bases by selects
+__device__ __forceinline__ double pow(double x, double y) {
+  double r = pow_pos(fabs(x), y);
+  const bool whole = rint(y) == y, odd = whole && rint(0.5 * y) != 0.5 * y;
+  r = x < 0.0 ? (whole ? (odd ? -r : r) : __builtin_nan("")) : r;
+  return x == 0.0 ? (y > 0.0 ? 0.0 : (y == 0.0 ? 1.0 : __builtin_inf())) : r;
+}
+}  // namespace f64
+
 // Precision policy of the pair arithmetic.  R = double: every operation in
-// FP64 with the library's correctly rounded elementary functions.  R = float:
+// FP64, elementary functions from f64 above or the library.  R = float:
 // dr comes from the fixed-point positions (Geo<float>), the pair terms use the gfx950
 // transcendental unit (v_exp_f32, v_sin/cos_f32, v_sqrt_f32, v_rcp_f32).
 template <class R> struct PM;
 template <> struct PM<double> {
-  // exponential exp(k*x) with a constant k prepared by kexp(k)
-  static __host__ __device__ __forceinline__ double kexp(double k) { return k; }
-  static __device__ __forceinline__ double expk(double kx) { return exp(kx); }
-  // sin(pi*x), cos(pi*x) with the reference's pi literal
-  static __device__ __forceinline__ void sincospi_(double x, double& s, double& c) { sincos(PFM_PI * x, &s, &c); }
-  static __device__ __forceinline__ double exp_(double x) { return exp(x); }
+  static __device__ __forceinline__ double exp_(double x) { return f64::exp(x); }
   static __device__ __forceinline__ double sqrt_(double x) { return sqrt(x); }
-  static __device__ __forceinline__ double rcp(double x) { return 1.0 / x; }
+  static __device__ __forceinline__ double rcp(double x) { return f64::rcp(x); }
   static __device__ __forceinline__ double cos_(double x) { return cos(x); }
   static __device__ __forceinline__ double sin_(double x) { return sin(x); }
-  static __device__ __forceinline__ double pow_(double x, double y) { return pow(x, y); }
+  static __device__ __forceinline__ double pow_(double x, double y) { return f64::pow(x, y); }
 };
 template <> struct PM<float> {
+  // exp(k x) = 2^(kexp(k) x)
   static __host__ __device__ __forceinline__ float kexp(double k) { return (float)(k * 1.4426950408889634); }
-  static __device__ __forceinline__ float expk(float kx) { return __builtin_amdgcn_exp2f(kx); }
-  // v_sin_f32 / v_cos_f32 take their argument in revolutions
-  static __device__ __forceinline__ void sincospi_(float x, float& s, float& c) {
-    s = __builtin_amdgcn_sinf(0.5f * x);
-    c = __builtin_amdgcn_cosf(0.5f * x);
-  }
   static __device__ __forceinline__ float exp_(float x) { return __expf(x); }
   static __device__ __forceinline__ float sqrt_(float x) { return __builtin_amdgcn_sqrtf(x); }
   static __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
@@ -153,13 +269,19 @@ __device__ __forceinline__ void cos_cutoff(R r, R R1, R R2, R inv_w, R& f, R& df
 // or beyond R2 are masked by the caller.  Returns f and dfr = f'(r)
 // (= df_cut * r of the reference, whose df_cut is f'/r), kdf = -pi/(2 (R2-R1)).
 template <class R>
-__device__ __forceinline__ void cutoff_bl(R r, R R1, R inv_w, R kdf, R& f, R& dfr) {
-  R x = (r - R1) * inv_w;
-  x = x < R(0) ? R(0) : (x > R(1) ? R(1) : x);
-  R sn, cs;
-  PM<R>::sincospi_(x, sn, cs);
-  f = R(0.5) + R(0.5) * cs;
-  dfr = kdf * sn;
+__device__ __forceinline__ void cutoff_bl(R r, R R1, R inv_w, R kdf, R& f, R& dfr);
+// FP64: through the half angle y = pi x / 2 in [0, pi/2], f = cos(y)^2 and
+// sin(pi x) = 2 sin(y) cos(y); f is exactly 1 and dfr exactly 0 at x = 0
+__device__ __forceinline__ double cutoff_half(double r, double R1, double inv_w) {
+  return fmin(fmax((r - R1) * (0.5 * PFM_PI * inv_w), 0.0), 0.5 * PFM_PI);
+}
+template <>
+__device__ __forceinline__ void cutoff_bl<double>(double r, double R1, double inv_w, double kdf, double& f,
+                                                  double& dfr) {
+  const double y = cutoff_half(r, R1, inv_w);
+  const double c = f64::cos_q1(y);
+  f = c * c;
+  dfr = (kdf + kdf) * (f64::sin_q1(y) * c);
 }
 // Mixed path: the argument in revolutions t = (r - R1) / (2 (R2 - R1)) is one
 // fused multiply-add (its constants are loop invariants), clamped to [0, 1/2]
@@ -172,12 +294,13 @@ __device__ __forceinline__ void cutoff_bl<float>(float r, float R1, float inv_w,
   dfr = kdf * __builtin_amdgcn_sinf(t);
 }
 
-// r = |dr| and 1/r from dr.dr: FP64 with the correctly rounded square root
-// and division; the mixed path from one v_rsq_f32 (r = d2 / sqrt(d2))
+// r = |dr| and 1/r from dr.dr: FP64 by f64::sqrt_rsqrt; the mixed path from
+// one v_rsq_f32 (r = d2 / sqrt(d2)).  Two atoms on one point give NaN in both.
 template <class R>
-__device__ __forceinline__ void dist_and_inverse(R d2, R& r, R& ir) {
-  r = PM<R>::sqrt_(d2);
-  ir = PM<R>::rcp(r);
+__device__ __forceinline__ void dist_and_inverse(R d2, R& r, R& ir);
+template <>
+__device__ __forceinline__ void dist_and_inverse<double>(double d2, double& r, double& ir) {
+  f64::sqrt_rsqrt(d2, r, ir);
 }
 template <>
 __device__ __forceinline__ void dist_and_inverse<float>(float d2, float& r, float& ir) {
