@@ -710,7 +710,7 @@ static int finalize(pfm_ctx* h) {
   h->hrep.assign(nrep, RepDev());
   std::vector<int> rank_all, xyz_all, crep_all;
   h->ncell = 0;
-  h->any_tile = h->any_rows = false;
+  std::vector<int> narrow_all;
   for (int r = 0; r < nrep; ++r) {
     RepDev& R = h->hrep[r];
     memset(&R, 0, sizeof R);
@@ -737,10 +737,9 @@ static int finalize(pfm_ctx* h) {
     R.clen = make_double3(cl[0], cl[1], cl[2]);
     R.inv_clen = make_double3(1.0 / cl[0], 1.0 / cl[1], 1.0 / cl[2]);
     R.cell_base = h->ncell;
-    R.tile = nc[0] >= 3 && nc[1] >= 3 && nc[2] >= 3;
+    const bool narrow = nc[0] < 3 || nc[1] < 3 || nc[2] < 3;
     R.zlo = 0.8 * bx[2];
     R.zhi = 0.9 * bx[2];
-    (R.tile ? h->any_tile : h->any_rows) = true;
     const int ncr = nc[0] * nc[1] * nc[2];
     std::vector<std::pair<uint64_t, int>> key(ncr);
     for (int z = 0; z < nc[2]; ++z)
@@ -758,6 +757,7 @@ static int finalize(pfm_ctx* h) {
       rank_all[h->ncell + lin] = h->ncell + k;
       xyz_all[h->ncell + k] = x | (y << 10) | (z << 20);
       crep_all[h->ncell + k] = r;
+      if (narrow) narrow_all.push_back(h->ncell + k);
     }
     h->ncell += ncr;
   }
@@ -771,6 +771,12 @@ static int finalize(pfm_ctx* h) {
   HIPCHK(h, hipMemcpyAsync(h->cell_rank, rank_all.data(), sizeof(int) * h->ncell, hipMemcpyHostToDevice, h->stream));
   if ((rc = dalloc(h, &h->cell_xyz, h->ncell))) return rc;
   HIPCHK(h, hipMemcpyAsync(h->cell_xyz, xyz_all.data(), sizeof(int) * h->ncell, hipMemcpyHostToDevice, h->stream));
+  h->n_narrow = (int)narrow_all.size();
+  if (h->n_narrow) {
+    if ((rc = dalloc(h, &h->narrow_cells, h->n_narrow))) return rc;
+    HIPCHK(h, hipMemcpyAsync(h->narrow_cells, narrow_all.data(), sizeof(int) * h->n_narrow, hipMemcpyHostToDevice,
+                             h->stream));
+  }
   if (nrep > 1) {
     if ((rc = dalloc(h, &h->cell_rep, h->ncell))) return rc;
     HIPCHK(h, hipMemcpyAsync(h->cell_rep, crep_all.data(), sizeof(int) * h->ncell, hipMemcpyHostToDevice, h->stream));
@@ -802,14 +808,19 @@ static int finalize(pfm_ctx* h) {
     for (int k = 0; k < it.nl_n; ++k) {
       ListDev& L = it.nl[k];
       {
-        // atoms per cell over the replicas that hold rows of the list
+        // One wave per cell only for many cells of few atoms (over the
+        // replicas that hold rows of the list): four lists of a binary gas,
+        // wave against workgroup: 3.4 atoms in each of 29,791 cells 71 and
+        // 112 us, 7.3 in 2,744 14 and 17, 9.1 in 21,952 103 and 116, 11.4 in
+        // 17,576 142 and 123, 13 in 4,913 105 and 44, 5.8 in 343 26 and 9
+        // (few waves, each a long chain of dependent steps).
         double atoms = 0.0, cells = 0.0;
         for (int r = 0; r < nrep; ++r) {
           if (gcnt[L.g1][r] == 0) continue;
           atoms += h->rep_n[r];
           cells += (double)h->hrep[r].nc[0] * h->hrep[r].nc[1] * h->hrep[r].nc[2];
         }
-        L.sparse_cells = cells > 0.0 && atoms < 14.0 * cells;
+        L.wave_cells = cells >= 2048.0 && atoms < 10.0 * cells;
       }
       // rows of the pair lists start on 16 bytes and end 32 entries early
       // enough that the passes' four-entry loads stay inside the array; the
@@ -852,7 +863,8 @@ static int finalize(pfm_ctx* h) {
   }
   // pair searches (ListDev::pair_*): lj / lj1g lists in build order, each
   // paired with the first later unpaired one of the same rows, cutoff and
-  // period when both are searched one wave per cell with over eight entries
+  // period when both hold over eight entries: the four lists of a batch's
+  // gases (18 atoms per cell) in one pass take 140 us instead of 4 x 116
   {
     struct Cand { int ii, k; };
     std::vector<Cand> order;
@@ -874,10 +886,10 @@ static int finalize(pfm_ctx* h) {
     }
     for (size_t x = 0; x < order.size(); ++x) {
       ListDev& A = h->inter[order[x].ii].nl[order[x].k];
-      if (A.pair_ii >= 0 || !A.sparse_cells || A.nmax <= 8) continue;
+      if (A.pair_ii >= 0 || A.nmax <= 8) continue;
       for (size_t y = x + 1; y < order.size(); ++y) {
         ListDev& B = h->inter[order[y].ii].nl[order[y].k];
-        if (B.pair_ii >= 0 || !B.sparse_cells || B.nmax <= 8 || B.g1 != A.g1 || rc_of(order[y]) != rc_of(order[x]) ||
+        if (B.pair_ii >= 0 || B.nmax <= 8 || B.g1 != A.g1 || rc_of(order[y]) != rc_of(order[x]) ||
             per_of(order[y]) != per_of(order[x]))
           continue;
         A.pair_ii = order[y].ii; A.pair_k = order[y].k; A.pair_lead = true;
@@ -2679,7 +2691,7 @@ int pfm_destroy(pfm_ctx* h) {
   for (auto e : h->rec.free_ev) (void)hipEventDestroy(e);
   auto F = [](void* p) { if (p) (void)hipFree(p); };
   F(h->pos4); F(h->vel4); F(h->frc4); F(h->pos4b); F(h->vel4b); F(h->frc4b); F(h->mask); F(h->maskb);
-  F(h->orig); F(h->origb); F(h->perm); F(h->atom_rank); F(h->scan_tmp); F(h->eb); F(h->qpos); F(h->rdev); F(h->rep); F(h->repb); F(h->cell_rep); F(h->d_rep_row0); F(h->d_rep_out);
+  F(h->orig); F(h->origb); F(h->perm); F(h->atom_rank); F(h->scan_tmp); F(h->eb); F(h->qpos); F(h->rdev); F(h->rep); F(h->repb); F(h->cell_rep); F(h->narrow_cells); F(h->d_rep_row0); F(h->d_rep_out);
   F(h->red_part); F(h->red_out); F(h->derr); F(h->cell_rank); F(h->cell_count); F(h->cell_start); F(h->cell_xyz);
   F(h->nhc_state);
   F(h->xfer);

@@ -385,7 +385,6 @@ struct RepDev {
   double3 clen, inv_clen;
   int nc[3];
   int cell_base;        // global rank (and linear index) of the grid's first cell
-  int tile;             // grid at least three cells wide in every direction
   double zlo, zhi;      // invert_z_velocities band
 };
 
@@ -482,10 +481,10 @@ struct ListDev {
   int* nbr = nullptr;   // [nrows*stride] internal atom indices
   int* rev = nullptr;   // [nrows*stride] slot of the row atom in the neighbour's row (tb, nn lists)
   bool built = false;
-  bool sparse_cells = false;  // the replicas holding its rows average few atoms per cell: one wave per cell
+  bool wave_cells = false;  // searched one wave per cell: many cells of few atoms
   // Pair search: an lj / lj1g list and another with the same rows, cutoff and
-  // rebuild steps, both searched one wave per cell, are built in one pass
-  // (launch_build_pair) by the earlier of the two in build order (the lead)
+  // rebuild steps are built in one pass (launch_build_pair) by the earlier of
+  // the two in build order (the lead)
   int pair_ii = -1, pair_k = -1;
   bool pair_lead = false;
   bool pair_sparse = false;  // the union of the two candidate groups is under half of the atoms
@@ -581,7 +580,9 @@ struct pfm_ctx {
   RepDev* rdev = nullptr;             // [nrep]
   int *rep = nullptr, *repb = nullptr;  // [N] replica of every internal atom (batches only)
   int* cell_rep = nullptr;            // [ncell] replica of every cell (batches only)
-  bool any_tile = false, any_rows = false;  // some replica searched by cell tiles / by rows
+  // cells of grids under three cells wide in some direction
+  int* narrow_cells = nullptr;
+  int n_narrow = 0;
   // per replica and group: first row of the replica in the group's rows
   std::vector<int> rep_row0[PFM_MAXG + 1];
   int* d_rep_row0 = nullptr;  // [(PFM_MAXG + 1) * (nrep + 1)]; slot 0: first internal atom of every replica

@@ -383,13 +383,13 @@ struct SearchArgs {
   int step, err_code;
   int exact;  // require exactly nmax entries (graphene nearest neighbours)
   // a second list with the same rows, cutoff and rebuild steps searched in
-  // the same pass (k_build_tile_wave<T, CMP, true>): g2bit is then the union
+  // the same pass (PAIR): g2bit is then the union
   // of the two candidate groups, g2bit1 / g2bit2 the groups of the two lists
   uint32_t g2bit1, g2bit2;
   int nmax2, stride2;
   int* nnum2;
   int* nbr2;
-  // a second pair in the same pass (k_build_tile_wave<T, CMP, true, true>):
+  // a second pair in the same pass (QUAD):
   // rows of another group (side b, disjoint from group 1), whose two lists
   // take the candidates of g2bit1 (b1) and of g2bit2 (b2); g1mem is then
   // the union of the two row groups' member bits
@@ -398,84 +398,6 @@ struct SearchArgs {
   int nmax_b1, stride_b1, nmax_b2, stride_b2;
   int *nnum_b1, *nbr_b1, *nnum_b2, *nbr_b2;
 };
-
-// T lanes per row atom scan the 27 (or fewer, for boxes under three cells
-// wide) surrounding cells; wave ballots compact the accepted candidates.
-template <int T>
-__global__ void __launch_bounds__(256) k_build(SearchArgs a, int nblocks_real) {
-  int lb = xcd_block(nblocks_real);
-  if (lb < 0) return;
-  int gt = lb * blockDim.x + threadIdx.x;
-  int row = gt / T, t = threadIdx.x & (T - 1);
-  if (row >= a.nrows) return;
-  int lane = threadIdx.x & 63;
-  int gshift = lane & ~(T - 1);
-  unsigned long long gmask = (T == 64) ? ~0ull : (((1ull << T) - 1ull) << gshift);
-  unsigned long long lower = (1ull << lane) - 1ull;
-  int i = a.rows[row];
-  const RepDev R = a.rdev[a.rep ? a.rep[i] : 0];
-  if (R.tile) return;  // searched by k_build_tile
-  if (!(a.mask[i] & a.g1bit)) {
-    // find_neighbours runs over the group's active atoms only (md_neighbours.f90:67)
-    if (t == 0) a.nnum[row] = 0;
-    return;
-  }
-  double4 pi = a.pos[i];
-  int c[3];
-  c[0] = cell_coord(pi.x, R.inv_clen.x, R.nc[0]);
-  c[1] = cell_coord(pi.y, R.inv_clen.y, R.nc[1]);
-  c[2] = cell_coord(pi.z, R.inv_clen.z, R.nc[2]);
-  int lo[3], cnt[3];
-  for (int d = 0; d < 3; ++d) {
-    if (R.nc[d] >= 3) { lo[d] = c[d] - 1; cnt[d] = 3; }
-    else { lo[d] = 0; cnt[d] = R.nc[d]; }
-  }
-  int count = 0;
-  int* out = a.nbr + (size_t)row * a.stride;
-  for (int oz = 0; oz < cnt[2]; ++oz) {
-    int z = lo[2] + oz; z = z < 0 ? z + R.nc[2] : (z >= R.nc[2] ? z - R.nc[2] : z);
-    for (int oy = 0; oy < cnt[1]; ++oy) {
-      int y = lo[1] + oy; y = y < 0 ? y + R.nc[1] : (y >= R.nc[1] ? y - R.nc[1] : y);
-      for (int ox = 0; ox < cnt[0]; ++ox) {
-        int x = lo[0] + ox; x = x < 0 ? x + R.nc[0] : (x >= R.nc[0] ? x - R.nc[0] : x);
-        int r = a.cell_rank[R.cell_base + (z * R.nc[1] + y) * R.nc[0] + x];
-        int s = a.cell_start[r], n = a.cell_count[r];
-        for (int base = 0; base < n; base += T) {
-          int k = base + t;
-          bool pred = false;
-          int j = 0;
-          if (k < n) {
-            j = a.bin ? a.bin[s + k] : s + k;
-            if (j != i && (a.mask[j] & a.g2bit)) {
-              double4 pj = a.pos[j];
-              double ax = pj.x - pi.x, ay = pj.y - pi.y, az = pj.z - pi.z;
-              ax = fma(-R.L.x, rint(ax * R.iL.x), ax);
-              ay = fma(-R.L.y, rint(ay * R.iL.y), ay);
-              az = fma(-R.L.z, rint(az * R.iL.z), az);
-              double d2 = fma(ax, ax, fma(ay, ay, az * az));
-              if (d2 < a.rc2_lo) pred = true;
-              else if (d2 <= a.rc2_hi) {
-                double dx, dy, dz;
-                pred = min_image_dist2(pi, pj, R.hb, dx, dy, dz) < a.rc2;
-              }
-            }
-          }
-          unsigned long long bits = __ballot(pred) & gmask;
-          if (pred) {
-            int slot = count + __popcll(bits & lower);
-            if (slot < a.nmax) out[slot] = j;
-          }
-          count += __popcll(bits);
-        }
-      }
-    }
-  }
-  if (t == 0) {
-    a.nnum[row] = count < a.nmax ? count : a.nmax;
-    if (count > a.nmax) raise_err(a.err, a.err_code, a.orig[i] + 1, count, a.step);
-    else if (a.exact && count != a.nmax) raise_err(a.err, PFM_E_GRAPHENE_NN, a.orig[i] + 1, count, a.step);
-  }
-}
 
 // slot of the row atom inside each neighbour's own row (Tersoff-Brenner's
 // `do l=1,nl%nnum(j); if(nl%nlist(l,j)==i) exit` and graphene's l1 search)
@@ -594,22 +516,83 @@ __global__ void k_nn_from_tb(int nrows, const int* __restrict__ rows, const int*
   if (k != 3) raise_err(err, PFM_E_GRAPHENE_NN, orig[i] + 1, k, step);
 }
 
-// Cell-tile list search: one workgroup per cell (grids at least three cells
-// wide).  The atoms of the 27 surrounding cells are staged in LDS as FP32
-// coordinates unwrapped into the frame of the centre cell's origin, with the
-// atom index in w.  Atoms outside group 2, and the padding after the last
-// atom, are staged far away, so they never pass the distance test.  With
-// CMP (group 2 under half of the atoms: another species' list) only the
-// group-2 atoms are staged, compacted in tile order by ballots and a prefix
-// over the workgroup's four waves, so the rows walk only real candidates.  Every group-1 atom of the centre cell is a row scanned by T
-// lanes; all rows of a wavefront walk the tile in the same order, so their
-// LDS reads are broadcasts.  Each lane takes 32 of its candidates (every T-th
-// slot) into a register bitmask, two instructions per candidate after the
-// distance; the row's lanes then take their output offsets from a prefix sum
-// over the T lanes and write their hits.  The FP32 distance decides unless it
-// lies within a relative 3e-5 of r_cut**2, where the reference's FP64
-// find_distance test (min_image_dist2) on the global positions decides.
+// Cell-tile list search: one workgroup per cell.  The atoms of the 27
+// surrounding cells are staged in LDS as FP32 coordinates unwrapped into the
+// frame of the centre cell's origin, with the atom index in w.  Atoms outside
+// group 2, and the padding after the last atom, are staged far away, so they
+// never pass the distance test.  With CMP (group 2 under half of the atoms:
+// another species' list) only the group-2 atoms are staged, compacted in tile
+// order by ballots and a prefix over the workgroup's four waves, so the rows
+// walk only real candidates.  Every group-1 atom of the centre cell is a row
+// scanned by T lanes; all rows of a wavefront walk the tile in the same order,
+// so their LDS reads are broadcasts.  Each lane takes 32 of its candidates
+// (every T-th slot) into a register bitmask, two instructions per candidate
+// after the distance; the row's lanes then take their output offsets from a
+// prefix sum over the T lanes and write their hits.  The FP32 distance decides
+// unless it lies within a relative 3e-5 of r_cut**2, where the reference's
+// FP64 find_distance test (min_image_dist2) on the global positions decides.
 // Tiles larger than the LDS buffer are staged in several passes.
+// PAIR and QUAD: two or four lists in one pass, see SearchArgs.
+//
+// Directions under three cells wide hold each of their cells once in the tile
+// (two or one instead of three) and cannot be unwrapped once per cell: there
+// the coordinates are staged as they are and every pair takes its nearest
+// image (TileImage), nine more instructions a candidate.  A row-by-row search
+// of such grids, whose candidates wait on two dependent loads each, took 45 us
+// for a 256-atom Cu replica's list.
+// The cells of such grids go through launches of their own (IMG, over
+// pfm_ctx::narrow_cells): a kernel that held both scans searched a
+// 131,072-atom Cu crystal in 67 us instead of 63.
+__device__ __forceinline__ bool narrow_grid(const RepDev& R) { return R.nc[0] < 3 || R.nc[1] < 3 || R.nc[2] < 3; }
+struct TileImage {
+  float3 L, iL;  // box and its inverse in the directions under three cells wide, 0 in the others
+  __device__ __forceinline__ TileImage(const RepDev& R)
+      : L(make_float3(R.nc[0] < 3 ? (float)R.L.x : 0.f, R.nc[1] < 3 ? (float)R.L.y : 0.f,
+                      R.nc[2] < 3 ? (float)R.L.z : 0.f)),
+        iL(make_float3(R.nc[0] < 3 ? (float)R.iL.x : 0.f, R.nc[1] < 3 ? (float)R.iL.y : 0.f,
+                       R.nc[2] < 3 ? (float)R.iL.z : 0.f)) {}
+  // the nearest image of a difference; the clamp keeps far-away padding far
+  static __device__ __forceinline__ float near(float d, float L, float iL) {
+    return fmaf(-L, rintf(__builtin_amdgcn_fmed3f(d * iL, -2.0f, 2.0f)), d);
+  }
+  template <bool IMG>
+  __device__ __forceinline__ void diff(const float4& v, float px, float py, float pz, float& dx, float& dy,
+                                       float& dz) const {
+    dx = v.x - px; dy = v.y - py; dz = v.z - pz;
+    if constexpr (IMG) {
+      dx = near(dx, L.x, iL.x); dy = near(dy, L.y, iL.y); dz = near(dz, L.z, iL.z);
+    }
+  }
+};
+
+// tile cell k (0..26) of a grid cell cc: its coordinates, and whether it is
+// one of the tile's own (a direction two cells wide holds offsets 0 and 1,
+// one cell wide offset 0)
+template <bool IMG>
+__device__ __forceinline__ bool tile_cell(const RepDev& R, const int* cc, int k, int* q) {
+  const int o[3] = {k % 3 - 1, (k / 3) % 3 - 1, k / 9 - 1};
+  bool own = true;
+  for (int d = 0; d < 3; ++d) {
+    const int nd = R.nc[d];
+    if (IMG) own = own && (nd >= 3 || o[d] == 0 || (nd == 2 && o[d] > 0));
+    q[d] = cc[d] + o[d];
+    q[d] = q[d] < 0 ? q[d] + nd : (q[d] >= nd ? q[d] - nd : q[d]);
+  }
+  return own;
+}
+
+// coordinate x of an atom of the tile cell at offset o, relative to the centre
+// cell's origin: the image next to the centre cell (directions of three cells
+// or more)
+template <bool IMG>
+__device__ __forceinline__ double unwrap(double x, int o, double L, int nd) {
+  if (!IMG || nd >= 3) {
+    if (o < 0 && x > 0.0) x -= L;
+    else if (o > 0 && x < 0.0) x += L;
+  }
+  return x;
+}
+
 // the row of atom i (if it has one) when its tile holds no candidate: what
 // the search writes for a row with no entries
 __device__ __forceinline__ void empty_row(const SearchArgs& a, const int* __restrict__ row_of, int i) {
@@ -627,18 +610,171 @@ struct TileCells {
   int start[27], cnt[27], off[28];
 };
 
-template <int T, bool CMP>
-__global__ void __launch_bounds__(256, CMP ? 5 : 6) k_build_tile(SearchArgs a, const int* __restrict__ rank_xyz,
-                                                    const int* __restrict__ row_of, int nblocks_real) {
+#define ENTRY_IDX 0x3fffffff  // staged index without the pair search's group bits
+
+// what staging keeps in w: the atom's index, with PAIR also its membership of
+// list 1's candidate group in bit 30 and of list 2's in bit 31
+template <bool PAIR>
+__device__ __forceinline__ float staged_w(const SearchArgs& a, int j, uint32_t mj) {
+  uint32_t w = (uint32_t)j;
+  if constexpr (PAIR) w |= ((mj & a.g2bit1) ? 0x40000000u : 0u) | ((mj & a.g2bit2) ? 0x80000000u : 0u);
+  return __uint_as_float(w);
+}
+
+// The rows of one list (PAIR: two) that a row atom's lanes fill: destinations
+// and counts.  QUAD: atoms of side b take side b's lists.
+template <int T, bool PAIR, bool QUAD>
+struct RowOut {
+  bool active;
+  int i, row, count, count2;
+  int *out, *out2, *nnum1, *nnum2;
+  int nmax1, nmax2;
+  __device__ __forceinline__ RowOut(const SearchArgs& a, const int* __restrict__ row_of, int atom, bool inrow) {
+    i = atom;
+    const uint32_t mi = a.mask[i];
+    const bool sb = QUAD && (mi & a.g1mem_b) != 0;
+    row = inrow ? (sb ? a.row_of_b[i] : row_of[i]) : -1;
+    active = row >= 0 && (mi & (sb ? a.g1bit_b : a.g1bit));
+    count = count2 = 0;
+    const size_t r = active ? row : 0;
+    nnum1 = sb ? a.nnum_b1 : a.nnum;
+    nmax1 = sb ? a.nmax_b1 : a.nmax;
+    out = (sb ? a.nbr_b1 : a.nbr) + r * (sb ? a.stride_b1 : a.stride);
+    nnum2 = out2 = nullptr;
+    nmax2 = 0;
+    if constexpr (PAIR) {
+      nnum2 = sb ? a.nnum_b2 : a.nnum2;
+      nmax2 = sb ? a.nmax_b2 : a.nmax2;
+      out2 = (sb ? a.nbr_b2 : a.nbr2) + r * (sb ? a.stride_b2 : a.stride2);
+    }
+  }
+  // the row's hits of one round into one list: offsets from a prefix sum over
+  // the row's lanes, entries without the group bits
+  static __device__ __forceinline__ void put(unsigned hit, const float4* sv, int t, int* o, int nmax, int& cnt) {
+    const int nh = __popc(hit);
+    int pre = nh;
+#pragma unroll
+    for (int d = 1; d < T; d <<= 1) {
+      int w = __shfl_up(pre, d, T);
+      if (t >= d) pre += w;
+    }
+    const int tot = __shfl(pre, T - 1, T);
+    int slot = cnt + pre - nh;
+    while (hit) {
+      const int b = __clz(hit);
+      hit &= ~(0x80000000u >> b);
+      if (slot < nmax) o[slot] = __float_as_int(sv[b * T].w) & ENTRY_IDX;
+      ++slot;
+    }
+    cnt += tot;
+  }
+  // one pass over np staged candidates (whole rounds of 32 T); own: the row
+  // atom's staged slot, or -1 to find it by index (find_self)
+  template <bool IMG>
+  __device__ __forceinline__ void scan(const SearchArgs& a, const TileImage& im, const float4* st, int np, int t,
+                                       int own, bool find_self, const double4& pi, float px, float py, float pz,
+                                       float hi, float lo, const double3& hb) {
+    const float win = hi - lo;
+    for (int c0 = 0; c0 < np; c0 += 32 * T) {
+      // bit 31-b <-> candidate slot c0 + t + b*T
+      const float4* sv = st + c0 + t;
+      // two masks with two instructions each per candidate after the
+      // differences: the margin m = hi - d2 as a chain of fused
+      // multiply-adds, whose sign bit (set for d2 > hi, and for the far
+      // padding's -inf) shifts into the miss mask, and the sign of
+      // (hi - lo) - m, set for d2 < lo (clearly inside r_cut); with PAIR the
+      // candidates of list 1's and of list 2's group in two more
+      unsigned miss = 0u, inside = 0u, m1 = 0u, m2 = 0u;
+#pragma unroll PAIR ? 4 : 8
+      for (int b = 0; b < 32; ++b) {
+        const float4 v = sv[b * T];
+        float dx, dy, dz;
+        im.diff<IMG>(v, px, py, pz, dx, dy, dz);
+        const float m = fmaf(-dx, dx, fmaf(-dy, dy, fmaf(-dz, dz, hi)));
+        miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(m), 31);
+        inside = __builtin_amdgcn_alignbit(inside, __float_as_uint(win - m), 31);
+        if constexpr (PAIR) {
+          const uint32_t wb = __float_as_uint(v.w);
+          m1 = __builtin_amdgcn_alignbit(m1, wb << 1, 31);
+          m2 = __builtin_amdgcn_alignbit(m2, wb, 31);
+        }
+      }
+      unsigned hit = ~miss;
+      // the row atom is not its own neighbour
+      const int ob = own - c0 - t;
+      if (ob >= 0 && ob < 32 * T && ob % T == 0) hit &= ~(0x80000000u >> (ob / T));
+      // hits inside the FP32 window: the FP64 test decides (with compacted
+      // staging that is not dense every hit is also checked for the row atom)
+      unsigned chk = find_self ? hit : hit & ~inside;
+      while (chk) {
+        const int b = __clz(chk);
+        chk &= ~(0x80000000u >> b);
+        const float4 v = sv[b * T];
+        const int j = __float_as_int(v.w) & ENTRY_IDX;
+        float dx, dy, dz;
+        im.diff<IMG>(v, px, py, pz, dx, dy, dz);
+        if (find_self && j == i) {
+          hit &= ~(0x80000000u >> b);
+        } else if (fmaf(dx, dx, fmaf(dy, dy, dz * dz)) >= lo) {
+          double ex, ey, ez;
+          if (!(min_image_dist2(pi, a.pos[j], hb, ex, ey, ez) < a.rc2)) hit &= ~(0x80000000u >> b);
+        }
+      }
+      if constexpr (PAIR) {
+        put(hit & m1, sv, t, out, nmax1, count);
+        put(hit & m2, sv, t, out2, nmax2, count2);
+      } else {
+        put(hit, sv, t, out, nmax1, count);
+      }
+    }
+  }
+  // the row's lengths, and the reference's errors
+  __device__ __forceinline__ void finish(const SearchArgs& a) const {
+    if (row < 0) return;
+    if (!active) {  // an inactive member of a growing group
+      nnum1[row] = 0;
+      if (PAIR) nnum2[row] = 0;
+      return;
+    }
+    nnum1[row] = count < nmax1 ? count : nmax1;
+    if (count > nmax1) raise_err(a.err, a.err_code, a.orig[i] + 1, count, a.step);
+    else if (a.exact && count != nmax1) raise_err(a.err, PFM_E_GRAPHENE_NN, a.orig[i] + 1, count, a.step);
+    if (PAIR) {
+      nnum2[row] = count2 < nmax2 ? count2 : nmax2;
+      if (count2 > nmax2) raise_err(a.err, a.err_code, a.orig[i] + 1, count2, a.step);
+    }
+  }
+};
+
+// every row of the cell's atoms empty: its tile holds no candidate
+template <bool QUAD>
+__device__ __forceinline__ void empty_rows(const SearchArgs& a, const int* __restrict__ row_of, int cs, int ncen,
+                                           int first, int step) {
+  for (int m = first; m < ncen; m += step) {
+    const int i = a.bin ? a.bin[cs + m] : cs + m;
+    if (QUAD && (a.mask[i] & a.g1mem_b)) {
+      const int row = a.row_of_b[i];
+      if (row >= 0) { a.nnum_b1[row] = 0; a.nnum_b2[row] = 0; }
+    } else {
+      empty_row(a, row_of, i);
+    }
+  }
+}
+
+template <int T, bool CMP, bool PAIR, bool QUAD, bool IMG>
+__global__ void __launch_bounds__(256, CMP || PAIR ? 5 : 6) k_build_tile(SearchArgs a, const int* __restrict__ rank_xyz,
+                                                    const int* __restrict__ row_of, int nblocks_real,
+                                                    const int* __restrict__ cells) {
   static_assert(TILE_MAX % (32 * T) == 0, "tile passes hold whole bitmask rounds");
   __shared__ float4 st[TILE_MAX];
   __shared__ TileCells tc;
   int c = xcd_block(nblocks_real);
   if (c < 0) return;
+  if (IMG) c = cells[c];
   const int ncen = a.cell_count[c];
   if (ncen == 0 || !(a.cell_grp[c] & a.g1mem)) return;  // no member of group 1 in the cell
   const RepDev& RG = a.rdev[a.cell_rep ? a.cell_rep[c] : 0];
-  if (!RG.tile) return;  // searched by k_build
+  if (!IMG && narrow_grid(RG)) return;  // searched by the IMG launch
   const int cs = a.cell_start[c];
   const int tid = threadIdx.x;
   // (cells without a row of this list, another species or another
@@ -647,23 +783,20 @@ __global__ void __launch_bounds__(256, CMP ? 5 : 6) k_build_tile(SearchArgs a, c
   const int cc[3] = {pk & 1023, (pk >> 10) & 1023, (pk >> 20) & 1023};
   const double org[3] = {cc[0] * RG.clen.x, cc[1] * RG.clen.y, cc[2] * RG.clen.z};
   const double3 boxL = RG.L, hb = RG.hb;
+  const int nc[3] = {RG.nc[0], RG.nc[1], RG.nc[2]};
+  const TileImage im(RG);
   bool cand = false;
   if (tid < 27) {
-    int o[3] = {tid % 3 - 1, (tid / 3) % 3 - 1, tid / 9 - 1};
     int q[3];
-    for (int d = 0; d < 3; ++d) {
-      int nd = RG.nc[d];
-      q[d] = cc[d] + o[d];
-      q[d] = q[d] < 0 ? q[d] + nd : (q[d] >= nd ? q[d] - nd : q[d]);
-    }
-    int r = a.cell_rank[RG.cell_base + (q[2] * RG.nc[1] + q[1]) * RG.nc[0] + q[0]];
+    const bool own = tile_cell<IMG>(RG, cc, tid, q);
+    int r = a.cell_rank[RG.cell_base + (q[2] * nc[1] + q[1]) * nc[0] + q[0]];
     tc.start[tid] = a.cell_start[r];
-    tc.cnt[tid] = a.cell_count[r];
+    tc.cnt[tid] = own ? a.cell_count[r] : 0;
     cand = (a.cell_grp[r] & a.g2bit) != 0;
   }
   if (!__syncthreads_or(cand)) {
     // no group-2 atom in the tile: every row of the cell is empty
-    for (int m = tid; m < ncen; m += 256) empty_row(a, row_of, a.bin ? a.bin[cs + m] : cs + m);
+    empty_rows<QUAD>(a, row_of, cs, ncen, tid, 256);
     return;
   }
   if (tid == 0) {
@@ -673,7 +806,7 @@ __global__ void __launch_bounds__(256, CMP ? 5 : 6) k_build_tile(SearchArgs a, c
   }
   __syncthreads();
   const int R = tc.off[27];
-  const float hi = (float)(a.rc2 * (1.0 + 3e-5)), lo = (float)(a.rc2 * (1.0 - 3e-5)), win = hi - lo;
+  const float hi = (float)(a.rc2 * (1.0 + 3e-5)), lo = (float)(a.rc2 * (1.0 - 3e-5));
 
   // stage the group-2 atoms of tile slots [s0, s1) compacted into st (slot
   // m < R belongs to the last tile cell k with off[k] <= m; off is
@@ -684,27 +817,29 @@ __global__ void __launch_bounds__(256, CMP ? 5 : 6) k_build_tile(SearchArgs a, c
   constexpr int KS = TILE_MAX / 256;
   __shared__ int wsum[KS][4];
   bool dense = true;
+  // slot m's record and whether its atom is in group 2
+  auto load = [&](int m, float4& v) -> bool {
+    int k = 0;
+#pragma unroll
+    for (int sft = 16; sft > 0; sft >>= 1)
+      if (k + sft < 27 && tc.off[k + sft] <= m) k += sft;
+    int j = tc.start[k] + (m - tc.off[k]);
+    if (a.bin) j = a.bin[j];
+    const double4 p = a.pos[j];
+    const uint32_t mj = a.mask[j];
+    v.x = (float)unwrap<IMG>(p.x - org[0], k % 3 - 1, boxL.x, nc[0]);
+    v.y = (float)unwrap<IMG>(p.y - org[1], (k / 3) % 3 - 1, boxL.y, nc[1]);
+    v.z = (float)unwrap<IMG>(p.z - org[2], k / 9 - 1, boxL.z, nc[2]);
+    v.w = staged_w<PAIR>(a, j, mj);
+    return (mj & a.g2bit) != 0;
+  };
+  const float4 far = make_float4(TILE_FAR, TILE_FAR, TILE_FAR, __int_as_float(-1));
   auto stage = [&](int s0, int s1) -> int {
     if constexpr (!CMP) {
       const int np = (s1 - s0 + 32 * T - 1) / (32 * T) * (32 * T);
       for (int m = s0 + tid; m < s0 + np; m += 256) {
-        float4 v = make_float4(TILE_FAR, TILE_FAR, TILE_FAR, __int_as_float(-1));
-        if (m < s1) {
-          int k = 0;
-#pragma unroll
-          for (int sft = 16; sft > 0; sft >>= 1)
-            if (k + sft < 27 && tc.off[k + sft] <= m) k += sft;
-          int j = tc.start[k] + (m - tc.off[k]);
-          if (a.bin) j = a.bin[j];
-          int o0 = k % 3 - 1, o1 = (k / 3) % 3 - 1, o2 = k / 9 - 1;
-          double4 p = a.pos[j];
-          double x = p.x - org[0], y = p.y - org[1], z = p.z - org[2];
-          if (o0 < 0 && x > 0.0) x -= boxL.x; else if (o0 > 0 && x < 0.0) x += boxL.x;
-          if (o1 < 0 && y > 0.0) y -= boxL.y; else if (o1 > 0 && y < 0.0) y += boxL.y;
-          if (o2 < 0 && z > 0.0) z -= boxL.z; else if (o2 > 0 && z < 0.0) z += boxL.z;
-          v.w = __int_as_float(j);
-          if (a.mask[j] & a.g2bit) { v.x = (float)x; v.y = (float)y; v.z = (float)z; }
-        }
+        float4 v = far;
+        if (m < s1 && !load(m, v)) v.x = v.y = v.z = TILE_FAR;
         st[m - s0] = v;
       }
       return np;
@@ -715,25 +850,8 @@ __global__ void __launch_bounds__(256, CMP ? 5 : 6) k_build_tile(SearchArgs a, c
 #pragma unroll
     for (int u = 0; u < KS; ++u) {
       const int m = s0 + u * 256 + tid;
-      keep[u] = false;
       v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (m < s1) {
-        int k = 0;
-#pragma unroll
-        for (int sft = 16; sft > 0; sft >>= 1)
-          if (k + sft < 27 && tc.off[k + sft] <= m) k += sft;
-        int j = tc.start[k] + (m - tc.off[k]);
-        if (a.bin) j = a.bin[j];
-        int o0 = k % 3 - 1, o1 = (k / 3) % 3 - 1, o2 = k / 9 - 1;
-        double4 p = a.pos[j];
-        keep[u] = (a.mask[j] & a.g2bit) != 0;
-        // unwrap: the image of atom j next to the centre cell
-        double x = p.x - org[0], y = p.y - org[1], z = p.z - org[2];
-        if (o0 < 0 && x > 0.0) x -= boxL.x; else if (o0 > 0 && x < 0.0) x += boxL.x;
-        if (o1 < 0 && y > 0.0) y -= boxL.y; else if (o1 > 0 && y < 0.0) y += boxL.y;
-        if (o2 < 0 && z > 0.0) z -= boxL.z; else if (o2 > 0 && z < 0.0) z += boxL.z;
-        v[u] = make_float4((float)x, (float)y, (float)z, __int_as_float(j));
-      }
+      keep[u] = m < s1 && load(m, v[u]);
     }
     unsigned long long bal[KS];
 #pragma unroll
@@ -752,7 +870,7 @@ __global__ void __launch_bounds__(256, CMP ? 5 : 6) k_build_tile(SearchArgs a, c
     }
     dense = base == s1 - s0;
     const int np = (base + 32 * T - 1) / (32 * T) * (32 * T);
-    for (int m = base + tid; m < np; m += 256) st[m] = make_float4(TILE_FAR, TILE_FAR, TILE_FAR, __int_as_float(-1));
+    for (int m = base + tid; m < np; m += 256) st[m] = far;
     return np;
   };
   const bool single = R <= TILE_MAX;
@@ -764,83 +882,22 @@ __global__ void __launch_bounds__(256, CMP ? 5 : 6) k_build_tile(SearchArgs a, c
     const int qq = q0 + tid / T;
     const bool inrow = qq < ncen;
     const int i = a.bin ? a.bin[cs + (inrow ? qq : 0)] : cs + (inrow ? qq : 0);
-    const int row = inrow ? row_of[i] : -1;
-    const bool active = row >= 0 && (a.mask[i] & a.g1bit);
+    RowOut<T, PAIR, QUAD> ro(a, row_of, i, inrow);
     const double4 pi = a.pos[i];
     const float px = (float)(pi.x - org[0]), py = (float)(pi.y - org[1]), pz = (float)(pi.z - org[2]);
-    int* out = a.nbr + (size_t)(active ? row : 0) * a.stride;
-    int count = 0;
     for (int s0 = 0; s0 < R; s0 += TILE_MAX) {
       if (!single) {
         __syncthreads();
         np = stage(s0, R < s0 + TILE_MAX ? R : s0 + TILE_MAX);
       }
       __syncthreads();
-      if (!active) continue;
+      if (!ro.active) continue;
       // the row atom's own staged slot when the pass is dense (else found by index)
-      const int own = (!CMP || dense) ? tc.off[13] + qq - s0 : -1;
-      for (int c0 = 0; c0 < np; c0 += 32 * T) {
-        // bit 31-b <-> candidate slot c0 + t + b*T
-        const float4* sv = st + c0 + t;
-        // two masks with two instructions each per candidate after the
-        // differences: the margin m = hi - d2 as a chain of fused
-        // multiply-adds, whose sign bit (set for d2 > hi, and for the far
-        // padding's -inf) shifts into the miss mask, and the sign of
-        // (hi - lo) - m, set for d2 < lo (clearly inside r_cut)
-        unsigned miss = 0u, inside = 0u;
-#pragma unroll 8
-        for (int b = 0; b < 32; ++b) {
-          const float4 v = sv[b * T];
-          float dx = v.x - px, dy = v.y - py, dz = v.z - pz;
-          const float m = fmaf(-dx, dx, fmaf(-dy, dy, fmaf(-dz, dz, hi)));
-          miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(m), 31);
-          inside = __builtin_amdgcn_alignbit(inside, __float_as_uint(win - m), 31);
-        }
-        unsigned hit = ~miss;
-        // the row atom is not its own neighbour
-        const int ob = own - c0 - t;
-        if (ob >= 0 && ob < 32 * T && ob % T == 0) hit &= ~(0x80000000u >> (ob / T));
-        // hits inside the FP32 window: the FP64 test decides (with compacted
-        // staging that is not dense every hit is also checked for the row atom)
-        unsigned chk = CMP && !dense ? hit : hit & ~inside;
-        while (chk) {
-          const int b = __clz(chk);
-          chk &= ~(0x80000000u >> b);
-          const float4 v = sv[b * T];
-          const int j = __float_as_int(v.w);
-          float dx = v.x - px, dy = v.y - py, dz = v.z - pz;
-          if (CMP && !dense && j == i) {
-            hit &= ~(0x80000000u >> b);
-          } else if (fmaf(dx, dx, fmaf(dy, dy, dz * dz)) >= lo) {
-            double ex, ey, ez;
-            if (!(min_image_dist2(pi, a.pos[j], hb, ex, ey, ez) < a.rc2)) hit &= ~(0x80000000u >> b);
-          }
-        }
-        // offsets of this lane's hits inside the row
-        const int nh = __popc(hit);
-        int pre = nh;
-#pragma unroll
-        for (int o = 1; o < T; o <<= 1) {
-          int v = __shfl_up(pre, o, T);
-          if (t >= o) pre += v;
-        }
-        const int tot = __shfl(pre, T - 1, T);
-        int slot = count + pre - nh;
-        while (hit) {
-          const int b = __clz(hit);
-          hit &= ~(0x80000000u >> b);
-          if (slot < a.nmax) out[slot] = __float_as_int(sv[b * T].w);
-          ++slot;
-        }
-        count += tot;
-      }
+      const bool find = CMP && !dense;
+      const int own = find ? -1 : tc.off[13] + qq - s0;
+      ro.template scan<IMG>(a, im, st, np, t, own, find, pi, px, py, pz, hi, lo, hb);
     }
-    if (row >= 0 && !active && t == 0) a.nnum[row] = 0;  // an inactive member of a growing group
-    if (active && t == 0) {
-      a.nnum[row] = count < a.nmax ? count : a.nmax;
-      if (count > a.nmax) raise_err(a.err, a.err_code, a.orig[i] + 1, count, a.step);
-      else if (a.exact && count != a.nmax) raise_err(a.err, PFM_E_GRAPHENE_NN, a.orig[i] + 1, count, a.step);
-    }
+    if (t == 0) ro.finish(a);
   }
 }
 
@@ -858,8 +915,7 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-#define ENTRY_IDX 0x3fffffff  // staged index without the pair search's group bits
-template <int T, bool CMP, bool PAIR, bool QUAD = false>
+template <int T, bool CMP, bool PAIR, bool QUAD>
 __global__ void __launch_bounds__(256, 5) k_build_tile_wave(SearchArgs a, const int* __restrict__ rank_xyz,
                                                          const int* __restrict__ row_of, int ncell,
                                                          int nblocks_real) {
@@ -874,39 +930,28 @@ __global__ void __launch_bounds__(256, 5) k_build_tile_wave(SearchArgs a, const 
   const int ncen = a.cell_count[c];
   if (ncen == 0 || !(a.cell_grp[c] & a.g1mem)) return;  // no member of group 1 in the cell
   const RepDev& RG = a.rdev[a.cell_rep ? a.cell_rep[c] : 0];
-  if (!RG.tile) return;  // searched by k_build
+  if (narrow_grid(RG)) return;  // searched by k_build_tile's IMG launch
   const int cs = a.cell_start[c];
   float4* st = stw[wv];
   const int pk = rank_xyz[c];
   const int cc[3] = {pk & 1023, (pk >> 10) & 1023, (pk >> 20) & 1023};
   const double org[3] = {cc[0] * RG.clen.x, cc[1] * RG.clen.y, cc[2] * RG.clen.z};
   const double3 boxL = RG.L, hb = RG.hb;
+  const int nc[3] = {RG.nc[0], RG.nc[1], RG.nc[2]};
+  const TileImage im(RG);
   // the 27 tile cells in lanes 0..26: first atom, count, exclusive offset
   int kst = 0, kcn = 0;
   bool cand = false;
   if (lane < 27) {
-    const int o[3] = {lane % 3 - 1, (lane / 3) % 3 - 1, lane / 9 - 1};
     int q[3];
-    for (int d = 0; d < 3; ++d) {
-      int nd = RG.nc[d];
-      q[d] = cc[d] + o[d];
-      q[d] = q[d] < 0 ? q[d] + nd : (q[d] >= nd ? q[d] - nd : q[d]);
-    }
-    const int r = a.cell_rank[RG.cell_base + (q[2] * RG.nc[1] + q[1]) * RG.nc[0] + q[0]];
+    const bool own = tile_cell<false>(RG, cc, lane, q);
+    const int r = a.cell_rank[RG.cell_base + (q[2] * nc[1] + q[1]) * nc[0] + q[0]];
     kst = a.cell_start[r];
-    kcn = a.cell_count[r];
+    kcn = own ? a.cell_count[r] : 0;
     cand = (a.cell_grp[r] & a.g2bit) != 0;
   }
   if (!__any(cand)) {
-    for (int m = lane; m < ncen; m += 64) {
-      const int i = a.bin ? a.bin[cs + m] : cs + m;
-      if (QUAD && (a.mask[i] & a.g1mem_b)) {
-        const int row = a.row_of_b[i];
-        if (row >= 0) { a.nnum_b1[row] = 0; a.nnum_b2[row] = 0; }
-      } else {
-        empty_row(a, row_of, i);
-      }
-    }
+    empty_rows<QUAD>(a, row_of, cs, ncen, lane, 64);
     return;
   }
   int inc = kcn;
@@ -918,7 +963,7 @@ __global__ void __launch_bounds__(256, 5) k_build_tile_wave(SearchArgs a, const 
   const int koff = inc - kcn;
   const int R = __shfl(inc, 63);
   const int koff13 = __shfl(koff, 13);
-  const float hi = (float)(a.rc2 * (1.0 + 3e-5)), lo = (float)(a.rc2 * (1.0 - 3e-5)), win = hi - lo;
+  const float hi = (float)(a.rc2 * (1.0 + 3e-5)), lo = (float)(a.rc2 * (1.0 - 3e-5));
   // tile slot m < R: the last cell k with off[k] <= m (every lane takes part)
   auto cell_of = [&](int m) -> int {
     int k = 0;
@@ -953,21 +998,13 @@ __global__ void __launch_bounds__(256, 5) k_build_tile_wave(SearchArgs a, const 
         if (m < s1) {
           int j = ks + (m - ko);
           if (a.bin) j = a.bin[j];
-          const int o0 = k % 3 - 1, o1 = (k / 3) % 3 - 1, o2 = k / 9 - 1;
           const double4 p = a.pos[j];
-          keep[u] = (a.mask[j] & a.g2bit) != 0;
-          double x = p.x - org[0], y = p.y - org[1], z = p.z - org[2];
-          if (o0 < 0 && x > 0.0) x -= boxL.x; else if (o0 > 0 && x < 0.0) x += boxL.x;
-          if (o1 < 0 && y > 0.0) y -= boxL.y; else if (o1 > 0 && y < 0.0) y += boxL.y;
-          if (o2 < 0 && z > 0.0) z -= boxL.z; else if (o2 > 0 && z < 0.0) z += boxL.z;
-          if constexpr (PAIR) {
-            // bit 30: in list 1's candidate group, bit 31: in list 2's
-            const uint32_t mj = a.mask[j];
-            v[u].w = __uint_as_float((uint32_t)j | ((mj & a.g2bit1) ? 0x40000000u : 0u) |
-                                     ((mj & a.g2bit2) ? 0x80000000u : 0u));
-          } else {
-            v[u].w = __int_as_float(j);
-          }
+          const uint32_t mj = a.mask[j];
+          keep[u] = (mj & a.g2bit) != 0;
+          const double x = unwrap<false>(p.x - org[0], k % 3 - 1, boxL.x, nc[0]);
+          const double y = unwrap<false>(p.y - org[1], (k / 3) % 3 - 1, boxL.y, nc[1]);
+          const double z = unwrap<false>(p.z - org[2], k / 9 - 1, boxL.z, nc[2]);
+          v[u].w = staged_w<PAIR>(a, j, mj);
           if (keep[u]) { v[u].x = (float)x; v[u].y = (float)y; v[u].z = (float)z; }
         }
       }
@@ -1002,139 +1039,54 @@ __global__ void __launch_bounds__(256, 5) k_build_tile_wave(SearchArgs a, const 
     const int qq = q0 + lane / T;
     const bool inrow = qq < ncen;
     const int i = a.bin ? a.bin[cs + (inrow ? qq : 0)] : cs + (inrow ? qq : 0);
-    const uint32_t mi = a.mask[i];
-    // QUAD: rows of side b take its row index and its two lists
-    const bool sb = QUAD && (mi & a.g1mem_b) != 0;
-    const int row = inrow ? (sb ? a.row_of_b[i] : row_of[i]) : -1;
-    const bool active = row >= 0 && (mi & (sb ? a.g1bit_b : a.g1bit));
+    RowOut<T, PAIR, QUAD> ro(a, row_of, i, inrow);
     const double4 pi = a.pos[i];
     const float px = (float)(pi.x - org[0]), py = (float)(pi.y - org[1]), pz = (float)(pi.z - org[2]);
-    int* const nbr1 = sb ? a.nbr_b1 : a.nbr;
-    int* const nbr2 = sb ? a.nbr_b2 : a.nbr2;
-    int* const nnum1 = sb ? a.nnum_b1 : a.nnum;
-    int* const nnum2 = sb ? a.nnum_b2 : a.nnum2;
-    const int nmax1 = sb ? a.nmax_b1 : a.nmax, nmax2 = sb ? a.nmax_b2 : a.nmax2;
-    int* out = nbr1 + (size_t)(active ? row : 0) * (sb ? a.stride_b1 : a.stride);
-    int* out2 = PAIR ? nbr2 + (size_t)(active ? row : 0) * (sb ? a.stride_b2 : a.stride2) : nullptr;
-    int count = 0, count2 = 0;
-    // the row's hits of one round into one list: offsets from a prefix sum
-    // over the row's lanes, entries without the group bits
-    auto put = [&](unsigned hit, const float4* sv, int* o, int nmax, int& cnt) {
-      const int nh = __popc(hit);
-      int pre = nh;
-#pragma unroll
-      for (int d = 1; d < T; d <<= 1) {
-        int w = __shfl_up(pre, d, T);
-        if (t >= d) pre += w;
-      }
-      const int tot = __shfl(pre, T - 1, T);
-      int slot = cnt + pre - nh;
-      while (hit) {
-        const int b = __clz(hit);
-        hit &= ~(0x80000000u >> b);
-        if (slot < nmax) o[slot] = __float_as_int(sv[b * T].w) & ENTRY_IDX;
-        ++slot;
-      }
-      cnt += tot;
-    };
     for (int s0 = 0; s0 < R; s0 += WTILE) {
       if (!single) {
         wave_sync();
         np = stage(s0, R < s0 + WTILE ? R : s0 + WTILE);
         wave_sync();
       }
-      if (!active) continue;
+      if (!ro.active) continue;
       // the row atom's own staged slot when the pass is dense (else found by index)
-      const int own = (!CMP || dense) ? koff13 + qq - s0 : -1;
-      for (int c0 = 0; c0 < np; c0 += 32 * T) {
-        const float4* sv = st + c0 + t;
-        unsigned miss = 0u, inside = 0u;  // as in k_build_tile
-        unsigned m1 = 0u, m2 = 0u;        // PAIR: candidates in list 1's / list 2's group
-#pragma unroll 4
-        for (int b = 0; b < 32; ++b) {
-          const float4 w = sv[b * T];
-          float dx = w.x - px, dy = w.y - py, dz = w.z - pz;
-          const float m = fmaf(-dx, dx, fmaf(-dy, dy, fmaf(-dz, dz, hi)));
-          miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(m), 31);
-          inside = __builtin_amdgcn_alignbit(inside, __float_as_uint(win - m), 31);
-          if constexpr (PAIR) {
-            const uint32_t wb = __float_as_uint(w.w);
-            m1 = __builtin_amdgcn_alignbit(m1, wb << 1, 31);
-            m2 = __builtin_amdgcn_alignbit(m2, wb, 31);
-          }
-        }
-        unsigned hit = ~miss;
-        const int ob = own - c0 - t;
-        if (ob >= 0 && ob < 32 * T && ob % T == 0) hit &= ~(0x80000000u >> (ob / T));
-        unsigned chk = CMP && !dense ? hit : hit & ~inside;
-        while (chk) {
-          const int b = __clz(chk);
-          chk &= ~(0x80000000u >> b);
-          const float4 w = sv[b * T];
-          const int j = __float_as_int(w.w) & ENTRY_IDX;
-          float dx = w.x - px, dy = w.y - py, dz = w.z - pz;
-          if (CMP && !dense && j == i) {
-            hit &= ~(0x80000000u >> b);
-          } else if (fmaf(dx, dx, fmaf(dy, dy, dz * dz)) >= lo) {
-            double ex, ey, ez;
-            if (!(min_image_dist2(pi, a.pos[j], hb, ex, ey, ez) < a.rc2)) hit &= ~(0x80000000u >> b);
-          }
-        }
-        if constexpr (PAIR) {
-          put(hit & m1, sv, out, nmax1, count);
-          put(hit & m2, sv, out2, nmax2, count2);
-        } else {
-          put(hit, sv, out, a.nmax, count);
-        }
-      }
+      const bool find = CMP && !dense;
+      const int own = find ? -1 : koff13 + qq - s0;
+      ro.template scan<false>(a, im, st, np, t, own, find, pi, px, py, pz, hi, lo, hb);
     }
-    if (row >= 0 && !active && t == 0) {
-      nnum1[row] = 0;
-      if (PAIR) nnum2[row] = 0;
-    }
-    if (active && t == 0) {
-      nnum1[row] = count < nmax1 ? count : nmax1;
-      if (count > nmax1) raise_err(a.err, a.err_code, a.orig[i] + 1, count, a.step);
-      else if (a.exact && count != nmax1) raise_err(a.err, PFM_E_GRAPHENE_NN, a.orig[i] + 1, count, a.step);
-      if (PAIR) {
-        nnum2[row] = count2 < nmax2 ? count2 : nmax2;
-        if (count2 > nmax2) raise_err(a.err, a.err_code, a.orig[i] + 1, count2, a.step);
-      }
-    }
+    if (t == 0) ro.finish(a);
   }
 }
 
-template <int T>
-static void launch_build_T(pfm_ctx* h, SearchArgs& a, const int* row_of) {
-  long threads = (long)a.nrows * T;
-  int nb = (int)((threads + 255) / 256);
-  PFM_LAUNCH(h, "build_rows", k_build<T>, pad8(nb), 256, a, nb);
-}
-
-static void launch_build(pfm_ctx* h, SearchArgs& a, const int* row_of, bool sparse, bool sparse_cells) {
-  if (h->any_tile && sparse_cells) {
-    const int nc = h->ncell, nb = (nc + 3) / 4;
-    if (sparse) {
-      if (a.nmax <= 8) PFM_LAUNCH(h, "build_list", (k_build_tile_wave<4, true, false>), pad8(nb), 256, a, h->cell_xyz, row_of, nc, nb);
-      else PFM_LAUNCH(h, "build_list", (k_build_tile_wave<8, true, false>), pad8(nb), 256, a, h->cell_xyz, row_of, nc, nb);
-    } else {
-      if (a.nmax <= 8) PFM_LAUNCH(h, "build_list", (k_build_tile_wave<4, false, false>), pad8(nb), 256, a, h->cell_xyz, row_of, nc, nb);
-      else PFM_LAUNCH(h, "build_list", (k_build_tile_wave<8, false, false>), pad8(nb), 256, a, h->cell_xyz, row_of, nc, nb);
-    }
-  } else if (h->any_tile) {
-    int nb = h->ncell;
-    if (sparse) {
-      if (a.nmax <= 8) PFM_LAUNCH(h, "build_list", (k_build_tile<4, true>), pad8(nb), 256, a, h->cell_xyz, row_of, nb);
-      else PFM_LAUNCH(h, "build_list", (k_build_tile<8, true>), pad8(nb), 256, a, h->cell_xyz, row_of, nb);
-    } else {
-      if (a.nmax <= 8) PFM_LAUNCH(h, "build_list", (k_build_tile<4, false>), pad8(nb), 256, a, h->cell_xyz, row_of, nb);
-      else PFM_LAUNCH(h, "build_list", (k_build_tile<8, false>), pad8(nb), 256, a, h->cell_xyz, row_of, nb);
+// one list (or with PAIR / QUAD the lists of a pair or two) by the kernel the
+// list takes: one wave per cell (ListDev::wave_cells) or one workgroup; the
+// cells of grids under three cells wide by a launch of their own
+template <bool PAIR, bool QUAD>
+static void launch_build(pfm_ctx* h, SearchArgs& a, const int* row_of, bool sparse, bool wave_cells) {
+  const int nc = h->ncell, nbw = (nc + 3) / 4;
+  const bool narrow = !PAIR && a.nmax <= 8;  // four lanes a row
+#define BUILD_AS(T, CMP)                                                                                           \
+  do {                                                                                                             \
+    if (h->n_narrow < nc && wave_cells)                                                                            \
+      PFM_LAUNCH(h, "build_list", (k_build_tile_wave<T, CMP, PAIR, QUAD>), pad8(nbw), 256, a, h->cell_xyz, row_of, \
+                 nc, nbw);                                                                                         \
+    else if (h->n_narrow < nc)                                                                                     \
+      PFM_LAUNCH(h, "build_list", (k_build_tile<T, CMP, PAIR, QUAD, false>), pad8(nc), 256, a, h->cell_xyz,        \
+                 row_of, nc, (const int*)nullptr);                                                                 \
+    if (h->n_narrow)                                                                                               \
+      PFM_LAUNCH(h, "build_list", (k_build_tile<T, CMP, PAIR, QUAD, true>), pad8(h->n_narrow), 256, a,             \
+                 h->cell_xyz, row_of, h->n_narrow, h->narrow_cells);                                               \
+  } while (0)
+  if constexpr (!PAIR) {
+    if (narrow) {
+      if (sparse) BUILD_AS(4, true);
+      else BUILD_AS(4, false);
+      return;
     }
   }
-  if (h->any_rows) {
-    if (a.nmax <= 8) launch_build_T<4>(h, a, row_of);
-    else launch_build_T<8>(h, a, row_of);
-  }
+  if (sparse) BUILD_AS(8, true);
+  else BUILD_AS(8, false);
+#undef BUILD_AS
 }
 
 // Build list k (0-based) of interaction ii.  For lj/ljc/morsec, list 1 is the
@@ -1182,6 +1134,10 @@ static SearchArgs search_args(pfm_ctx* h, int ii, int k, int step) {
 static void list_post(pfm_ctx* h, int ii, int k, int step) {
   Inter& it = h->inter[ii];
   ListDev& L = it.nl[k];
+  if (L.nrows == 0) {
+    L.built = true;
+    return;
+  }
   int nb = (L.nrows + 255) / 256;
   if (it.kind == PFM_TB || it.kind == PFM_REBOSC || (k == 2 && !(int)it.p[it.kind == PFM_LJC ? 5 : 6])) {
     PFM_LAUNCH(h, "list_rev", k_rev, nb, 256, L.nrows, h->grp.rows[L.g1], h->grp.row_of[L.g1], L.nnum, L.nbr,
@@ -1206,21 +1162,18 @@ int launch_build_list(pfm_ctx* h, int ii, int k, int step) {
   if (L.nrows == 0) { L.built = true; return PFM_OK; }
   SearchArgs a = search_args(h, ii, k, step);
   // candidates of another species: stage only those
-  launch_build(h, a, h->grp.row_of[L.g1], 2L * h->grp.size[L.g2] < (long)h->N, L.sparse_cells);
+  launch_build<false, false>(h, a, h->grp.row_of[L.g1], 2L * h->grp.size[L.g2] < (long)h->N, L.wave_cells);
   list_post(h, ii, k, step);
   return PFM_OK;
 }
 
-// Two lists of one pair (ListDev::pair): one wavefront-per-cell pass stages
-// the union of their candidate groups once and writes both (replicas that
-// take the row search run it per list).
+// Two lists of one pair (ListDev::pair): one pass stages the union of their
+// candidate groups once and writes both.
 int launch_build_pair(pfm_ctx* h, int ii, int k, int jj, int kk, int step) {
   ListDev& L1 = h->inter[ii].nl[k];
-  ListDev& L2 = h->inter[jj].nl[kk];
   SearchArgs a = search_args(h, ii, k, step);
   SearchArgs b = search_args(h, jj, kk, step);
-  const int* row_of = h->grp.row_of[L1.g1];
-  if (h->any_tile && L1.nrows > 0) {
+  if (L1.nrows > 0) {
     SearchArgs p = a;
     p.g2bit1 = a.g2bit;
     p.g2bit2 = b.g2bit;
@@ -1229,15 +1182,7 @@ int launch_build_pair(pfm_ctx* h, int ii, int k, int jj, int kk, int step) {
     p.stride2 = b.stride;
     p.nnum2 = b.nnum;
     p.nbr2 = b.nbr;
-    const int nc = h->ncell, nb = (nc + 3) / 4;
-    if (L1.pair_sparse)
-      PFM_LAUNCH(h, "build_list", (k_build_tile_wave<8, true, true>), pad8(nb), 256, p, h->cell_xyz, row_of, nc, nb);
-    else
-      PFM_LAUNCH(h, "build_list", (k_build_tile_wave<8, false, true>), pad8(nb), 256, p, h->cell_xyz, row_of, nc, nb);
-  }
-  if (h->any_rows) {
-    if (L1.nrows > 0) launch_build_T<8>(h, a, row_of);
-    if (L2.nrows > 0) launch_build_T<8>(h, b, row_of);
+    launch_build<true, false>(h, p, h->grp.row_of[L1.g1], L1.pair_sparse, L1.wave_cells);
   }
   list_post(h, ii, k, step);
   list_post(h, jj, kk, step);
@@ -1254,9 +1199,7 @@ int launch_build_quad(pfm_ctx* h, int ii, int k, int jj, int kk, int b1i, int b1
   SearchArgs b = search_args(h, jj, kk, step);
   SearchArgs c = search_args(h, b1i, b1k, step);
   SearchArgs d = search_args(h, b2i, b2k, step);
-  const int* row_of = h->grp.row_of[L1.g1];
-  const int* row_of_b = h->grp.row_of[B1.g1];
-  if (h->any_tile && (L1.nrows > 0 || B1.nrows > 0)) {
+  if (L1.nrows > 0 || B1.nrows > 0) {
     SearchArgs p = a;
     p.g2bit1 = a.g2bit;
     p.g2bit2 = b.g2bit;
@@ -1265,18 +1208,10 @@ int launch_build_quad(pfm_ctx* h, int ii, int k, int jj, int kk, int b1i, int b1
     p.g1bit_b = c.g1bit;
     p.g1mem_b = c.g1mem;
     p.g1mem = a.g1mem | c.g1mem;
-    p.row_of_b = row_of_b;
+    p.row_of_b = h->grp.row_of[B1.g1];
     p.nmax_b1 = c.nmax; p.stride_b1 = c.stride; p.nnum_b1 = c.nnum; p.nbr_b1 = c.nbr;
     p.nmax_b2 = d.nmax; p.stride_b2 = d.stride; p.nnum_b2 = d.nnum; p.nbr_b2 = d.nbr;
-    const int nc = h->ncell, nb = (nc + 3) / 4;
-    if (L1.pair_sparse)
-      PFM_LAUNCH(h, "build_list", (k_build_tile_wave<8, true, true, true>), pad8(nb), 256, p, h->cell_xyz, row_of, nc, nb);
-    else
-      PFM_LAUNCH(h, "build_list", (k_build_tile_wave<8, false, true, true>), pad8(nb), 256, p, h->cell_xyz, row_of, nc, nb);
-  }
-  if (h->any_rows) {
-    if (L1.nrows > 0) { launch_build_T<8>(h, a, row_of); launch_build_T<8>(h, b, row_of); }
-    if (B1.nrows > 0) { launch_build_T<8>(h, c, row_of_b); launch_build_T<8>(h, d, row_of_b); }
+    launch_build<true, true>(h, p, h->grp.row_of[L1.g1], L1.pair_sparse, L1.wave_cells);
   }
   list_post(h, ii, k, step);
   list_post(h, jj, kk, step);
