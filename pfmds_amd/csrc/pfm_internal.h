@@ -136,6 +136,12 @@ __device__ __forceinline__ void sqrt_rsqrt(double d2, double& r, double& ir) {
   const double s = d2 * ir;
   r = fma(fma(-s, s, d2), 0.5 * ir, s);
 }
+// sqrt(d2) for normal d2 > 0 (d2 = 0: NaN)
+__device__ __forceinline__ double sqrt(double d2) {
+  double r, ir;
+  sqrt_rsqrt(d2, r, ir);
+  return r;
+}
 // 2^n (1 + r + r^2 ...): e**r for |r| <= ln2/2 by degree 11, scaled
 __device__ __forceinline__ double exp_tail(double r, double n) {
   double q = sc(0x1.af2391d7f5e6cp-26);
@@ -231,7 +237,7 @@ __device__ __forceinline__ double pow(double x, double y) {
 template <class R> struct PM;
 template <> struct PM<double> {
   static __device__ __forceinline__ double exp_(double x) { return f64::exp(x); }
-  static __device__ __forceinline__ double sqrt_(double x) { return sqrt(x); }
+  static __device__ __forceinline__ double sqrt_(double x) { return f64::sqrt(x); }
   static __device__ __forceinline__ double rcp(double x) { return f64::rcp(x); }
   static __device__ __forceinline__ double cos_(double x) { return cos(x); }
   static __device__ __forceinline__ double sin_(double x) { return sin(x); }

@@ -93,7 +93,8 @@ def test_dimer_scan(name):
     np.testing.assert_array_equal(f[:, 0], -f[:, 1])
 
 
-@pytest.mark.parametrize("kind,delt", [("morsec", 0.5), ("morsec", 1.0), ("morsec", 3.3), ("ljc", 2.7), ("ljc", 4.0)])
+@pytest.mark.parametrize("kind,delt", [("morsec", 0.5), ("morsec", 1.0), ("morsec", 2.0), ("morsec", 3.3), ("ljc", 2.7), ("ljc", 3.0),
+                                       ("ljc", 4.0), ("ljc", 5.0)])
 def test_cosine_exponents(kind, delt):
     s = configs.graphene_on_cu(cx=14, cy=8, gx=14, gy=8, layers=4, seed=31, jitter=0.1)
     lists = s.interactions[2].lists
