@@ -710,7 +710,7 @@ static int finalize(pfm_ctx* h) {
   h->hrep.assign(nrep, RepDev());
   std::vector<int> rank_all, xyz_all, crep_all;
   h->ncell = 0;
-  std::vector<int> narrow_all;
+  h->any_narrow = false;
   for (int r = 0; r < nrep; ++r) {
     RepDev& R = h->hrep[r];
     memset(&R, 0, sizeof R);
@@ -737,7 +737,7 @@ static int finalize(pfm_ctx* h) {
     R.clen = make_double3(cl[0], cl[1], cl[2]);
     R.inv_clen = make_double3(1.0 / cl[0], 1.0 / cl[1], 1.0 / cl[2]);
     R.cell_base = h->ncell;
-    const bool narrow = nc[0] < 3 || nc[1] < 3 || nc[2] < 3;
+    h->any_narrow = h->any_narrow || nc[0] < 3 || nc[1] < 3 || nc[2] < 3;
     R.zlo = 0.8 * bx[2];
     R.zhi = 0.9 * bx[2];
     const int ncr = nc[0] * nc[1] * nc[2];
@@ -757,7 +757,6 @@ static int finalize(pfm_ctx* h) {
       rank_all[h->ncell + lin] = h->ncell + k;
       xyz_all[h->ncell + k] = x | (y << 10) | (z << 20);
       crep_all[h->ncell + k] = r;
-      if (narrow) narrow_all.push_back(h->ncell + k);
     }
     h->ncell += ncr;
   }
@@ -771,12 +770,6 @@ static int finalize(pfm_ctx* h) {
   HIPCHK(h, hipMemcpyAsync(h->cell_rank, rank_all.data(), sizeof(int) * h->ncell, hipMemcpyHostToDevice, h->stream));
   if ((rc = dalloc(h, &h->cell_xyz, h->ncell))) return rc;
   HIPCHK(h, hipMemcpyAsync(h->cell_xyz, xyz_all.data(), sizeof(int) * h->ncell, hipMemcpyHostToDevice, h->stream));
-  h->n_narrow = (int)narrow_all.size();
-  if (h->n_narrow) {
-    if ((rc = dalloc(h, &h->narrow_cells, h->n_narrow))) return rc;
-    HIPCHK(h, hipMemcpyAsync(h->narrow_cells, narrow_all.data(), sizeof(int) * h->n_narrow, hipMemcpyHostToDevice,
-                             h->stream));
-  }
   if (nrep > 1) {
     if ((rc = dalloc(h, &h->cell_rep, h->ncell))) return rc;
     HIPCHK(h, hipMemcpyAsync(h->cell_rep, crep_all.data(), sizeof(int) * h->ncell, hipMemcpyHostToDevice, h->stream));
@@ -2814,7 +2807,7 @@ int pfm_destroy(pfm_ctx* h) {
   for (auto e : h->rec.free_ev) (void)hipEventDestroy(e);
   auto F = [](void* p) { if (p) (void)hipFree(p); };
   F(h->pos4); F(h->vel4); F(h->frc4); F(h->pos4b); F(h->vel4b); F(h->frc4b); F(h->mask); F(h->maskb);
-  F(h->orig); F(h->origb); F(h->perm); F(h->atom_rank); F(h->scan_tmp); F(h->eb); F(h->qpos); F(h->rdev); F(h->rep); F(h->repb); F(h->cell_rep); F(h->narrow_cells); F(h->d_rep_row0); F(h->d_rep_out);
+  F(h->orig); F(h->origb); F(h->perm); F(h->atom_rank); F(h->scan_tmp); F(h->eb); F(h->qpos); F(h->rdev); F(h->rep); F(h->repb); F(h->cell_rep); F(h->d_rep_row0); F(h->d_rep_out);
   F(h->red_part); F(h->red_out); F(h->derr); F(h->cell_rank); F(h->cell_count); F(h->cell_start); F(h->cell_xyz);
   F(h->nhc_state);
   F(h->xfer);

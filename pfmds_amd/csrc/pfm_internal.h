@@ -586,9 +586,7 @@ struct pfm_ctx {
   RepDev* rdev = nullptr;             // [nrep]
   int *rep = nullptr, *repb = nullptr;  // [N] replica of every internal atom (batches only)
   int* cell_rep = nullptr;            // [ncell] replica of every cell (batches only)
-  // cells of grids under three cells wide in some direction
-  int* narrow_cells = nullptr;
-  int n_narrow = 0;
+  bool any_narrow = false;  // some replica's grid is under three cells wide in some direction
   // per replica and group: first row of the replica in the group's rows
   std::vector<int> rep_row0[PFM_MAXG + 1];
   int* d_rep_row0 = nullptr;  // [(PFM_MAXG + 1) * (nrep + 1)]; slot 0: first internal atom of every replica

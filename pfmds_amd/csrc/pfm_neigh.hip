@@ -540,17 +540,19 @@ __global__ void k_nn_from_tb(int nrows, const int* __restrict__ rows, const int*
 // image (TileImage), nine more instructions a candidate.  A row-by-row search
 // of such grids, whose candidates wait on two dependent loads each, took 45 us
 // for a 256-atom Cu replica's list.
-// The cells of such grids go through launches of their own (IMG, over
-// pfm_ctx::narrow_cells): a kernel that held both scans searched a
-// 131,072-atom Cu crystal in 67 us instead of 63.
+// Handles with such a grid take the IMG kernels, which hold both scans and
+// choose by cell (launches of their own for the narrow cells waited on 28 us
+// of dependent steps each: a 12-replica batch's step 37.2 -> 33.6 us without).
 __device__ __forceinline__ bool narrow_grid(const RepDev& R) { return R.nc[0] < 3 || R.nc[1] < 3 || R.nc[2] < 3; }
 struct TileImage {
   float3 L, iL;  // box and its inverse in the directions under three cells wide, 0 in the others
+  // a value equal on all lanes, in a scalar register
+  static __device__ __forceinline__ float uni(bool on, double x) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(on ? (float)x : 0.f)));
+  }
   __device__ __forceinline__ TileImage(const RepDev& R)
-      : L(make_float3(R.nc[0] < 3 ? (float)R.L.x : 0.f, R.nc[1] < 3 ? (float)R.L.y : 0.f,
-                      R.nc[2] < 3 ? (float)R.L.z : 0.f)),
-        iL(make_float3(R.nc[0] < 3 ? (float)R.iL.x : 0.f, R.nc[1] < 3 ? (float)R.iL.y : 0.f,
-                       R.nc[2] < 3 ? (float)R.iL.z : 0.f)) {}
+      : L(make_float3(uni(R.nc[0] < 3, R.L.x), uni(R.nc[1] < 3, R.L.y), uni(R.nc[2] < 3, R.L.z))),
+        iL(make_float3(uni(R.nc[0] < 3, R.iL.x), uni(R.nc[1] < 3, R.iL.y), uni(R.nc[2] < 3, R.iL.z))) {}
   // the nearest image of a difference; the clamp keeps far-away padding far
   static __device__ __forceinline__ float near(float d, float L, float iL) {
     return fmaf(-L, rintf(__builtin_amdgcn_fmed3f(d * iL, -2.0f, 2.0f)), d);
@@ -671,10 +673,11 @@ struct RowOut {
   // one pass over np staged candidates (whole rounds of 32 T); own: the row
   // atom's staged slot, or -1 to find it by index (find_self)
   template <bool IMG>
-  __device__ __forceinline__ void scan(const SearchArgs& a, const TileImage& im, const float4* st, int np, int t,
+  __device__ __forceinline__ void scan(const SearchArgs& a, const RepDev& RG, const float4* st, int np, int t,
                                        int own, bool find_self, const double4& pi, float px, float py, float pz,
                                        float hi, float lo, const double3& hb) {
     const float win = hi - lo;
+    const TileImage im(RG);
     for (int c0 = 0; c0 < np; c0 += 32 * T) {
       // bit 31-b <-> candidate slot c0 + t + b*T
       const float4* sv = st + c0 + t;
@@ -763,18 +766,15 @@ __device__ __forceinline__ void empty_rows(const SearchArgs& a, const int* __res
 
 template <int T, bool CMP, bool PAIR, bool QUAD, bool IMG>
 __global__ void __launch_bounds__(256, CMP || PAIR ? 5 : 6) k_build_tile(SearchArgs a, const int* __restrict__ rank_xyz,
-                                                    const int* __restrict__ row_of, int nblocks_real,
-                                                    const int* __restrict__ cells) {
+                                                    const int* __restrict__ row_of, int nblocks_real) {
   static_assert(TILE_MAX % (32 * T) == 0, "tile passes hold whole bitmask rounds");
   __shared__ float4 st[TILE_MAX];
   __shared__ TileCells tc;
   int c = xcd_block(nblocks_real);
   if (c < 0) return;
-  if (IMG) c = cells[c];
   const int ncen = a.cell_count[c];
   if (ncen == 0 || !(a.cell_grp[c] & a.g1mem)) return;  // no member of group 1 in the cell
   const RepDev& RG = a.rdev[a.cell_rep ? a.cell_rep[c] : 0];
-  if (!IMG && narrow_grid(RG)) return;  // searched by the IMG launch
   const int cs = a.cell_start[c];
   const int tid = threadIdx.x;
   // (cells without a row of this list, another species or another
@@ -784,7 +784,6 @@ __global__ void __launch_bounds__(256, CMP || PAIR ? 5 : 6) k_build_tile(SearchA
   const double org[3] = {cc[0] * RG.clen.x, cc[1] * RG.clen.y, cc[2] * RG.clen.z};
   const double3 boxL = RG.L, hb = RG.hb;
   const int nc[3] = {RG.nc[0], RG.nc[1], RG.nc[2]};
-  const TileImage im(RG);
   bool cand = false;
   if (tid < 27) {
     int q[3];
@@ -895,7 +894,8 @@ __global__ void __launch_bounds__(256, CMP || PAIR ? 5 : 6) k_build_tile(SearchA
       // the row atom's own staged slot when the pass is dense (else found by index)
       const bool find = CMP && !dense;
       const int own = find ? -1 : tc.off[13] + qq - s0;
-      ro.template scan<IMG>(a, im, st, np, t, own, find, pi, px, py, pz, hi, lo, hb);
+      if (IMG && narrow_grid(RG)) ro.template scan<true>(a, RG, st, np, t, own, find, pi, px, py, pz, hi, lo, hb);
+      else ro.template scan<false>(a, RG, st, np, t, own, find, pi, px, py, pz, hi, lo, hb);
     }
     if (t == 0) ro.finish(a);
   }
@@ -930,7 +930,6 @@ __global__ void __launch_bounds__(256, 5) k_build_tile_wave(SearchArgs a, const 
   const int ncen = a.cell_count[c];
   if (ncen == 0 || !(a.cell_grp[c] & a.g1mem)) return;  // no member of group 1 in the cell
   const RepDev& RG = a.rdev[a.cell_rep ? a.cell_rep[c] : 0];
-  if (narrow_grid(RG)) return;  // searched by k_build_tile's IMG launch
   const int cs = a.cell_start[c];
   float4* st = stw[wv];
   const int pk = rank_xyz[c];
@@ -938,7 +937,6 @@ __global__ void __launch_bounds__(256, 5) k_build_tile_wave(SearchArgs a, const 
   const double org[3] = {cc[0] * RG.clen.x, cc[1] * RG.clen.y, cc[2] * RG.clen.z};
   const double3 boxL = RG.L, hb = RG.hb;
   const int nc[3] = {RG.nc[0], RG.nc[1], RG.nc[2]};
-  const TileImage im(RG);
   // the 27 tile cells in lanes 0..26: first atom, count, exclusive offset
   int kst = 0, kcn = 0;
   bool cand = false;
@@ -1052,30 +1050,30 @@ __global__ void __launch_bounds__(256, 5) k_build_tile_wave(SearchArgs a, const 
       // the row atom's own staged slot when the pass is dense (else found by index)
       const bool find = CMP && !dense;
       const int own = find ? -1 : koff13 + qq - s0;
-      ro.template scan<false>(a, im, st, np, t, own, find, pi, px, py, pz, hi, lo, hb);
+      ro.template scan<false>(a, RG, st, np, t, own, find, pi, px, py, pz, hi, lo, hb);
     }
     if (t == 0) ro.finish(a);
   }
 }
 
 // one list (or with PAIR / QUAD the lists of a pair or two) by the kernel the
-// list takes: one wave per cell (ListDev::wave_cells) or one workgroup; the
-// cells of grids under three cells wide by a launch of their own
+// list takes: one wave per cell (ListDev::wave_cells) or one workgroup, the
+// latter with the nearest-image scan when some grid is under three cells wide
 template <bool PAIR, bool QUAD>
 static void launch_build(pfm_ctx* h, SearchArgs& a, const int* row_of, bool sparse, bool wave_cells) {
   const int nc = h->ncell, nbw = (nc + 3) / 4;
   const bool narrow = !PAIR && a.nmax <= 8;  // four lanes a row
 #define BUILD_AS(T, CMP)                                                                                           \
   do {                                                                                                             \
-    if (h->n_narrow < nc && wave_cells)                                                                            \
+    if (h->any_narrow)                                                                                             \
+      PFM_LAUNCH(h, "build_list", (k_build_tile<T, CMP, PAIR, QUAD, true>), pad8(nc), 256, a, h->cell_xyz, row_of, \
+                 nc);                                                                                              \
+    else if (wave_cells)                                                                                           \
       PFM_LAUNCH(h, "build_list", (k_build_tile_wave<T, CMP, PAIR, QUAD>), pad8(nbw), 256, a, h->cell_xyz, row_of, \
                  nc, nbw);                                                                                         \
-    else if (h->n_narrow < nc)                                                                                     \
+    else                                                                                                           \
       PFM_LAUNCH(h, "build_list", (k_build_tile<T, CMP, PAIR, QUAD, false>), pad8(nc), 256, a, h->cell_xyz,        \
-                 row_of, nc, (const int*)nullptr);                                                                 \
-    if (h->n_narrow)                                                                                               \
-      PFM_LAUNCH(h, "build_list", (k_build_tile<T, CMP, PAIR, QUAD, true>), pad8(h->n_narrow), 256, a,             \
-                 h->cell_xyz, row_of, h->n_narrow, h->narrow_cells);                                               \
+                 row_of, nc);                                                                                      \
   } while (0)
   if constexpr (!PAIR) {
     if (narrow) {
