@@ -414,12 +414,11 @@ struct LjP {
   double eps4, sig, R1, R2, invw;
 };
 
-// (E with a.e_row null: the converse rows nl(2), which carry no energy)
+// a row's lj entries into acc
 template <int T, class R, bool E>
-__device__ __forceinline__ void lj_rows(const RowArgs& a, const LjP& P, int blk) {
-  ROW_PROLOGUE_AT(T, blk)
+__device__ __forceinline__ void lj_walk(const LjP& P, const Geo<R>& G, const typename Geo<R>::P& pi,
+                                        const int* __restrict__ nbrow, int n, int t, int i, RowAcc<R>& acc) {
   const R R1 = P.R1, R2 = P.R2, invw = P.invw, sig = P.sig, e4 = P.eps4, kdf = -0.5 * PFM_PI * P.invw;
-  RowAcc<R> acc;
   walk_row<T, R>(G, nbrow, n, t, i, [&](int, const typename Geo<R>::P& q, bool valid) {
     R dx, dy, dz;
     R r, ir;
@@ -436,6 +435,14 @@ __device__ __forceinline__ void lj_rows(const RowArgs& a, const LjP& P, int blk)
       acc.energy(in ? v : R(0));
     }
   }, [&] { acc.flush(); });
+}
+
+// (E with a.e_row null: the converse rows nl(2), which carry no energy)
+template <int T, class R, bool E>
+__device__ __forceinline__ void lj_rows(const RowArgs& a, const LjP& P, int blk) {
+  ROW_PROLOGUE_AT(T, blk)
+  RowAcc<R> acc;
+  lj_walk<T, R, E>(P, G, pi, nbrow, n, t, i, acc);
   const double fx = group_sum<T>(acc.fx), fy = group_sum<T>(acc.fy), fz = group_sum<T>(acc.fz);
   const double e = E ? group_sum<T>(acc.e) : 0.0;
   if (t == 0) {
@@ -459,12 +466,11 @@ struct Lj1gP {
 };
 
 // The weights come from the entries' tags (k_lj1g_tag): bit 30 the pair is in
-// i's half list, bit 31 in j's.
+// i's half list, bit 31 in j's.  A row's entries into acc.
 template <int T, class R, bool E>
-__device__ __forceinline__ void lj1g_rows(const RowArgs& a, const Lj1gP& P, int blk) {
-  ROW_PROLOGUE_AT(T, blk)
+__device__ __forceinline__ void lj1g_walk(const Lj1gP& P, const Geo<R>& G, const typename Geo<R>::P& pi,
+                                          const int* __restrict__ nbrow, int n, int t, int i, RowAcc<R>& acc) {
   const R R1 = P.R1, R2 = P.R2, invw = P.invw, c6 = P.c6, c12 = P.c12, c6t6 = P.c6t6, c12t12 = P.c12t12;
-  RowAcc<R> acc;
   walk_row_tag<T, R>(G, nbrow, n, t, i, [&](const typename Geo<R>::P& q, unsigned tag, bool valid) {
     int wh = valid && (tag & 1u) ? 1 : 0;
     int w = wh + (valid && (tag & 2u) ? 1 : 0);
@@ -497,11 +503,49 @@ __device__ __forceinline__ void lj1g_rows(const RowArgs& a, const Lj1gP& P, int 
       acc.energy(wh ? v : R(0));
     }
   }, [&] { acc.flush(); });
+}
+
+template <int T, class R, bool E>
+__device__ __forceinline__ void lj1g_rows(const RowArgs& a, const Lj1gP& P, int blk) {
+  ROW_PROLOGUE_AT(T, blk)
+  RowAcc<R> acc;
+  lj1g_walk<T, R, E>(P, G, pi, nbrow, n, t, i, acc);
   const double fx = group_sum<T>(acc.fx), fy = group_sum<T>(acc.fy), fz = group_sum<T>(acc.fz);
   const double e = E ? group_sum<T>(acc.e) : 0.0;
   if (t == 0) {
     write_force(a, i, fx, fy, fz);
     if (E) a.e_row[row] = e;
+  }
+}
+
+// lj1g rows and the lj rows of the same atoms (a species' own pairs, then its
+// pairs with the other species) in one pass: the row atom's loads, the
+// reduction and the force write are shared, and a binary gas's forces need
+// one launch instead of two
+struct LjRows {
+  int stride;
+  const int* nnum;
+  const int* nbr;
+  double* e_row;  // null: the converse rows nl(2)
+  LjP p;
+};
+template <int T, class R, bool E>
+__device__ __forceinline__ void lj_both_rows(const RowArgs& a, const Lj1gP& P, const LjRows& b, int blk) {
+  ROW_PROLOGUE_AT(T, blk)
+  const int n2 = b.nnum[row];
+  RowAcc<R> acc;
+  lj1g_walk<T, R, E>(P, G, pi, nbrow, n, t, i, acc);
+  const double e1 = acc.e;
+  acc.e = 0;
+  lj_walk<T, R, E>(b.p, G, pi, b.nbr + (size_t)row * b.stride, n2, t, i, acc);
+  const double fx = group_sum<T>(acc.fx), fy = group_sum<T>(acc.fy), fz = group_sum<T>(acc.fz);
+  const double es = E ? group_sum<T>(e1) : 0.0, el = E ? group_sum<T>(acc.e) : 0.0;
+  if (t == 0) {
+    write_force(a, i, fx, fy, fz);
+    if (E) {
+      a.e_row[row] = es;
+      if (b.e_row) b.e_row[row] = el;
+    }
   }
 }
 
@@ -1030,7 +1074,7 @@ __global__ void __launch_bounds__(256) k_cos_nn_metal(RowArgs an, RowArgs am, Co
 // each sub-range is XCD-remapped on its own.
 
 #define MULTI_MAXP 6
-enum MultiKind { MK_LJ1G = 0, MK_LJ = 1, MK_RJL_DENSITY = 2, MK_RJL_FORCE = 3 };
+enum MultiKind { MK_LJ1G = 0, MK_LJ = 1, MK_RJL_DENSITY = 2, MK_RJL_FORCE = 3, MK_LJ_BOTH = 4 };
 struct MultiPass {
   int kind, start, np, nb;  // first block of the sub-range, its padded and real block counts
   RowArgs a;
@@ -1040,6 +1084,7 @@ struct MultiPass {
     Lj1gP lj1g;
   } p;
   double* eb;
+  LjRows lj;  // MK_LJ_BOTH
 };
 struct MultiArgs {
   int n;
@@ -1057,6 +1102,7 @@ __global__ void __launch_bounds__(256) k_multi(MultiArgs A) {
   switch (S.kind) {
     case MK_LJ1G: lj1g_rows<T, R, E>(S.a, S.p.lj1g, lb); break;
     case MK_LJ: lj_rows<T, R, E>(S.a, S.p.lj, lb); break;
+    case MK_LJ_BOTH: lj_both_rows<T, R, E>(S.a, S.p.lj1g, S.lj, lb); break;
     case MK_RJL_DENSITY: rjl_density_rows<T, R>(S.a, S.p.rjl, S.eb, lb); break;
     default: rjl_force_rows<T, R, E>(S.a, S.p.rjl, S.eb, lb); break;
   }
@@ -1198,7 +1244,8 @@ static Lj1gP lj1g_params(const Inter& it) {
                it.p[2], it.p[3], 1.0 / (it.p[3] - it.p[2])};
 }
 
-// Phases of lj / lj1g / rjl passes: each pass goes into the earliest phase
+// Phases of lj / lj1g / rjl passes (an lj1g takes the lj list of its own rows
+// into its pass): each pass goes into the earliest phase
 // after its prerequisite (an rjl force after its density) holding no pass
 // that writes any of its atoms (forces, or the density's per-atom value).
 // Worth it when fewer launches result; other interactions keep separate
@@ -1213,17 +1260,42 @@ static void plan_multi(pfm_ctx* h) {
     int group, after;
   };
   std::vector<P> passes;
+  // an lj list whose rows are an lj1g's rows goes into that lj1g's pass
+  std::vector<std::pair<int, int>> taken;
+  auto partner = [&](int g) -> std::pair<int, int> {
+    for (size_t jj = 0; jj < h->inter.size(); ++jj)
+      for (int k = 0; k < 2; ++k) {
+        const std::pair<int, int> c{(int)jj, k};
+        if (h->inter[jj].kind == PFM_LJ && h->inter[jj].nl[k].g1 == g &&
+            std::find(taken.begin(), taken.end(), c) == taken.end())
+          return c;
+      }
+    return {-1, 0};
+  };
+  size_t launches = 0;  // of the passes one by one
+  for (size_t ii = 0; ii < h->inter.size(); ++ii) {
+    const Inter& it = h->inter[ii];
+    if (it.kind == PFM_LJ1G) {
+      const auto c = partner(it.nl[0].g1);
+      if (c.first >= 0) taken.push_back(c);
+      passes.push_back({{(int)ii, c.first >= 0 ? MK_LJ_BOTH : MK_LJ1G, 0, false, c.first, c.second}, it.nl[0].g1, -1});
+      launches += c.first >= 0 ? 2 : 1;
+    }
+  }
   for (size_t ii = 0; ii < h->inter.size(); ++ii) {
     const Inter& it = h->inter[ii];
     const int I = (int)ii;
-    if (it.kind == PFM_LJ1G) {
-      passes.push_back({{I, MK_LJ1G, 0}, it.nl[0].g1, -1});
-    } else if (it.kind == PFM_LJ) {
-      for (int k = 0; k < 2; ++k) passes.push_back({{I, MK_LJ, k}, it.nl[k].g1, -1});
+    if (it.kind == PFM_LJ) {
+      for (int k = 0; k < 2; ++k)
+        if (std::find(taken.begin(), taken.end(), std::make_pair(I, k)) == taken.end()) {
+          passes.push_back({{I, MK_LJ, k, false, -1, 0}, it.nl[k].g1, -1});
+          ++launches;
+        }
     } else if (it.kind == PFM_RJL) {
-      passes.push_back({{I, MK_RJL_DENSITY, 0}, it.nl[0].g1, -1});
-      passes.push_back({{I, MK_RJL_FORCE, 0}, it.nl[0].g1, (int)passes.size() - 1});
-    } else {
+      passes.push_back({{I, MK_RJL_DENSITY, 0, false, -1, 0}, it.nl[0].g1, -1});
+      passes.push_back({{I, MK_RJL_FORCE, 0, false, -1, 0}, it.nl[0].g1, (int)passes.size() - 1});
+      launches += 2;
+    } else if (it.kind != PFM_LJ1G) {
       return;
     }
   }
@@ -1255,7 +1327,7 @@ static void plan_multi(pfm_ctx* h) {
     phase_of[a] = ph;
     nphase = std::max(nphase, ph + 1);
   }
-  if (nphase >= (int)passes.size()) return;
+  if (nphase >= (int)launches) return;
   M.phases.assign(nphase, {});
   for (size_t a = 0; a < passes.size(); ++a) M.phases[phase_of[a]].push_back(passes[a].pass);
   // first writers in launch order (phases in turn; the passes of a phase
@@ -1316,10 +1388,15 @@ static int multi_forces(pfm_ctx* h, bool energy, bool first) {
       S.a = row_args(h, it, ps.list, first && ps.first ? 0 : 1);
       if (S.a.nrows == 0) continue;
       if (ps.kind == MK_LJ && ps.list == 1) S.a.e_row = nullptr;  // nl(2) rows carry no energy
-      if (ps.kind == MK_LJ1G) S.p.lj1g = lj1g_params(it);
+      if (ps.kind == MK_LJ1G || ps.kind == MK_LJ_BOTH) S.p.lj1g = lj1g_params(it);
       else if (ps.kind == MK_LJ) S.p.lj = lj_params(it);
       else S.p.rjl = rjl_params(it);
       S.eb = h->eb;
+      if (ps.kind == MK_LJ_BOTH) {
+        Inter& jt = h->inter[ps.inter2];
+        const ListDev& L2 = jt.nl[ps.list2];
+        S.lj = LjRows{L2.stride, L2.nnum, L2.nbr, ps.list2 == 0 ? jt.e_row : nullptr, lj_params(jt)};
+      }
       S.nb = row_blocks(S.a.nrows, T, BS);
       S.np = pad8(S.nb);
       S.start = start;

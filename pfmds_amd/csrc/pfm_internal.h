@@ -670,8 +670,11 @@ struct pfm_ctx {
     // or writes only atoms an earlier pass wrote (no mixed group)
     bool first_ok = false;
     struct Pass {
-      int inter, kind, list;  // kind: 0 lj1g, 1 lj rows of list `list`, 2 rjl density, 3 rjl force
-      bool first;             // a force pass whose atoms no earlier pass writes
+      // kind: 0 lj1g, 1 lj rows of list `list`, 2 rjl density, 3 rjl force,
+      // 4 lj1g with the lj rows of inter2's list2 (the same rows)
+      int inter, kind, list;
+      bool first;  // a force pass whose atoms no earlier pass writes
+      int inter2, list2;
     };
     std::vector<std::vector<Pass>> phases;
   } mp;
