@@ -1209,7 +1209,6 @@ __global__ void k_spec_copy(int N, int back, double4* __restrict__ pos, double4*
 static int spec_alloc(pfm_ctx* h, int k) {
   if (h->spec_k >= k) return PFM_OK;
   auto F = [](void* p) { if (p) (void)hipFree(p); };
-  F(h->xfer);
   F(h->spec_e); F(h->sp_pos); F(h->sp_vel); F(h->sp_frc); F(h->sp_mask); F(h->sp_orig);
   h->spec_e = nullptr; h->sp_pos = h->sp_vel = h->sp_frc = nullptr; h->sp_mask = nullptr; h->sp_orig = nullptr;
   h->spec_k = 0;

@@ -66,3 +66,19 @@ def test_after_sorts_and_from_a_thread():
     b.set_state(p, v)
     b.run("nve", 1.0, 0, 0, False)
     assert np.abs(b.state()[2] - f).max() < 1e-12 * np.abs(f).max()
+
+
+def test_copy_state_around_nvms_blocks():
+    """The staging of pfm_copy_state outlives the first nvms block of its
+    handle (whose ring once released it)."""
+    s = configs.fcc_cu_rgl(nx=6, seed=9, temperature=80.0)
+    a, b = gpu_ctx(s), gpu_ctx(s)
+    a.run("nve", 1.0, 0, 5, False)
+    b.run("nve", 1.0, 0, 0, False)
+    for _ in range(2):
+        b.copy_state_from(a)
+        p, v, _ = a.state()
+        q, w, _ = b.state()
+        np.testing.assert_array_equal(p, q)
+        np.testing.assert_array_equal(v, w)
+        b.run("nvms", 1.0, 0, 25, True, 1e-30)
