@@ -58,7 +58,10 @@ __global__ void k_kick_drift(int N, double4* __restrict__ pos, double4* __restri
                              const int* __restrict__ rep, const RepDev* __restrict__ rdev) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N) return;
-  kick_drift_atom(i, pos[i], mask[i], P, rep, rdev, qs, pos, vel, frc, qpos, false, err, orig, step);
+  // the force is read whether or not the atom moves, so its load does not
+  // wait on the mask's
+  const double4 v = vel[i];
+  kick_drift_atom(i, pos[i], v, frc[i], kick_factor(v.w), mask[i], P, rep, rdev, qs, pos, vel, frc, qpos, err, orig, step);
 }
 
 // fixed-point copy of the positions (mixed path), refreshed at the start of
@@ -115,6 +118,36 @@ __device__ __forceinline__ CSum block_csum(CSum v, double* sh) {
   return r;
 }
 
+// The same sums of NQ pairs per thread at once: the exchanges of the NQ
+// butterflies overlap and the block meets once instead of NQ times.  Thread 0
+// returns the block's pairs, bit for bit those of block_csum.
+template <int NQ>
+__device__ __forceinline__ void block_csum_n(CSum (&v)[NQ], double* sh) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) v[q].add(CSum{__shfl_xor(v[q].s, o), __shfl_xor(v[q].c, o)});
+  constexpr int nw = RED_THREADS / 64;
+  const int w = threadIdx.x >> 6;
+  __syncthreads();  // sh may still be read by the last call
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      sh[(q * nw + w) * 2] = v[q].s;
+      sh[(q * nw + w) * 2 + 1] = v[q].c;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      CSum r{sh[q * nw * 2], sh[q * nw * 2 + 1]};
+      for (int k = 1; k < nw; ++k) r.add(CSum{sh[(q * nw + k) * 2], sh[(q * nw + k) * 2 + 1]});
+      v[q] = r;
+    }
+  }
+}
+
 // Per-block partials of compensated sums: row q of a grid of nb blocks keeps
 // the s parts at part[2q nb + b] and the c parts at part[(2q+1) nb + b].
 __device__ __forceinline__ void put_part(double* part, int q, int nb, int b, const CSum& v) {
@@ -129,34 +162,40 @@ __device__ __forceinline__ CSum reduce_part(const double* part, int q, int nb, d
   return block_csum(a, sh);
 }
 
-// second half: kick xyz/z, then for nvms the projections
-// molecular_static_xyz/1D_velocities (md_integrators.f90:99-145)
+// second half of one atom: kick xyz/z, then for nvms the projections
+// molecular_static_xyz/1D_velocities (md_integrators.f90:99-145).  Returns
+// whether the atom moves.
+// The fused multiply-adds are written out: what the compiler would
+// contract differs between the kernels that call this, and an nvms run has
+// to give the same bits through each of them.
+__device__ __forceinline__ bool kick2_atom(double4& v, const double4& f, double k, uint32_t m, const IntP& P,
+                                           bool nvms) {
+  const bool bx = (m & P.bxyz) != 0, bz = (m & P.bz) != 0;
+  if (!(bx || bz)) return false;
+  if (bx) { v.x = fma(f.x * k, P.ts1, v.x); v.y = fma(f.y * k, P.ts1, v.y); v.z = fma(f.z * k, P.ts1, v.z); }
+  if (bz) v.z = fma(f.z * k, P.ts1, v.z);
+  if (nvms) {
+    if (bx) {
+      const double fv = fma(f.z, v.z, fma(f.x, v.x, f.y * v.y)), ff = fma(f.z, f.z, fma(f.x, f.x, f.y * f.y));
+      if (fv > 0.0 && ff > 1e-12) { double c = fv / ff; v.x = c * f.x; v.y = c * f.y; v.z = c * f.z; }
+      else { v.x = 0; v.y = 0; v.z = 0; }
+    }
+    if (bz) {
+      const double fv = fma(f.z, v.z, fma(f.x, v.x, f.y * v.y));
+      if (!(fv > 0.0)) { v.x = 0; v.y = 0; v.z = 0; }
+    }
+  }
+  return true;
+}
+
 __global__ void k_kick2(int N, double4* __restrict__ vel, const double4* __restrict__ frc,
                         const uint32_t* __restrict__ mask, IntP P, int nvms) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N) return;
   uint32_t m = mask[i];
   double4 v = vel[i], f = frc[i];  // loaded beside the mask, not after it
-  bool bx = (m & P.bxyz) != 0, bz = (m & P.bz) != 0;
-  if (!(bx || bz)) return;
-  double k = 1.0 / v.w / PFM_MASS_COEF;
-  if (bx) { v.x = v.x + f.x * k * P.ts1; v.y = v.y + f.y * k * P.ts1; v.z = v.z + f.z * k * P.ts1; }
-  if (bz) v.z = v.z + f.z * k * P.ts1;
-  if (nvms) {
-    if (bx) {
-      double fv = f.x * v.x + f.y * v.y + f.z * v.z, ff = f.x * f.x + f.y * f.y + f.z * f.z;
-      if (fv > 0.0 && ff > 1e-12) { double c = fv / ff; v.x = c * f.x; v.y = c * f.y; v.z = c * f.z; }
-      else { v.x = 0; v.y = 0; v.z = 0; }
-    }
-    if (bz) {
-      double fv = f.x * v.x + f.y * v.y + f.z * v.z;
-      if (!(fv > 0.0)) { v.x = 0; v.y = 0; v.z = 0; }
-    }
-  }
-  vel[i] = v;
+  if (kick2_atom(v, f, kick_factor(v.w), m, P, nvms != 0)) vel[i] = v;
 }
-
-
 
 __global__ void k_scale(int N, double4* __restrict__ vel, const uint32_t* __restrict__ mask, IntP P) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -248,10 +287,52 @@ __global__ void k_rec_bump(int* ctr, int e, int x) {
   if (x) ctr[1] = ctr[1] + 1;
 }
 
-struct RecPartArgs {
-  int ni, N;
+struct RowEnergies {
+  int ni;
   const double* e_row[PFM_MAXI];  // per-row energies of every interaction
   int e_rows[PFM_MAXI];
+};
+
+// a thread's first row energy of the interactions k0 .. k0 + 3
+__device__ __forceinline__ void first_row_energies(const RowEnergies& E, int k0, double (&x)[4]) {
+  const int i = blockIdx.x * RED_THREADS + threadIdx.x;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) x[q] = k0 + q < E.ni && i < E.e_rows[k0 + q] ? E.e_row[k0 + q][i] : 0.0;
+}
+
+// Per-block partials of every interaction's row energies and, as row ni, of
+// the sum `ke` holds per thread: four sums share one exchange (block_csum_n).
+// x holds the first_row_energies of interaction 0, loaded ahead by the caller.
+__device__ __forceinline__ void energy_row_parts(const RowEnergies& E, double (&x)[4], const CSum& ke, double* part,
+                                                 double* sh) {
+  const int nb = gridDim.x, b = blockIdx.x, t = threadIdx.x;
+  for (int k0 = 0; k0 <= E.ni; k0 += 4) {
+    if (k0) first_row_energies(E, k0, x);
+    CSum a[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (k0 + q == E.ni) {
+        a[q] = ke;
+        continue;
+      }
+      a[q] = CSum{0.0, 0.0};
+      a[q].add(x[q]);
+      if (k0 + q < E.ni)
+        for (int i = (b + nb) * RED_THREADS + t; i < E.e_rows[k0 + q]; i += nb * RED_THREADS)
+          a[q].add(E.e_row[k0 + q][i]);
+    }
+    block_csum_n<4>(a, sh);
+    if (t == 0) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        if (k0 + q <= E.ni) put_part(part, k0 + q, nb, b, a[q]);
+    }
+  }
+}
+
+struct RecPartArgs {
+  int N;
+  RowEnergies E;
   const double4 *pos, *vel, *frc;
   const uint32_t* mask;
   uint32_t ke_bit, all_bit;  // all_moving, all_atoms
@@ -269,12 +350,8 @@ struct RecPartArgs {
 __global__ void __launch_bounds__(RED_THREADS) k_rec_part(RecPartArgs A) {
   __shared__ double sh[2 * RED_THREADS];
   const int nb = gridDim.x, b = blockIdx.x, t = threadIdx.x;
-  for (int k = 0; k < A.ni; ++k) {
-    CSum a{0.0, 0.0};
-    for (int i = b * RED_THREADS + t; i < A.e_rows[k]; i += nb * RED_THREADS) a.add(A.e_row[k][i]);
-    CSum s = block_csum(a, sh);
-    if (t == 0) put_part(A.epart, k, nb, b, s);
-  }
+  double x[4];
+  first_row_energies(A.E, 0, x);
   CSum ke{0.0, 0.0};
   CSum a[10];
   for (int q = 0; q < 10; ++q) a[q] = CSum{0.0, 0.0};
@@ -293,11 +370,11 @@ __global__ void __launch_bounds__(RED_THREADS) k_rec_part(RecPartArgs A) {
       a[9].add(v.w);
     }
   }
-  CSum s = block_csum(ke, sh);
-  if (t == 0) put_part(A.epart, A.ni, nb, b, s);
+  energy_row_parts(A.E, x, ke, A.epart, sh);
   if (!A.opart) return;
+  __syncthreads();
   for (int q = 0; q < 10; ++q) {
-    s = block_csum(a[q], sh);
+    CSum s = block_csum(a[q], sh);
     if (t == 0) put_part(A.opart, q, nb, b, s);
   }
   sh[t] = vmax;
@@ -1086,17 +1163,24 @@ static void nhc_first_half(pfm_ctx* h, double dt) {
   PFM_LAUNCH(h, "nhc", k_nhc_chain, 1, RED_THREADS, Q.nq, A, h->red_part, nb);
 }
 
+static RowEnergies row_energies(pfm_ctx* h) {
+  RowEnergies E;
+  memset(&E, 0, sizeof E);
+  E.ni = (int)h->inter.size();
+  for (int k = 0; k < E.ni; ++k) {
+    E.e_row[k] = h->inter[k].e_row;
+    E.e_rows[k] = h->inter[k].e_rows;
+  }
+  return E;
+}
+
 // per-block partials of the interaction energies and the all_moving kinetic
 // energy into red_part, and of the out block into `opart` unless it is null
 static void energy_parts(pfm_ctx* h, double* opart) {
   RecPartArgs A;
   memset(&A, 0, sizeof A);
-  A.ni = (int)h->inter.size();
   A.N = h->N;
-  for (int k = 0; k < A.ni; ++k) {
-    A.e_row[k] = h->inter[k].e_row;
-    A.e_rows[k] = h->inter[k].e_rows;
-  }
+  A.E = row_energies(h);
   A.pos = h->pos4;
   A.vel = h->vel4;
   A.frc = h->frc4;
@@ -1192,30 +1276,92 @@ static int energies(pfm_ctx* h, bool nvt) {
 
 // ------------------------------------------------------------ nvms blocks
 
-// the state of one step into ring slot k, or back from it
-__global__ void k_spec_copy(int N, int back, double4* __restrict__ pos, double4* __restrict__ vel,
-                            double4* __restrict__ frc, uint32_t* __restrict__ mask, int* __restrict__ orig,
-                            double4* __restrict__ rpos, double4* __restrict__ rvel, double4* __restrict__ rfrc,
-                            uint32_t* __restrict__ rmask, int* __restrict__ rorig) {
+// the state of the step in a ring slot back into the handle's buffers
+__global__ void k_spec_back(int N, double4* __restrict__ pos, double4* __restrict__ vel, double4* __restrict__ frc,
+                            uint32_t* __restrict__ mask, int* __restrict__ orig, const double4* __restrict__ rpos,
+                            const double4* __restrict__ rvel, const double4* __restrict__ rfrc,
+                            const uint32_t* __restrict__ rmask, const int* __restrict__ rorig) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= N) return;
-  if (back) {
-    pos[i] = rpos[i]; vel[i] = rvel[i]; frc[i] = rfrc[i]; mask[i] = rmask[i]; orig[i] = rorig[i];
-  } else {
-    rpos[i] = pos[i]; rvel[i] = vel[i]; rfrc[i] = frc[i]; rmask[i] = mask[i]; rorig[i] = orig[i];
+  pos[i] = rpos[i]; vel[i] = rvel[i]; frc[i] = rfrc[i]; mask[i] = rmask[i]; orig[i] = rorig[i];
+}
+
+struct SpecStepArgs {
+  int N;
+  int kick, drift;  // second half of this step (not step 0); first half of the next one
+  IntP P;
+  double4 *pos, *vel, *frc;
+  const uint32_t* mask;
+  const int* orig;
+  double4 *rpos, *rvel, *rfrc;  // the step's ring slot
+  uint32_t* rmask;
+  int* rorig;
+  uint32_t ke_bit;
+  RowEnergies E;
+  double* part;
+  DevErr* err;
+  int step;  // of the next step, for the drift's errors
+  uint4* qpos;
+  double3 qs;
+  const int* rep;
+  const RepDev* rdev;
+};
+
+// The end of an nvms step inside a block: second half with the projections,
+// the step's state into its ring slot, the partials of its energies (order of
+// k_rec_part) and, unless the block ends or a record reads the state, the
+// first half of the next step.  Each of these passes is bound by its launch
+// and a chain of dependent loads and divisions at the sizes that are relaxed;
+// here one set of loads serves them all (6,312 atoms: 6.7 us, where separate
+// kernels took 3.1 + 2.7 + 6.1 + 3.1 and 4.4 for the sums of the step, which
+// now wait for the end of the block; a step of that slab 63.7 -> 49.7 us).
+__global__ void __launch_bounds__(RED_THREADS) k_spec_step(SpecStepArgs A) {
+  __shared__ double sh[2 * RED_THREADS];
+  double x[4];
+  first_row_energies(A.E, 0, x);
+  CSum ke{0.0, 0.0};
+  for (int i = blockIdx.x * RED_THREADS + threadIdx.x; i < A.N; i += gridDim.x * RED_THREADS) {
+    const double4 p = A.pos[i], f = A.frc[i];
+    double4 v = A.vel[i];
+    const uint32_t m = A.mask[i];
+    const int o = A.orig[i];
+    const double k = kick_factor(v.w);
+    const bool moves = A.kick && kick2_atom(v, f, k, m, A.P, true);
+    // the two half kicks round as in the separate kernels: no fma takes a
+    // product of the projection across, no product serves both
+    double4 f2 = f;
+    asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(f2.x), "+v"(f2.y), "+v"(f2.z));
+    A.rpos[i] = p; A.rvel[i] = v; A.rfrc[i] = f; A.rmask[i] = m; A.rorig[i] = o;
+    if (m & A.ke_bit) ke.add(v.w * (v.x * v.x + v.y * v.y + v.z * v.z) / 2 * PFM_MASS_COEF);
+    if (A.drift)
+      kick_drift_atom(i, p, v, f2, k, m, A.P, A.rep, A.rdev, A.qs, A.pos, A.vel, A.frc, A.qpos, A.err, A.orig, A.step);
+    else if (moves)
+      A.vel[i] = v;
   }
+  energy_row_parts(A.E, x, ke, A.part, sh);
+}
+
+// the energies of a block's steps: row q of step k is block k * nq + q
+__global__ void __launch_bounds__(RED_THREADS) k_spec_energies(int nq, int nb, const double* __restrict__ part,
+                                                               double* __restrict__ out) {
+  __shared__ double sh[2 * RED_THREADS];
+  const int k = blockIdx.x / nq, q = blockIdx.x % nq;
+  CSum s = reduce_part(part + (size_t)k * 2 * nq * nb, q, nb, sh);
+  if (threadIdx.x == 0) out[blockIdx.x] = s.value();
 }
 
 static int spec_alloc(pfm_ctx* h, int k) {
   if (h->spec_k >= k) return PFM_OK;
   auto F = [](void* p) { if (p) (void)hipFree(p); };
-  F(h->spec_e); F(h->sp_pos); F(h->sp_vel); F(h->sp_frc); F(h->sp_mask); F(h->sp_orig);
-  h->spec_e = nullptr; h->sp_pos = h->sp_vel = h->sp_frc = nullptr; h->sp_mask = nullptr; h->sp_orig = nullptr;
+  F(h->spec_e); F(h->spec_part); F(h->sp_pos); F(h->sp_vel); F(h->sp_frc); F(h->sp_mask); F(h->sp_orig);
+  h->spec_e = h->spec_part = nullptr; h->sp_pos = h->sp_vel = h->sp_frc = nullptr; h->sp_mask = nullptr; h->sp_orig = nullptr;
   h->spec_k = 0;
   const size_t n = (size_t)k * h->N;
   const size_t nr = h->nrep > 1 ? (size_t)h->nrep : 0;  // batches: per-replica rows after the whole-system rows
   int rc;
-  if ((rc = dalloc(h, &h->spec_e, (size_t)k * (h->inter.size() + 1) * (1 + nr))) || (rc = dalloc(h, &h->sp_pos, n)) ||
+  if ((rc = dalloc(h, &h->spec_e, (size_t)k * (h->inter.size() + 1) * (1 + nr))) ||
+      (rc = dalloc(h, &h->spec_part, (size_t)k * (h->inter.size() + 1) * 2 * h->red_blocks)) ||
+      (rc = dalloc(h, &h->sp_pos, n)) ||
       (rc = dalloc(h, &h->sp_vel, n)) || (rc = dalloc(h, &h->sp_frc, n)) || (rc = dalloc(h, &h->sp_mask, n)) ||
       (rc = dalloc(h, &h->sp_orig, n)))
     return rc;
@@ -1223,20 +1369,38 @@ static int spec_alloc(pfm_ctx* h, int k) {
   return PFM_OK;
 }
 
-// the energies of the step into slot k (the sums of energies(); for a batch
-// also each replica's, after the spec_k whole-system rows) and its state
-static void spec_record(pfm_ctx* h, int k) {
-  const int nb = h->red_blocks, ni = (int)h->inter.size(), N = h->N;
-  energy_parts(h, nullptr);
-  PFM_LAUNCH(h, "energy", k_reduce_rows, 1, RED_THREADS, ni + 1, nb, h->red_part, h->spec_e + (size_t)k * (ni + 1));
+// the end of a step of an nvms block: its state and the partials of its
+// energies into slot k (for a batch also each replica's energies, after the
+// spec_k whole-system rows); `kick` applies the second half, `drift` the first
+// half of the next step, whose number `next` the drift's errors carry
+static void spec_record(pfm_ctx* h, int k, const IntP& P, bool kick, bool drift, int next) {
+  const int ni = (int)h->inter.size(), N = h->N;
+  const size_t o = (size_t)k * N;
+  SpecStepArgs S;
+  memset(&S, 0, sizeof S);
+  S.N = N;
+  S.kick = kick ? 1 : 0;
+  S.drift = drift ? 1 : 0;
+  S.P = P;
+  S.pos = h->pos4; S.vel = h->vel4; S.frc = h->frc4; S.mask = h->mask; S.orig = h->orig;
+  S.rpos = h->sp_pos + o; S.rvel = h->sp_vel + o; S.rfrc = h->sp_frc + o; S.rmask = h->sp_mask + o;
+  S.rorig = h->sp_orig + o;
+  S.ke_bit = 1u << (h->roles[0] - 1);
+  S.E = row_energies(h);
+  S.part = h->spec_part + (size_t)k * (ni + 1) * 2 * h->red_blocks;
+  S.err = h->derr;
+  S.step = next - h->step_base;
+  S.qpos = h->qpos;
+  S.qs = h->qscale;
+  S.rep = h->rep;
+  S.rdev = h->rdev;
+  PFM_LAUNCH(h, "spec", k_spec_step, h->red_blocks, RED_THREADS, S);
   if (h->nrep > 1) {
     RepEnergyArgs A = rep_energy_args(h);
+    A.vel = S.rvel;
     A.out = h->spec_e + (size_t)h->spec_k * (ni + 1) + (size_t)k * h->nrep * (ni + 1);
     PFM_LAUNCH(h, "energy", k_rep_energy, h->nrep, RED_THREADS, A);
   }
-  const size_t o = (size_t)k * N;
-  PFM_LAUNCH(h, "spec", k_spec_copy, (N + 255) / 256, 256, N, 0, h->pos4, h->vel4, h->frc4, h->mask, h->orig,
-             h->sp_pos + o, h->sp_vel + o, h->sp_frc + o, h->sp_mask + o, h->sp_orig + o);
 }
 
 // rebuild every list due at step s, in settings order; re-sort the atoms
@@ -1853,7 +2017,8 @@ static int run_steps(pfm_ctx* h, int integ, double dt, int s0, int s1, int energ
   // nvms blocks: the steps from spec_base on record their energies and
   // states into ring slots instead of reading energies back
   bool spec_on = false;
-  int spec_base = 0;
+  int spec_base = 0, spec_end = 0;
+  bool drifted = false;  // the last step's spec_record took this step's first half
   // one md() step: the body of md_simulation.f90:137-231
   auto body = [&](int s) -> int {
     int rc;
@@ -1883,8 +2048,10 @@ static int run_steps(pfm_ctx* h, int integ, double dt, int s0, int s1, int energ
         Q.scale = 1;
         nhc_pending = false;
       }
-      PFM_LAUNCH(h, "kick_drift", k_kick_drift, nb, 256, N, h->pos4, h->vel4, h->frc4, h->mask, Q, h->derr, h->orig,
-                 s - h->step_base, h->qpos, h->qscale, h->rep, h->rdev);
+      if (!drifted)
+        PFM_LAUNCH(h, "kick_drift", k_kick_drift, nb, 256, N, h->pos4, h->vel4, h->frc4, h->mask, Q, h->derr, h->orig,
+                   s - h->step_base, h->qpos, h->qscale, h->rep, h->rdev);
+      drifted = false;
     } else if (!first_writes) {
       PFM_LAUNCH(h, "zero_forces", k_zero_masked, nb, 256, N, h->frc4, h->mask, all_bit);
     }
@@ -1907,13 +2074,17 @@ static int run_steps(pfm_ctx* h, int integ, double dt, int s0, int s1, int energ
       } else if (integ != PFM_NVMS && !report && s < s1) {
         // nothing reads the velocities before the next step's first half
         kick_pending = true;
-      } else {
+      } else if (!spec_on) {
         PFM_LAUNCH(h, "kick2", k_kick2, nb, 256, N, h->vel4, h->frc4, h->mask, P, integ == PFM_NVMS ? 1 : 0);
       }
       h->sim_time = h->sim_time + dt;
     }
     if (spec_on) {
-      spec_record(h, s - spec_base);
+      drifted = s < spec_end && !re && !rx;
+      IntP Q = P;
+      Q.invert = h->invert_z;
+      Q.zero_bit = first_writes ? 0u : all_bit;
+      spec_record(h, s - spec_base, Q, s != 0, drifted, s + 1);
     } else if (energy) {
       if ((rc = energies(h, integ == PFM_NVT))) return rc;
       if ((rc = check_err(h, s))) return rc;
@@ -2043,6 +2214,7 @@ static int run_steps(pfm_ctx* h, int integ, double dt, int s0, int s1, int energ
       const std::vector<double> rpe0 = h->rep_pe;
       spec_on = true;
       spec_base = s;
+      spec_end = end;
       int rc2 = PFM_OK;
       if (capture && s > 0 && s % K == 0 && n == K) {
         rc2 = run_block(s, K);
@@ -2051,6 +2223,7 @@ static int run_steps(pfm_ctx* h, int integ, double dt, int s0, int s1, int energ
       }
       spec_on = false;
       if (rc2) return rc2;
+      PFM_LAUNCH(h, "energy", k_spec_energies, n * w, RED_THREADS, w, h->red_blocks, h->spec_part, h->spec_e);
       if (ne_b + nx_b > 0) {
         notes.clear();
         double tt = t_start;
@@ -2112,7 +2285,7 @@ static int run_steps(pfm_ctx* h, int integ, double dt, int s0, int s1, int energ
         R.q.pop_back();
       }
       const size_t o = (size_t)jl * h->N;
-      PFM_LAUNCH(h, "spec", k_spec_copy, (h->N + 255) / 256, 256, h->N, 1, h->pos4, h->vel4, h->frc4, h->mask,
+      PFM_LAUNCH(h, "spec", k_spec_back, (h->N + 255) / 256, 256, h->N, h->pos4, h->vel4, h->frc4, h->mask,
                  h->orig, h->sp_pos + o, h->sp_vel + o, h->sp_frc + o, h->sp_mask + o, h->sp_orig + o);
       // lists, cells and rows follow the restored state at the next step
       h->need_sort = true;
@@ -2810,7 +2983,7 @@ int pfm_destroy(pfm_ctx* h) {
   F(h->red_part); F(h->red_out); F(h->derr); F(h->cell_rank); F(h->cell_count); F(h->cell_start); F(h->cell_xyz);
   F(h->nhc_state);
   F(h->xfer);
-  F(h->spec_e); F(h->sp_pos); F(h->sp_vel); F(h->sp_frc); F(h->sp_mask); F(h->sp_orig);
+  F(h->spec_e); F(h->spec_part); F(h->sp_pos); F(h->sp_vel); F(h->sp_frc); F(h->sp_mask); F(h->sp_orig);
   if (h->h_red) (void)hipHostFree(h->h_red);
   if (h->herr) (void)hipHostFree(h->herr);
   if (h->stage) (void)hipHostFree(h->stage);

@@ -425,29 +425,28 @@ __device__ __forceinline__ void invert_v(double4& v, double z, double lo, double
   if ((z > lo && z < mid && v.z > 0.0) || (z < hi && z > mid && v.z < 0.0)) v.z = -v.z;
 }
 
+__device__ __forceinline__ double kick_factor(double mass) { return 1.0 / mass / PFM_MASS_COEF; }
+
 // First half of a step for atom i: [the previous step's second half kick
 // (deferred), same operations as k_kick2], [invert_z_velocities], [NHC
 // scaling], kick xyz/z, drift xyz/z with single wrap (md_integrators.f90:7-97),
 // the fixed-point copy, zero_forces, and check_positions of the next step
-// (md_general.f90:342-364).  The position goes to pos_out and the fixed-point
-// copy to q_out; with out_of_place both are written for every atom (moving or
-// not), otherwise only where the atom moved.
-__device__ __forceinline__ void kick_drift_atom(int i, double4 p, uint32_t m, const IntP& P, const int* rep,
-                                                const RepDev* rdev, double3 qs, double4* pos_out, double4* vel,
-                                                double4* frc, uint4* q_out, bool out_of_place, DevErr* err,
+// (md_general.f90:342-364).  p, v and f are the atom's state before it, k
+// its kick_factor.
+__device__ __forceinline__ void kick_drift_atom(int i, double4 p, double4 v, const double4& f, double k,
+                                                uint32_t m, const IntP& P, const int* rep, const RepDev* rdev, double3 qs,
+                                                double4* pos, double4* vel, double4* frc, uint4* qpos, DevErr* err,
                                                 const int* orig, int step) {
   double Lx = P.box[0], Ly = P.box[1], Lz = P.box[2], zlo = P.zlo, zhi = P.zhi;
+  // held in scalar registers: left to itself the compiler selects the address
+  // (argument or replica table) and loads each through it, behind the branch
+  asm volatile("" : "+s"(Lx), "+s"(Ly), "+s"(Lz), "+s"(zlo), "+s"(zhi));
   if (rep) {
     const RepDev& R = rdev[rep[i]];
     Lx = R.L.x; Ly = R.L.y; Lz = R.L.z; zlo = R.zlo; zhi = R.zhi; qs = R.qs;
   }
-  // the force is read whether or not the atom moves, so its load does not
-  // wait on the mask's
-  double4 v = vel[i];
-  const double4 f = frc[i];
   bool bx = (m & P.bxyz) != 0, bz = (m & P.bz) != 0;
   if (P.pre_kick && (bx || bz)) {
-    double k = 1.0 / v.w / PFM_MASS_COEF;
     if (bx) { v.x = v.x + f.x * k * P.ts1; v.y = v.y + f.y * k * P.ts1; v.z = v.z + f.z * k * P.ts1; }
     if (bz) v.z = v.z + f.z * k * P.ts1;
   }
@@ -457,7 +456,6 @@ __device__ __forceinline__ void kick_drift_atom(int i, double4 p, uint32_t m, co
       if (m & P.chain_bit[c]) { double s = P.chain_s[c]; v.x *= s; v.y *= s; v.z *= s; }
   }
   if (bx || bz) {
-    double k = 1.0 / v.w / PFM_MASS_COEF;
     if (bx) { v.x = v.x + f.x * k * P.ts1; v.y = v.y + f.y * k * P.ts1; v.z = v.z + f.z * k * P.ts1; }
     if (bz) v.z = v.z + f.z * k * P.ts1;
     if (bx) {
@@ -467,9 +465,9 @@ __device__ __forceinline__ void kick_drift_atom(int i, double4 p, uint32_t m, co
     }
     if (bz) p.z = wrap1(p.z + v.z * P.ts0, Lz);
   }
-  if (bx || bz || out_of_place) {
-    pos_out[i] = p;
-    if (q_out) q_out[i] = quantize(p, qs, 0u);
+  if (bx || bz) {
+    pos[i] = p;
+    if (qpos) qpos[i] = quantize(p, qs, 0u);
   }
   vel[i] = v;
   if (m & P.zero_bit) frc[i] = make_double4(0, 0, 0, 0);
@@ -648,6 +646,7 @@ struct pfm_ctx {
   // nvms blocks (pfm_set_speculation): per-step energies and states of a block
   bool speculate = true;
   int spec_k = 0;                        // ring slots
+  double* spec_part = nullptr;           // device [spec_k][n_inter + 1] partial rows of the energies (k_rec_part)
   double* spec_e = nullptr;              // device [spec_k][n_inter + 1]: interaction energies, ke
   double4 *sp_pos = nullptr, *sp_vel = nullptr, *sp_frc = nullptr;  // [spec_k][N]
   uint32_t* sp_mask = nullptr;
