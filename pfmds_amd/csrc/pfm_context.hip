@@ -51,19 +51,6 @@ struct NhcDev {
   uint32_t bit;
 };
 
-// first half of a step for every atom (kick_drift_atom)
-__global__ void k_kick_drift(int N, double4* __restrict__ pos, double4* __restrict__ vel,
-                             double4* __restrict__ frc, const uint32_t* __restrict__ mask, IntP P, DevErr* err,
-                             const int* __restrict__ orig, int step, uint4* __restrict__ qpos, double3 qs,
-                             const int* __restrict__ rep, const RepDev* __restrict__ rdev) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  // the force is read whether or not the atom moves, so its load does not
-  // wait on the mask's
-  const double4 v = vel[i];
-  kick_drift_atom(i, pos[i], v, frc[i], kick_factor(v.w), mask[i], P, rep, rdev, qs, pos, vel, frc, qpos, err, orig, step);
-}
-
 // fixed-point copy of the positions (mixed path), refreshed at the start of
 // every run so positions set from the host are picked up
 __global__ void k_quantize(int N, const double4* __restrict__ pos, uint4* __restrict__ qpos, double3 qs,
@@ -222,16 +209,20 @@ __global__ void __launch_bounds__(RED_THREADS) k_ke_part(int N, const double4* _
                                                          const uint32_t* __restrict__ mask, MaskQ Q,
                                                          double* __restrict__ part) {
   __shared__ double sh[2 * RED_THREADS];
-  CSum acc[RED_MAXQ];
-  for (int q = 0; q < Q.nq; ++q) acc[q] = CSum{0.0, 0.0};
+  CSum acc[RED_MAXQ];  // in registers: every index below is a constant
+#pragma unroll
+  for (int q = 0; q < RED_MAXQ; ++q) acc[q] = CSum{0.0, 0.0};
   for (int i = blockIdx.x * RED_THREADS + threadIdx.x; i < N; i += gridDim.x * RED_THREADS) {
     double4 v = vel[i];
     uint32_t m = mask[i];
     double ke = v.w * (v.x * v.x + v.y * v.y + v.z * v.z) / 2 * PFM_MASS_COEF;
-    for (int q = 0; q < Q.nq; ++q)
-      if (m & Q.bit[q]) acc[q].add(ke);
+#pragma unroll
+    for (int q = 0; q < RED_MAXQ; ++q)
+      if (q < Q.nq && (m & Q.bit[q])) acc[q].add(ke);
   }
-  for (int q = 0; q < Q.nq; ++q) {
+#pragma unroll
+  for (int q = 0; q < RED_MAXQ; ++q) {
+    if (q >= Q.nq) break;
     CSum s = block_csum(acc[q], sh);
     if (threadIdx.x == 0) put_part(part, q, gridDim.x, blockIdx.x, s);
   }
@@ -501,106 +492,176 @@ __global__ void __launch_bounds__(RED_THREADS) k_rep_energy(RepEnergyArgs A) {
   if (threadIdx.x == 0) A.out[r * (A.ni + 1) + A.ni] = ke.value();
 }
 
-// integrate_nose_hoover_chain (md_integrators.f90:200-245) on one chain with
-// the chain group's kinetic energy ke; returns the velocity scale s
-__device__ double nhc_update(NhcDev& h, double ke, double ts1, double ts2, double ts3) {
-  double kt = h.kt;
-  double kedif = 2.0 * ke - 3.0 * h.L * kt;
-  int M = h.M;
-  double b = 1.0;
-  double* v = h.v;
-  const double* q = h.q;
-  if (M == 1) {
-    v[0] = v[0] + kedif / q[0] * ts2;
-  } else {
-    v[M - 1] = v[M - 1] + (q[M - 2] * v[M - 2] * v[M - 2] - kt) / q[M - 1] * ts2;
-    for (int i = M - 2; i >= 1; --i) {
-      b = exp(-v[i + 1] * ts3);
-      v[i] = v[i] * (b * b) + (q[i - 1] * v[i - 1] * v[i - 1] - kt) / q[i] * ts2 * b;
-    }
-    b = exp(-v[1] * ts3);
-    v[0] = v[0] * (b * b) + kedif / q[0] * ts2 * b;
+// One chain in a wavefront: lane j holds x, v and q of thermostat j and 1/q.
+// The update is one serial chain of arithmetic; with its state in registers,
+// read across lanes, no step of it waits for memory.
+struct NhcLane {
+  double x, v, q, rq, kt, L;
+  int M;
+  __device__ __forceinline__ void load(const NhcDev& d) {
+    const int j = threadIdx.x & 15;
+    x = d.x[j]; v = d.v[j]; q = d.q[j];
+    kt = d.kt; L = d.L; M = __builtin_amdgcn_readfirstlane(d.M);
+    rq = 1.0 / q;
   }
-  h.s = exp(-v[0] * ts1);
-  kedif = 2.0 * ke * (h.s * h.s) - 3.0 * h.L * kt;
-  for (int i = 0; i < M; ++i) h.x[i] = h.x[i] + v[i] * ts1;
-  if (M == 1) {
-    v[0] = v[0] + kedif / q[0] * ts2;
-  } else {
-    v[0] = v[0] * (b * b) + kedif / q[0] * ts2 * b;
-    for (int i = 1; i <= M - 2; ++i) {
-      b = exp(-v[i + 1] * ts3);
-      v[i] = v[i] * (b * b) + (q[i - 1] * v[i - 1] * v[i - 1] - kt) / q[i] * ts2 * b;
-    }
-    v[M - 1] = v[M - 1] + (q[M - 2] * v[M - 2] * v[M - 2] - kt) / q[M - 1] * ts2;
+  __device__ __forceinline__ void store(NhcDev& d) const {
+    const int j = threadIdx.x;
+    if (j < M) { d.x[j] = x; d.v[j] = v; }
   }
-  return h.s;
-}
+  static __device__ __forceinline__ double at(double a, int j) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(a), j),
+                            __builtin_amdgcn_readlane(__double2loint(a), j));
+  }
+  __device__ __forceinline__ void set(int j, double a) {
+    if ((int)threadIdx.x == j) v = a;
+  }
+  // n / q[j], correctly rounded from the rounded reciprocal (Markstein)
+  __device__ __forceinline__ double over_q(double n, int j) const {
+    const double r = at(rq, j), d = at(q, j), y = n * r;
+    return __builtin_amdgcn_div_fixup(fma(fma(-d, y, n), r, y), d, n);  // q zero or infinite as n / q
+  }
+  // the force on thermostat j >= 1 from the one before it, times ts2 / q[j]
+  __device__ __forceinline__ double push(int j, double ts2) const {
+    const double vp = at(v, j - 1);
+    return over_q(fma(at(q, j - 1) * vp, vp, -kt), j) * ts2;
+  }
 
-// Reduce each chain's kinetic-energy partials (fixed order) and apply one NHC
-// half step (twice = 0), or the second half of this step followed by the first
-// half of the next (twice = 1).  Nothing changes the velocities between those
-// two halves except invert_z_velocities, which keeps the kinetic energy, so
-// the second one uses s^2 * ke; s_out receives the product of the scales,
-// applied to the velocities by the next kick.  One block.
-struct ChainArgs {
-  NhcDev* C;
-  double* s_out;
-  double ts1, ts2, ts3;
-  int twice;
+  // integrate_nose_hoover_chain (md_integrators.f90:200-245) with the chain
+  // group's kinetic energy ke; returns the velocity scale s
+  __device__ __forceinline__ double update(double ke, double ts1, double ts2, double ts3) {
+    const double g = 3.0 * L * kt;
+    double b = 1.0, bj = 1.0;  // bj: lane j keeps exp(-v[j + 1] ts3), which the way back needs again
+    if (M > 1) {
+      double vn = at(v, M - 1) + push(M - 1, ts2);
+      set(M - 1, vn);
+      for (int j = M - 2; j >= 1; --j) {
+        b = f64::exp(-vn * ts3);
+        if ((int)threadIdx.x == j) bj = b;
+        vn = fma(push(j, ts2), b, at(v, j) * (b * b));
+        set(j, vn);
+      }
+      b = f64::exp(-vn * ts3);
+    }
+    const double v0 = fma(over_q(fma(2.0, ke, -g), 0) * ts2, b, at(v, 0) * (b * b));
+    const double s = f64::exp(-v0 * ts1);
+    set(0, v0);
+    x = fma(v, ts1, x);
+    set(0, fma(over_q(fma(2.0 * ke, s * s, -g), 0) * ts2, b, v0 * (b * b)));
+    for (int j = 1; j <= M - 2; ++j) {
+      b = at(bj, j);
+      set(j, fma(push(j, ts2), b, at(v, j) * (b * b)));
+    }
+    if (M > 1) set(M - 1, at(v, M - 1) + push(M - 1, ts2));
+    return s;
+  }
 };
 
+struct ChainArgs {
+  NhcDev* C;         // the chain states
+  const NhcDev* C0;  // where they are read: C, or the copy of k_kick2_ke
+  double* s_out;     // per-chain velocity scale
+  double ts1, ts2, ts3;
+};
+
+// Reduce chain c's kinetic-energy partials (fixed order) and apply one NHC
+// half step, or with `twice` the second half of a step followed by the first
+// half of the next.  Nothing changes the velocities between those two halves
+// except invert_z_velocities, which keeps the kinetic energy, so the second
+// one uses s^2 * ke.  Wave 0 returns the product of the velocity scales; the
+// states are stored where `keep` is set.
+__device__ __forceinline__ double chain_update(int c, const ChainArgs& A, const double* part, int nb, bool twice,
+                                               bool keep, double* sh) {
+  const bool first = threadIdx.x < 64;
+  NhcLane h;
+  if (first) h.load(A.C0[c]);
+  const double ke = reduce_part(part, c, nb, sh).value();
+  double s = 1.0;
+  if (first) {
+    s = h.update(ke, A.ts1, A.ts2, A.ts3);
+    if (twice) s *= h.update(s * s * ke, A.ts1, A.ts2, A.ts3);
+    if (keep) h.store(A.C[c]);
+  }
+  return s;
+}
+
+// one NHC half step of every chain; the scale is applied to the velocities by
+// the next kick or by k_scale.  One block.
 __global__ void __launch_bounds__(RED_THREADS) k_nhc_chain(int nchain, ChainArgs A, const double* __restrict__ part,
                                                            int nb) {
   __shared__ double sh[2 * RED_THREADS];
-  // the chain's serial update reads and writes its state many times over:
-  // work on a copy in LDS, loaded and stored by the whole block at once
-  __shared__ NhcDev st;
-  constexpr int W = sizeof(NhcDev) / sizeof(double);
   for (int c = 0; c < nchain; ++c) {
-    for (int j = threadIdx.x; j < W; j += RED_THREADS) ((double*)&st)[j] = ((const double*)&A.C[c])[j];
-    const double ke = reduce_part(part, c, nb, sh).value();  // ends with a barrier: the copy is complete
-    if (threadIdx.x == 0) {
-      double s = nhc_update(st, ke, A.ts1, A.ts2, A.ts3);
-      if (A.twice) s *= nhc_update(st, s * s * ke, A.ts1, A.ts2, A.ts3);
-      A.s_out[c] = s;
-    }
-    __syncthreads();
-    for (int j = threadIdx.x; j < W; j += RED_THREADS) ((double*)&A.C[c])[j] = ((const double*)&st)[j];
-    __syncthreads();
+    const double s = chain_update(c, A, part, nb, false, true, sh);
+    if (threadIdx.x == 0) A.s_out[c] = s;
   }
 }
 
+// First half of a step for every atom (kick_drift_atom).  With NHC the chains
+// first take the second half of the last step and the first half of this one
+// from the partials of k_kick2_ke: every block reduces them and updates the
+// chains for itself, while its atoms' loads are under way, and block 0 keeps
+// the result.
+template <bool NHC>
+__global__ void __launch_bounds__(RED_THREADS)
+    k_kick_drift(int N, double4* __restrict__ pos, double4* __restrict__ vel, double4* __restrict__ frc,
+                 const uint32_t* __restrict__ mask, IntP P, DevErr* err, const int* __restrict__ orig, int step,
+                 uint4* __restrict__ qpos, double3 qs, const int* __restrict__ rep, const RepDev* __restrict__ rdev,
+                 ChainArgs A, const double* __restrict__ part, int nb) {
+  const int i = blockIdx.x * RED_THREADS + threadIdx.x;
+  if (!NHC && i >= N) return;
+  const int j = NHC ? min(i, N - 1) : i;
+  // the force is read whether or not the atom moves, so its load does not
+  // wait on the mask's
+  const double4 p = pos[j], v = vel[j], f = frc[j];
+  const uint32_t m = mask[j];
+  if (NHC) {
+    __shared__ double sh[2 * RED_THREADS];
+    __shared__ double cs[PFM_MAXNHC];
+    for (int c = 0; c < P.nchain; ++c) {
+      const double s = chain_update(c, A, part, nb, true, blockIdx.x == 0, sh);
+      if (threadIdx.x == 0) cs[c] = s;
+    }
+    __syncthreads();
+    if (i >= N) return;
+    kick_drift_atom(i, p, v, f, kick_factor(v.w), m, P, cs, rep, rdev, qs, pos, vel, frc, qpos, err, orig, step);
+  } else {
+    kick_drift_atom(i, p, v, f, kick_factor(v.w), m, P, P.chain_s, rep, rdev, qs, pos, vel, frc, qpos, err, orig,
+                    step);
+  }
+}
 
-
-// second half with the kinetic energies of the chain groups after the kick
-// (the input of the second NHC half step), per block, grid-stride
+// Second half of a step with the kinetic energies of the chain groups after
+// the kick (the input of the second NHC half step), per block, grid-stride.
+// Where the next step's k_kick_drift<true> follows, only the energies are
+// formed (it repeats the kick) and the chain states are copied for its blocks
+// to read while its first block writes the new ones.
 __global__ void __launch_bounds__(RED_THREADS) k_kick2_ke(int N, double4* __restrict__ vel,
                                                           const double4* __restrict__ frc,
                                                           const uint32_t* __restrict__ mask, IntP P, MaskQ Q,
-                                                          double* __restrict__ part) {
+                                                          double* __restrict__ part, const NhcDev* __restrict__ C,
+                                                          NhcDev* __restrict__ C0) {
   __shared__ double sh[2 * RED_THREADS];
-  CSum acc[RED_MAXQ];
-  for (int q = 0; q < Q.nq; ++q) acc[q] = CSum{0.0, 0.0};
+  CSum acc[RED_MAXQ];  // in registers: every index below is a constant
+#pragma unroll
+  for (int q = 0; q < RED_MAXQ; ++q) acc[q] = CSum{0.0, 0.0};
   for (int i = blockIdx.x * RED_THREADS + threadIdx.x; i < N; i += gridDim.x * RED_THREADS) {
     uint32_t m = mask[i];
-    bool bx = (m & P.bxyz) != 0, bz = (m & P.bz) != 0;
     double4 v = vel[i];
     const double4 f = frc[i];  // not waiting on the mask
-    if (bx || bz) {
-      double k = 1.0 / v.w / PFM_MASS_COEF;
-      if (bx) { v.x = v.x + f.x * k * P.ts1; v.y = v.y + f.y * k * P.ts1; v.z = v.z + f.z * k * P.ts1; }
-      if (bz) v.z = v.z + f.z * k * P.ts1;
-      vel[i] = v;
-    }
+    if (kick2_atom(v, f, kick_factor(v.w), m, P, false) && !C0) vel[i] = v;
     double ke = v.w * (v.x * v.x + v.y * v.y + v.z * v.z) / 2 * PFM_MASS_COEF;
-    for (int q = 0; q < Q.nq; ++q)
-      if (m & Q.bit[q]) acc[q].add(ke);
+#pragma unroll
+    for (int q = 0; q < RED_MAXQ; ++q)
+      if (q < Q.nq && (m & Q.bit[q])) acc[q].add(ke);
   }
-  for (int q = 0; q < Q.nq; ++q) {
+#pragma unroll
+  for (int q = 0; q < RED_MAXQ; ++q) {
+    if (q >= Q.nq) break;
     CSum s = block_csum(acc[q], sh);
     if (threadIdx.x == 0) put_part(part, q, gridDim.x, blockIdx.x, s);
   }
+  if (C0 && blockIdx.x == 0)
+    for (int j = threadIdx.x; j < Q.nq * (int)(sizeof(NhcDev) / sizeof(double)); j += RED_THREADS)
+      ((double*)C0)[j] = ((const double*)C)[j];
 }
 
 // ------------------------------------------------------------- host helpers
@@ -1084,7 +1145,8 @@ static int finalize(pfm_ctx* h) {
       d.s = 1.0;
       d.bit = 1u << (h->nhc[c].group - 1);
     }
-    if ((rc = dalloc(h, (NhcDev**)&h->nhc_state, cs.size()))) return rc;
+    if ((rc = dalloc(h, (NhcDev**)&h->nhc_state, cs.size())) ||
+        (rc = dalloc(h, (NhcDev**)&h->nhc_state0, cs.size()))) return rc;
     HIPCHK(h, hipMemcpyAsync(h->nhc_state, cs.data(), sizeof(NhcDev) * cs.size(), hipMemcpyHostToDevice, h->stream));
     h->e_nhc.assign(h->nhc.size(), 0.0);
   }
@@ -1155,10 +1217,13 @@ static MaskQ chain_masks(pfm_ctx* h) {
 }
 
 // first NHC half step of a step: kinetic energies, then the chains
+static ChainArgs chain_args(pfm_ctx* h, double dt, const double* from) {
+  return ChainArgs{(NhcDev*)h->nhc_state, (const NhcDev*)from, h->red_out + 16, dt / 2.0, dt / 4.0, dt / 8.0};
+}
 static void nhc_first_half(pfm_ctx* h, double dt) {
   int nb = h->red_blocks;
   MaskQ Q = chain_masks(h);
-  ChainArgs A{(NhcDev*)h->nhc_state, h->red_out + 16, dt / 2.0, dt / 4.0, dt / 8.0, 0};
+  const ChainArgs A = chain_args(h, dt, h->nhc_state);
   PFM_LAUNCH(h, "nhc", k_ke_part, nb, RED_THREADS, h->N, h->vel4, h->mask, Q, h->red_part);
   PFM_LAUNCH(h, "nhc", k_nhc_chain, 1, RED_THREADS, Q.nq, A, h->red_part, nb);
 }
@@ -1334,7 +1399,7 @@ __global__ void __launch_bounds__(RED_THREADS) k_spec_step(SpecStepArgs A) {
     A.rpos[i] = p; A.rvel[i] = v; A.rfrc[i] = f; A.rmask[i] = m; A.rorig[i] = o;
     if (m & A.ke_bit) ke.add(v.w * (v.x * v.x + v.y * v.y + v.z * v.z) / 2 * PFM_MASS_COEF);
     if (A.drift)
-      kick_drift_atom(i, p, v, f2, k, m, A.P, A.rep, A.rdev, A.qs, A.pos, A.vel, A.frc, A.qpos, A.err, A.orig, A.step);
+      kick_drift_atom(i, p, v, f2, k, m, A.P, A.P.chain_s, A.rep, A.rdev, A.qs, A.pos, A.vel, A.frc, A.qpos, A.err, A.orig, A.step);
     else if (moves)
       A.vel[i] = v;
   }
@@ -2046,11 +2111,17 @@ static int run_steps(pfm_ctx* h, int integ, double dt, int s0, int s1, int energ
       if (nvt) {
         if (!nhc_pending) nhc_first_half(h, dt);
         Q.scale = 1;
-        nhc_pending = false;
       }
-      if (!drifted)
-        PFM_LAUNCH(h, "kick_drift", k_kick_drift, nb, 256, N, h->pos4, h->vel4, h->frc4, h->mask, Q, h->derr, h->orig,
-                   s - h->step_base, h->qpos, h->qscale, h->rep, h->rdev);
+      if (nhc_pending) {
+        Q.pre_kick = 1;
+        PFM_LAUNCH(h, "kick_drift", k_kick_drift<true>, nb, RED_THREADS, N, h->pos4, h->vel4, h->frc4, h->mask, Q,
+                   h->derr, h->orig, s - h->step_base, h->qpos, h->qscale, h->rep, h->rdev,
+                   chain_args(h, dt, h->nhc_state0), h->red_part, h->red_blocks);
+        nhc_pending = false;
+      } else if (!drifted) {
+        PFM_LAUNCH(h, "kick_drift", k_kick_drift<false>, nb, RED_THREADS, N, h->pos4, h->vel4, h->frc4, h->mask, Q,
+                   h->derr, h->orig, s - h->step_base, h->qpos, h->qscale, h->rep, h->rdev, ChainArgs{}, nullptr, 0);
+      }
       drifted = false;
     } else if (!first_writes) {
       PFM_LAUNCH(h, "zero_forces", k_zero_masked, nb, 256, N, h->frc4, h->mask, all_bit);
@@ -2062,15 +2133,17 @@ static int run_steps(pfm_ctx* h, int integ, double dt, int s0, int s1, int energ
     if ((rc = launch_forces(h, energy || re, first_writes))) return rc;
     if (s != 0) {
       if (nvt) {
-        // second half step; on steps with nothing to report, the chain update
-        // also takes the first half of the next step (k_nhc_chain)
-        MaskQ C = chain_masks(h);
-        bool fuse = !report && s < s1;
-        ChainArgs A{(NhcDev*)h->nhc_state, h->red_out + 16, dt / 2.0, dt / 4.0, dt / 8.0, fuse ? 1 : 0};
-        PFM_LAUNCH(h, "kick2", k_kick2_ke, h->red_blocks, RED_THREADS, N, h->vel4, h->frc4, h->mask, P, C, h->red_part);
-        PFM_LAUNCH(h, "nhc", k_nhc_chain, 1, RED_THREADS, C.nq, A, h->red_part, h->red_blocks);
-        if (fuse) nhc_pending = true;
-        else PFM_LAUNCH(h, "nhc_scale", k_scale, nb, 256, N, h->vel4, h->mask, P);
+        // second half step; on steps with nothing to report, the next step's
+        // first half takes it and both halves of the chain update with it
+        nhc_pending = !report && s < s1;
+        const MaskQ C = chain_masks(h);
+        PFM_LAUNCH(h, "kick2", k_kick2_ke, h->red_blocks, RED_THREADS, N, h->vel4, h->frc4, h->mask, P, C, h->red_part,
+                   (const NhcDev*)h->nhc_state, nhc_pending ? (NhcDev*)h->nhc_state0 : nullptr);
+        if (!nhc_pending) {
+          PFM_LAUNCH(h, "nhc", k_nhc_chain, 1, RED_THREADS, C.nq, chain_args(h, dt, h->nhc_state), h->red_part,
+                     h->red_blocks);
+          PFM_LAUNCH(h, "nhc_scale", k_scale, nb, 256, N, h->vel4, h->mask, P);
+        }
       } else if (integ != PFM_NVMS && !report && s < s1) {
         // nothing reads the velocities before the next step's first half
         kick_pending = true;
@@ -2981,7 +3054,7 @@ int pfm_destroy(pfm_ctx* h) {
   F(h->pos4); F(h->vel4); F(h->frc4); F(h->pos4b); F(h->vel4b); F(h->frc4b); F(h->mask); F(h->maskb);
   F(h->orig); F(h->origb); F(h->perm); F(h->atom_rank); F(h->scan_tmp); F(h->eb); F(h->qpos); F(h->rdev); F(h->rep); F(h->repb); F(h->cell_rep); F(h->d_rep_row0); F(h->d_rep_out);
   F(h->red_part); F(h->red_out); F(h->derr); F(h->cell_rank); F(h->cell_count); F(h->cell_start); F(h->cell_xyz);
-  F(h->nhc_state);
+  F(h->nhc_state); F(h->nhc_state0);
   F(h->xfer);
   F(h->spec_e); F(h->spec_part); F(h->sp_pos); F(h->sp_vel); F(h->sp_frc); F(h->sp_mask); F(h->sp_orig);
   if (h->h_red) (void)hipHostFree(h->h_red);

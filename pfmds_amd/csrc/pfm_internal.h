@@ -432,11 +432,11 @@ __device__ __forceinline__ double kick_factor(double mass) { return 1.0 / mass /
 // scaling], kick xyz/z, drift xyz/z with single wrap (md_integrators.f90:7-97),
 // the fixed-point copy, zero_forces, and check_positions of the next step
 // (md_general.f90:342-364).  p, v and f are the atom's state before it, k
-// its kick_factor.
+// its kick_factor, chain_s the chains' velocity scales.
 __device__ __forceinline__ void kick_drift_atom(int i, double4 p, double4 v, const double4& f, double k,
-                                                uint32_t m, const IntP& P, const int* rep, const RepDev* rdev, double3 qs,
-                                                double4* pos, double4* vel, double4* frc, uint4* qpos, DevErr* err,
-                                                const int* orig, int step) {
+                                                uint32_t m, const IntP& P, const double* chain_s, const int* rep,
+                                                const RepDev* rdev, double3 qs, double4* pos, double4* vel,
+                                                double4* frc, uint4* qpos, DevErr* err, const int* orig, int step) {
   double Lx = P.box[0], Ly = P.box[1], Lz = P.box[2], zlo = P.zlo, zhi = P.zhi;
   // held in scalar registers: left to itself the compiler selects the address
   // (argument or replica table) and loads each through it, behind the branch
@@ -446,14 +446,14 @@ __device__ __forceinline__ void kick_drift_atom(int i, double4 p, double4 v, con
     Lx = R.L.x; Ly = R.L.y; Lz = R.L.z; zlo = R.zlo; zhi = R.zhi; qs = R.qs;
   }
   bool bx = (m & P.bxyz) != 0, bz = (m & P.bz) != 0;
-  if (P.pre_kick && (bx || bz)) {
-    if (bx) { v.x = v.x + f.x * k * P.ts1; v.y = v.y + f.y * k * P.ts1; v.z = v.z + f.z * k * P.ts1; }
-    if (bz) v.z = v.z + f.z * k * P.ts1;
+  if (P.pre_kick) {
+    if (bx) { v.x = fma(f.x * k, P.ts1, v.x); v.y = fma(f.y * k, P.ts1, v.y); v.z = fma(f.z * k, P.ts1, v.z); }
+    if (bz) v.z = fma(f.z * k, P.ts1, v.z);
   }
   if (P.invert) invert_v(v, p.z, zlo, zhi);
   if (P.scale) {
     for (int c = 0; c < P.nchain; ++c)
-      if (m & P.chain_bit[c]) { double s = P.chain_s[c]; v.x *= s; v.y *= s; v.z *= s; }
+      if (m & P.chain_bit[c]) { double s = chain_s[c]; v.x *= s; v.y *= s; v.z *= s; }
   }
   if (bx || bz) {
     if (bx) { v.x = v.x + f.x * k * P.ts1; v.y = v.y + f.y * k * P.ts1; v.z = v.z + f.z * k * P.ts1; }
@@ -609,6 +609,7 @@ struct pfm_ctx {
   std::vector<Nhc> nhc;
   // NHC chain state on device: x[16], v[16], q[16], s, e, ke per chain
   double* nhc_state = nullptr;
+  double* nhc_state0 = nullptr;  // copy the blocks of k_kick_drift<true> read
   // cells
   int nc[3] = {1, 1, 1}, ncell = 1;
   double cell_len[3];

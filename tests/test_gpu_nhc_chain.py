@@ -1,0 +1,42 @@
+"""Nose-Hoover chains of every length class (1, 2, 3 and the longest, 16), one
+and two of them, one of length 1 with an infinite mass (a thermostat that does not
+move), on sizes about one workgroup: positions, velocities, chain states and
+chain energies against the oracle in FP64, after steps with nothing to report
+(chains advanced by the next step's first half) and one that reports.
+
+Bound: 1e-10 of the largest value, as in the other FP64 comparisons with the
+oracle over some tens of steps."""
+import numpy as np
+import pytest
+
+from pfmds_amd import configs
+from pfmds_amd.system import NHC, KB
+from tests.harness import gpu_ctx, oracle_ctx, rel_inf
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,chains", [(255, [1]), (256, [2]), (257, [3, 1]), (513, [16, 2]), (300, [16]), (300, [0])])
+def test_chains(n, chains):
+    s = configs.lj_gas_lattice(n, 0.02, 71, 150.0)
+    s.nhcs = []
+    for k, M in enumerate(chains):
+        g = 3 if len(chains) == 1 else k + 1
+        m = n if g == 3 else n // 2
+        q = 3 * m * KB * 100.0 * 20.0 ** 2
+        s.nhcs.append(NHC(g, 100.0, M or 1, q if M else float("inf")))
+    res = []
+    for make in (oracle_ctx, gpu_ctx):
+        c = make(s)
+        c.run("nvt", 0.5, 0, 0, True)
+        c.run("nvt", 0.5, 1, 40, False)
+        c.run("nvt", 0.5, 41, 55, True)
+        res.append((c.state(), c.energies(), [c.get_chain(k + 1, h.M) for k, h in enumerate(s.nhcs)]))
+        c.close()
+    (so, eo, co), (sg, eg, cg) = res
+    for x, y in zip(sg, so):
+        assert rel_inf(x, y) < 1e-10
+    if chains != [0]:
+        np.testing.assert_allclose(eg["e_nhc"], eo["e_nhc"], rtol=1e-10)
+    for (xg, vg), (xo, vo) in zip(cg, co):
+        assert rel_inf(xg, xo) < 1e-10 and rel_inf(vg, vo) < 1e-10
