@@ -1889,6 +1889,9 @@ int pfm_create_batch(pfm_ctx** out, int nrep, const int* n_atoms, const double* 
     return rc;
   for (int d = 0; d < 3; ++d) (&h->qscale.x)[d] = 4294967296.0 / boxes[d];
   if (precision == PFM_MIXED && (rc = dalloc(h, &h->qpos, n))) return rc;
+  int dev = 0;
+  HIPCHK(h, hipGetDevice(&dev));
+  HIPCHK(h, hipDeviceGetAttribute(&h->cus, hipDeviceAttributeMultiprocessorCount, dev));
   h->red_blocks = std::max(1, std::min(1024, (n + RED_THREADS - 1) / RED_THREADS));
   // compensated partial rows: an (s, c) pair per block
   if ((rc = dalloc(h, &h->red_part, (size_t)2 * (PFM_MAXI + 1 + RED_MAXQ) * h->red_blocks))) return rc;

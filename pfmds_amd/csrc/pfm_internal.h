@@ -630,6 +630,7 @@ struct pfm_ctx {
   double* red_part = nullptr;  // partial sums
   double* red_out = nullptr;   // device scalars
   double* h_red = nullptr;     // pinned host mirror
+  int cus = 256;  // compute units of the device
   int red_blocks = 0;
   DevErr* derr = nullptr;
   DevErr* herr = nullptr;  // pinned

@@ -53,6 +53,7 @@ constexpr int NF = 40, NFP = 48, NH = 64, NMON = 35;
 #define SUR_EG 4
 #endif
 #define SUR_L (2 * SUR_EG)
+#define SUR_LW 32  // lanes per row where the rows are few (sur_split)
 // monomials u_x^a u_y^b u_z^c of degree 0..4 in degree order; each is its
 // parent times one coordinate
 constexpr int kPar[NMON] = {0, 0, 0, 0, 1, 2, 3, 2, 3, 3, 4, 5, 6, 7, 8, 9, 7, 8,
@@ -153,22 +154,6 @@ template <> __device__ __forceinline__ Geo<float> sgeo<float>(const RowArgsS& a,
 // species through arithmetic masks (no divergence between carbon and metal
 // neighbours) and six of the twelve radial etas.  The SUR_EG entry groups
 // are summed by butterfly shuffles at the end.
-#define SUR_ROW_PROLOGUE                                  \
-  int lb = xcd_block(nb_real);                            \
-  if (lb < 0) return;                                     \
-  int gt = lb * blockDim.x + threadIdx.x;                 \
-  int row = gt / SUR_L, q = threadIdx.x & (SUR_L - 1);   \
-  if (row >= a.nrows) return;                             \
-  int i = a.rows[row];                                    \
-  const Geo<R> Gm = sgeo<R>(a, i);                        \
-  const typename Geo<R>::P pi = Gm.at(i);                 \
-  int n = a.nnum[row];                                    \
-  const int* nbrow = a.nbr + (size_t)row * a.stride;      \
-  const int ke = q & 1, eg = q >> 1;                      \
-  const float eta = K.etaa[ke];                           \
-  float e2k[6];                                           \
-  _Pragma("unroll") for (int k = 0; k < 6; ++k) e2k[k] = K.eta2[6 * ke + k];
-
 // sum over the SUR_EG entry groups of a row (lanes q ^ 2k)
 template <int N, class V>
 __device__ __forceinline__ void sum_groups(V* v) {
@@ -179,14 +164,17 @@ __device__ __forceinline__ void sum_groups(V* v) {
   }
 }
 
-// separation of a gathered entry, in FP32 (dr in FP64 then rounded, or fixed point)
+// separation of a gathered entry, in FP32 (dr in FP64 then rounded, or fixed
+// point).  The lead entry of a block and the other three round their squares
+// in another order: descriptors keep the bits they have had, since a last bit
+// can move a BF16 input of the network.
 template <class R>
 __device__ __forceinline__ float sur_dr_rec(const Geo<R>& Gm, const typename Geo<R>::P& pi,
-                                            const typename Geo<R>::P& pj, float& x, float& y, float& z) {
+                                            const typename Geo<R>::P& pj, bool lead, float& x, float& y, float& z) {
   R dx, dy, dz;
   Gm.d2(pi, pj, dx, dy, dz);
   x = (float)dx; y = (float)dy; z = (float)dz;
-  return x * x + y * y + z * z;
+  return lead ? fmaf(z, z, fmaf(y, y, x * x)) : fmaf(z, z, fmaf(x, x, y * y));
 }
 
 // The row walks take the row in blocks of four consecutive entries: the lanes
@@ -194,12 +182,18 @@ __device__ __forceinline__ float sur_dr_rec(const Geo<R>& Gm, const typename Geo
 // index load (rows start on 16 bytes and are padded past their end), then
 // the four records, group bits and AUXF values are gathered before the
 // arithmetic on the first, so a block waits on two memory latencies rather
-// than every entry on one.  Entries past the row's end are skipped.
+// than every entry on one; in the mixed path the next block's indices are
+// loaded beside it (in FP64 they would spill).  Entries past the row's end are
+// skipped.
 #define SUR_NOAUX(j) 0
 #define SUR_WALK_BEGIN(AUXT, AUXF) SUR_WALK_BEGIN_G(AUXT, AUXF, eg, SUR_EG)
 #define SUR_WALK_BEGIN_G(AUXT, AUXF, GRP, NGRP)                                                       \
+  int4 nx_;                                                                                           \
+  if constexpr (sizeof(R) == 4) nx_ = *reinterpret_cast<const int4*>(nbrow + 4 * min((GRP), max(n - 1, 0) >> 2)); \
   for (int p0 = 4 * (GRP); p0 < n; p0 += 4 * (NGRP)) {                                                \
-    const int4 v4_ = *reinterpret_cast<const int4*>(nbrow + p0);                                      \
+    if constexpr (sizeof(R) == 8) nx_ = *reinterpret_cast<const int4*>(nbrow + p0);                   \
+    const int4 v4_ = nx_;                                                                             \
+    if constexpr (sizeof(R) == 4) nx_ = *reinterpret_cast<const int4*>(nbrow + min(p0 + 4 * (NGRP), (n - 1) & ~3)); \
     const int jj_[4] = {v4_.x, p0 + 1 < n ? v4_.y : i, p0 + 2 < n ? v4_.z : i, p0 + 3 < n ? v4_.w : i}; \
     typename Geo<R>::P pp_[4];                                                                        \
     uint32_t mm_[4];                                                                                  \
@@ -224,7 +218,7 @@ __device__ __forceinline__ float sur_dr_rec(const Geo<R>& Gm, const typename Geo
 __device__ __forceinline__ void sur_cut(const SurK& K, float r, float& fc, float& fcp) {
   float s, c;
   __sincosf(K.pirc * r, &s, &c);
-  fc = 0.5f + 0.5f * c;
+  fc = fmaf(c, 0.5f, 0.5f);
   fcp = -0.5f * K.pirc * s;
 }
 
@@ -232,14 +226,14 @@ __device__ __forceinline__ void sur_cut(const SurK& K, float r, float& fc, float
 __device__ __forceinline__ void g5_of(const float* S, float* out) {
   out[0] = S[0] + S[1];
   out[1] = S[0] - S[1];
-  out[2] = 0.125f * (S[0] + 4.0f * S[1] + 6.0f * S[2] + 4.0f * S[3] + S[4]);
-  out[3] = 0.125f * (S[0] - 4.0f * S[1] + 6.0f * S[2] - 4.0f * S[3] + S[4]);
+  out[2] = 0.125f * (fmaf(4.0f, S[3], fmaf(6.0f, S[2], fmaf(4.0f, S[1], S[0]))) + S[4]);
+  out[3] = 0.125f * (fmaf(-4.0f, S[3], fmaf(6.0f, S[2], fmaf(-4.0f, S[1], S[0]))) + S[4]);
 }
 // adjoint of g5_of: dE/dS[n] from dE/dG5[0..3]
 __device__ __forceinline__ void g5_adj(const float* g, float* dS) {
   float a = 0.125f * (g[2] + g[3]), b = 0.125f * (g[2] - g[3]);
-  dS[0] = g[0] + g[1] + a;
-  dS[1] = g[0] - g[1] + 4.0f * b;
+  dS[0] = fmaf(0.125f, g[2] + g[3], g[0] + g[1]);
+  dS[1] = fmaf(4.0f, b, g[0] - g[1]);
   dS[2] = 6.0f * a;
   dS[3] = 4.0f * b;
   dS[4] = a;
@@ -247,7 +241,33 @@ __device__ __forceinline__ void g5_adj(const float* g, float* dS) {
 
 // The row passes as functions of one row's lanes, shared by the separate
 // kernels (training reads their stored moments and features) and the fused
-// inference kernel (k_sur_fused), so both give the same bits.
+// inference kernel (k_sur_fused), so both give the same bits: where a sum of
+// products leaves a choice, its fused multiply-adds are written out (the
+// compiler's own choice differs from one kernel to another).
+
+// the terms of one entry in the moments walk
+struct MomentTerms {
+  float ex, w, fc, u[3];
+  bool cj;
+  __device__ __forceinline__ MomentTerms(const SurK& K, float dx, float dy, float dz, float r2, float eta, bool cj)
+      : cj(cj) {
+    const float r = __builtin_amdgcn_sqrtf(r2), ir = 1.0f / r;
+    float fcp;
+    sur_cut(K, r, fc, fcp);
+    ex = __expf(-eta * r2);
+    w = ex * fc;
+    u[0] = dx * ir; u[1] = dy * ir; u[2] = dz * ir;
+  }
+  // the weight among the carbon neighbours and among the others, the latter
+  // with the rounding of w where the neighbour is carbon
+  __device__ __forceinline__ float carbon() const { return cj ? w : 0.0f; }
+  __device__ __forceinline__ float other(float wc) const { return fmaf(ex, fc, -wc); }
+  __device__ __forceinline__ void monomials(float* mono) const {
+    mono[0] = 1.0f;
+#pragma unroll
+    for (int t = 1; t < NMON; ++t) mono[t] = mono[kPar[t]] * u[kCrd[t]];
+  }
+};
 
 // moments and radial sums of the row over lane q's entries, summed over the
 // four entry groups (every lane of the row holds the totals of its eta)
@@ -263,28 +283,20 @@ __device__ __forceinline__ void sur_moments(const SurK& K, const Geo<R>& Gm, con
   for (int k = 0; k < 6; ++k) { gc[k] = 0.0f; gx[k] = 0.0f; }
   SUR_WALK_BEGIN(int, SUR_NOAUX)
     float dx, dy, dz;
-    float r2 = sur_dr_rec<R>(Gm, pi, pj, dx, dy, dz);
+    float r2 = sur_dr_rec<R>(Gm, pi, pj, u_ == 0, dx, dy, dz);
     if (!(r2 < K.rc2)) continue;
-    bool cj = (mj & K.bit1) != 0;
-    float r = __builtin_amdgcn_sqrtf(r2), ir = 1.0f / r;
-    float fc, fcp;
-    sur_cut(K, r, fc, fcp);
-    (void)fcp;
-    float w = __expf(-eta * r2) * fc;
-    float wc = cj ? w : 0.0f, wx = w - wc;
-    float u[3] = {dx * ir, dy * ir, dz * ir};
+    const MomentTerms T(K, dx, dy, dz, r2, eta, (mj & K.bit1) != 0);
     float mono[NMON];
-    mono[0] = 1.0f;
-#pragma unroll
-    for (int t = 1; t < NMON; ++t) mono[t] = mono[kPar[t]] * u[kCrd[t]];
+    T.monomials(mono);
+    const float wc = T.carbon(), wx = T.other(wc);
 #pragma unroll
     for (int t = 0; t < NMON; ++t) { mc[t] += wc * mono[t]; mx[t] += wx * mono[t]; }
-    dd[0] += wc * w;
+    dd[0] += wc * T.w;
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
-      float v = __expf(-e2k[k] * r2) * fc;
-      gc[k] += cj ? v : 0.0f;
-      gx[k] += cj ? 0.0f : v;
+      float v = __expf(-e2k[k] * r2) * T.fc;
+      gc[k] += T.cj ? v : 0.0f;
+      gx[k] += T.cj ? 0.0f : v;
     }
   SUR_WALK_END
   sum_groups<NMON>(mc);
@@ -295,19 +307,98 @@ __device__ __forceinline__ void sur_moments(const SurK& K, const Geo<R>& Gm, con
   dd0 = dd[0];
 }
 
+// from lanes that hold one species' moments and three of its radial sums
+// (lanes q and q ^ 8 differ in the species, q and q ^ 16 in the three) to
+// all of them in every lane
+__device__ __forceinline__ void both_species(const float* m, const float* g, bool metal, bool high, float* mc,
+                                             float* mx, float* gc, float* gx) {
+#pragma unroll
+  for (int t = 0; t < NMON; ++t) {
+    const float o = __shfl_xor(m[t], 8, SUR_LW);
+    mc[t] = metal ? o : m[t];
+    mx[t] = metal ? m[t] : o;
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const float s = __shfl_xor(g[k], 8, SUR_LW), gc0 = metal ? s : g[k], gx0 = metal ? g[k] : s;
+    const float c1 = __shfl_xor(gc0, 16, SUR_LW), x1 = __shfl_xor(gx0, 16, SUR_LW);
+    gc[k] = high ? c1 : gc0; gc[3 + k] = high ? gc0 : c1;
+    gx[k] = high ? x1 : gx0; gx[3 + k] = high ? gx0 : x1;
+  }
+}
+
+// The same sums in the same order by SUR_LW lanes of a row (SUR_LW / SUR_L
+// times the lanes): lanes q and q ^ 8 take the same entries for one species
+// each, q and q ^ 16 three of the six radial etas each.  Every lane returns
+// the totals of both, so all that follows is as above.
+template <class R>
+__device__ __forceinline__ void sur_moments_wide(const SurK& K, const Geo<R>& Gm, const typename Geo<R>::P& pi,
+                                                 const int* __restrict__ nbrow, int n, int i, int q, int eg, float eta,
+                                                 const float* e2k, const uint32_t* __restrict__ mask, float* mc,
+                                                 float* mx, float& dd0, float* gc, float* gx) {
+  const bool metal = (q & 8) != 0, high = (q & 16) != 0;
+  float m[NMON], g[3] = {0.0f, 0.0f, 0.0f}, e2[3], dd[1] = {0.0f};
+#pragma unroll
+  for (int t = 0; t < NMON; ++t) m[t] = 0.0f;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) e2[k] = high ? e2k[3 + k] : e2k[k];
+  SUR_WALK_BEGIN(int, SUR_NOAUX)
+    float dx, dy, dz;
+    float r2 = sur_dr_rec<R>(Gm, pi, pj, u_ == 0, dx, dy, dz);
+    if (!(r2 < K.rc2)) continue;
+    const MomentTerms T(K, dx, dy, dz, r2, eta, (mj & K.bit1) != 0);
+    float mono[NMON];
+    T.monomials(mono);
+    const bool mine = T.cj != metal;
+    const float wc = T.carbon(), ws = metal ? T.other(wc) : wc;
+#pragma unroll
+    for (int t = 0; t < NMON; ++t) m[t] += ws * mono[t];
+    dd[0] += wc * T.w;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) g[k] += mine ? __expf(-e2[k] * r2) * T.fc : 0.0f;
+  SUR_WALK_END
+  sum_groups<NMON>(m);
+  sum_groups<1>(dd);
+  sum_groups<3>(g);
+  dd0 = dd[0];
+  both_species(m, g, metal, high, mc, mx, gc, gx);
+}
+
+// by the LN lanes of a row, q this lane's place among them
+template <class R, int LN>
+__device__ __forceinline__ void sur_moments_of(const SurK& K, const Geo<R>& Gm, const typename Geo<R>::P& pi,
+                                               const int* __restrict__ nbrow, int n, int i, int q,
+                                               const uint32_t* __restrict__ mask, float* mc, float* mx, float& dd,
+                                               float* gc, float* gx) {
+  const int ke = q & 1, eg = (q >> 1) & (SUR_EG - 1);
+  const float eta = K.etaa[ke];
+  float e2k[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) e2k[k] = K.eta2[6 * ke + k];
+  if constexpr (LN == SUR_L) sur_moments<R>(K, Gm, pi, nbrow, n, i, eg, eta, e2k, mask, mc, mx, dd, gc, gx);
+  else sur_moments_wide<R>(K, Gm, pi, nbrow, n, i, q, eg, eta, e2k, mask, mc, mx, dd, gc, gx);
+}
+
 // the 20 descriptors of angular eta ke from the row's sums, into Gr[0..39]
 __device__ __forceinline__ void sur_features(int ke, const float* mc, const float* mx, float dd, const float* gc,
                                              const float* gx, float* Gr) {
 #pragma unroll
   for (int k = 0; k < 6; ++k) { Gr[6 * ke + k] = gc[k]; Gr[12 + 6 * ke + k] = gx[k]; }
-  float Scc[5] = {0, 0, 0, 0, 0}, Scx[5] = {0, 0, 0, 0, 0};
+  // the first term of a degree is added to the rounded second one
+  float Scc[5], Scx[5];
 #pragma unroll
   for (int t = 0; t < NMON; ++t) {
-    Scc[kDeg[t]] += kMul[t] * mc[t] * mc[t];
-    Scx[kDeg[t]] += kMul[t] * mc[t] * mx[t];
+    const float k = kMul[t] * mc[t];
+    const int d = kDeg[t];
+    const bool head = t == 0 || kDeg[t - 1] != d, second = !head && (t == 1 || kDeg[t >= 2 ? t - 2 : 0] != d);
+    Scx[d] = head ? k * mx[t] : fmaf(k, mx[t], Scx[d]);
+    if (head) Scc[d] = mc[t];
+    else if (second) Scc[d] = fmaf(Scc[d], Scc[d], k * mc[t]);
+    else Scc[d] = fmaf(mc[t], k, Scc[d]);
   }
+  Scc[0] = fmaf(mc[0], mc[0], -dd);
 #pragma unroll
-  for (int m = 0; m < 5; ++m) Scc[m] -= dd;
+  for (int m = 1; m < 5; ++m) Scc[m] -= dd;
   float o[4];
   g5_of(Scc, o);
 #pragma unroll
@@ -317,12 +408,31 @@ __device__ __forceinline__ void sur_features(int ke, const float* mc, const floa
   for (int m = 0; m < 4; ++m) Gr[32 + ke * 4 + m] = o[m];
 }
 
-template <class R>
-__global__ void __launch_bounds__(256) k_sur_desc(RowArgsS a, SurK K, const uint32_t* __restrict__ mask, int nb_real) {
-  SUR_ROW_PROLOGUE
+// The blocks of a row pass: nmain blocks of 256 / SUR_L rows, then ntail
+// blocks of 256 / SUR_LW rows with more lanes each (sur_split)
+struct SurSplit {
+  int nmain, ntail;
+  int grid() const { return pad8(nmain) + ntail; }
+};
+__device__ __forceinline__ int sur_main_block(const SurSplit& S) {
+  const int nb = (S.nmain + 7) & ~7, b = blockIdx.x;
+  const int lb = (b & 7) * (nb >> 3) + (b >> 3);  // as xcd_block
+  return lb < S.nmain ? lb : -1;
+}
+
+template <class R, int LN>
+__device__ __forceinline__ void sur_desc_rows(const RowArgsS& a, const SurK& K, const uint32_t* __restrict__ mask,
+                                              int row0) {
+  const int row = row0 + threadIdx.x / LN, q = threadIdx.x & (LN - 1);
+  if (row >= a.nrows) return;
+  const int i = a.rows[row], n = a.nnum[row];
+  const Geo<R> Gm = sgeo<R>(a, i);
+  const typename Geo<R>::P pi = Gm.at(i);
+  const int* nbrow = a.nbr + (size_t)row * a.stride;
+  const int ke = q & 1;
   float mc[NMON], mx[NMON], dd, gc[6], gx[6];
-  sur_moments<R>(K, Gm, pi, nbrow, n, i, eg, eta, e2k, mask, mc, mx, dd, gc, gx);
-  if (eg != 0) return;
+  sur_moments_of<R, LN>(K, Gm, pi, nbrow, n, i, q, mask, mc, mx, dd, gc, gx);
+  if (q >= 2) return;
   float* Mc = K.M + ((size_t)row * 4 + ke) * 36;
   float* Mx = K.M + ((size_t)row * 4 + 2 + ke) * 36;
 #pragma unroll
@@ -330,6 +440,17 @@ __global__ void __launch_bounds__(256) k_sur_desc(RowArgsS a, SurK K, const uint
   Mc[NMON] = dd;
   Mx[NMON] = 0.0f;
   sur_features(ke, mc, mx, dd, gc, gx, K.G + (size_t)row * NF);
+}
+
+template <class R>
+__global__ void __launch_bounds__(256) k_sur_desc(RowArgsS a, SurK K, const uint32_t* __restrict__ mask, SurSplit S) {
+  const int t = (int)blockIdx.x - ((S.nmain + 7) & ~7);
+  if (t >= 0) {
+    sur_desc_rows<R, SUR_LW>(a, K, mask, S.nmain * (256 / SUR_L) + t * (256 / SUR_LW));
+  } else {
+    const int lb = sur_main_block(S);
+    if (lb >= 0) sur_desc_rows<R, SUR_L>(a, K, mask, lb * (256 / SUR_L));
+  }
 }
 
 // Perceptron on MFMA: 16 atoms per wavefront.  Writes E_i (e_row) and
@@ -466,27 +587,44 @@ __device__ __forceinline__ void sur_back_coef(const float* g, int ke, const floa
 #pragma unroll
   for (int t = 0; t < NMON; ++t) {
     float mcv = Mc[t], mxv = Mx[t];
-    ac[t] = kMul[t] * (2.0f * mcv * dScc[kDeg[t]] + mxv * dScx[kDeg[t]]);
+    ac[t] = kMul[t] * fmaf(2.0f * mcv, dScc[kDeg[t]], mxv * dScx[kDeg[t]]);
     ax[t] = kMul[t] * mcv * dScx[kDeg[t]];
   }
 }
 
-// the adjoints of one row and eta in LDS: ax at s[0..NMON), ac at
-// s[NMON..2 NMON); the address depends on the entry's species, so the reads
-// stay in the entry loop instead of occupying 70 registers for the whole walk
+// The adjoints of one row and eta in LDS: ax at s[0..NMON), ac at s[36..36 +
+// NMON); the address depends on the entry's species, so the reads stay in the
+// entry loop instead of occupying 70 registers for the whole walk.  They are
+// read four at a time; with a pitch of 76 floats the 16 places that the lanes
+// of a wavefront (eight rows, two species) read at once lie in distinct banks.
+constexpr int CA = 36, CP = 2 * CA + 4;
 struct SurCoefLds {
   const float* s;
-  __device__ __forceinline__ float operator()(bool cj, int t) const { return s[(cj ? NMON : 0) + t]; }
+  __device__ __forceinline__ void load(bool cj, float* a) const {
+    const float4* p = reinterpret_cast<const float4*>(s + (cj ? CA : 0));
+#pragma unroll
+    for (int t = 0; t < CA / 4; ++t) {
+      const float4 v = p[t];
+      const float w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (4 * t + k < NMON) a[4 * t + k] = w[k];
+    }
+  }
+  static __device__ __forceinline__ void store(float* s, const float* ac, const float* ax) {
+#pragma unroll
+    for (int t = 0; t < NMON; ++t) { s[t] = ax[t]; s[CA + t] = ac[t]; }
+  }
 };
 
 // dE_i/d(dr_ij) of every entry of the row (into drow) from dE/dG of the row
 // (g, in LDS) and the monomial adjoints of the two angular etas (coef0,
-// coef1).  Lane q of the row takes the entry blocks q, q + SUR_L, ... and
+// coef1).  Lane q of the row's LN takes the entry blocks q, q + LN, ... and
 // both etas of each entry, so the separation, cutoff and monomials are formed
 // once per entry; the etas run one after the other (a loop, so only one set
 // of adjoints is live) and d_ij is the eta-0 share plus the eta-1 share.
 // Every lane returns the row's sum_j dE_i/d(dr_ij) (FP64).
-template <class R, class C>
+template <class R, int LN, class C>
 __device__ __forceinline__ void sur_back_walk(const SurK& K, const Geo<R>& Gm, const typename Geo<R>::P& pi,
                                               const int* __restrict__ nbrow, int n, int i, int q,
                                               const uint32_t* __restrict__ mask, const float* g, const C& coef0,
@@ -494,17 +632,17 @@ __device__ __forceinline__ void sur_back_walk(const SurK& K, const Geo<R>& Gm, c
   float dD[2];
 #pragma unroll
   for (int ke = 0; ke < 2; ++ke) {
-    float gcc[4], gcx[4], dScc[5], dScx[5];
+    float gcc[4], dScc[5];
 #pragma unroll
-    for (int m = 0; m < 4; ++m) { gcc[m] = g[24 + ke * 4 + m]; gcx[m] = g[32 + ke * 4 + m]; }
+    for (int m = 0; m < 4; ++m) gcc[m] = g[24 + ke * 4 + m];
     g5_adj(gcc, dScc);
-    g5_adj(gcx, dScx);
-    dD[ke] = -(dScc[0] + dScc[1] + dScc[2] + dScc[3] + dScc[4]);
+    const float a = 0.125f * (gcc[2] + gcc[3]), b = 0.125f * (gcc[2] - gcc[3]);
+    dD[ke] = -fmaf(0.125f, gcc[2] + gcc[3], fmaf(4.0f, b, fmaf(6.0f, a, dScc[0] + dScc[1])));
   }
   sf[0] = 0.0; sf[1] = 0.0; sf[2] = 0.0;
-  SUR_WALK_BEGIN_G(int, SUR_NOAUX, q, SUR_L)
+  SUR_WALK_BEGIN_G(int, SUR_NOAUX, q, LN)
     float dx, dy, dz;
-    float r2 = sur_dr_rec<R>(Gm, pi, pj, dx, dy, dz);
+    float r2 = sur_dr_rec<R>(Gm, pi, pj, u_ == 0, dx, dy, dz);
     float c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
     if (r2 < K.rc2) {
       bool cj = (mj & K.bit1) != 0;
@@ -523,32 +661,30 @@ __device__ __forceinline__ void sur_back_walk(const SurK& K, const Geo<R>& Gm, c
         const C coef = ke ? coef1 : coef0;
         const float eta = K.etaa[ke];
         float ex = __expf(-eta * r2);
-        float w = ex * fc, wp = ex * (fcp - 2.0f * eta * r * fc);
+        float w = ex * fc, wp = ex * fmaf(-fc, 2.0f * eta * r, fcp);
         float adj[NMON];
+        coef.load(cj, adj);
         float P = 0.0f;
 #pragma unroll
-        for (int t = 0; t < NMON; ++t) {
-          adj[t] = coef(cj, t);
-          P += adj[t] * mono[t];
-        }
+        for (int t = 0; t < NMON; ++t) P = fmaf(adj[t], mono[t], P);
         float gu[3] = {0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int t = NMON - 1; t >= 1; --t) {
-          adj[kPar[t]] += adj[t] * u[kCrd[t]];
-          gu[kCrd[t]] += adj[t] * mono[kPar[t]];
+          adj[kPar[t]] = fmaf(adj[t], u[kCrd[t]], adj[kPar[t]]);
+          gu[kCrd[t]] = fmaf(adj[t], mono[kPar[t]], gu[kCrd[t]]);
         }
-        float Q = u[0] * gu[0] + u[1] * gu[1] + u[2] * gu[2];
-        float wr = w * ir;
-        float cu = wp * P - wr * Q + (cj ? 2.0f * (ke ? dD[1] : dD[0]) * w * wp : 0.0f);
+        const float Q = fmaf(u[2], gu[2], fmaf(u[1], gu[1], u[0] * gu[0]));
+        const float wr = w * ir;
+        float cu = fmaf(wp, P, -(wr * Q)) + (cj ? 2.0f * (ke ? dD[1] : dD[0]) * w * wp : 0.0f);
 #pragma unroll
         for (int k = 0; k < 6; ++k) {
           const float e2 = K.eta2[6 * ke + k];
           float x = __expf(-e2 * r2);
-          cu += gr[6 * ke + k] * x * (fcp - 2.0f * e2 * r * fc);
+          cu = fmaf(gr[6 * ke + k] * x, fmaf(-fc, 2.0f * e2 * r, fcp), cu);
         }
-        c0 += cu * u[0] + wr * gu[0];
-        c1 += cu * u[1] + wr * gu[1];
-        c2 += cu * u[2] + wr * gu[2];
+        c0 += fmaf(wr, gu[0], cu * u[0]);
+        c1 += fmaf(wr, gu[1], cu * u[1]);
+        c2 += fmaf(wr, gu[2], cu * u[2]);
       }
     }
     drow[p] = make_float4(c0, c1, c2, 0.0f);
@@ -557,31 +693,25 @@ __device__ __forceinline__ void sur_back_walk(const SurK& K, const Geo<R>& Gm, c
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
 #pragma unroll
-    for (int o = 1; o < SUR_L; o <<= 1) sf[c] += __shfl_xor(sf[c], o, SUR_L);
+    for (int o = 1; o < LN; o <<= 1) sf[c] += __shfl_xor(sf[c], o, LN);
   }
 }
 
 // dE_i/d(dr_ij) of every entry of the row, and the row atom's own share
 // sum_j dE_i/d(dr_ij) (FP64); the row's dE/dG and (lanes 0 and 1) the
 // adjoints of each eta go to LDS first
-template <class R>
-__global__ void __launch_bounds__(256) k_sur_back(RowArgsS a, SurK K, const uint32_t* __restrict__ mask, int nb_real) {
-  constexpr int RB = 256 / SUR_L, CP = 2 * NMON + 3;
-  __shared__ float sc[RB * 2 * CP], sg[RB * NF];
-  const int lb = xcd_block(nb_real);
-  if (lb < 0) return;
-  const int row = (lb * blockDim.x + threadIdx.x) / SUR_L, q = threadIdx.x & (SUR_L - 1);
-  const int lrow = threadIdx.x / SUR_L;
+template <class R, int LN>
+__device__ __forceinline__ void sur_back_rows(const RowArgsS& a, const SurK& K, const uint32_t* __restrict__ mask,
+                                              int row0, float* sc, float* sg) {
+  const int lrow = threadIdx.x / LN, row = row0 + lrow, q = threadIdx.x & (LN - 1);
   const bool live = row < a.nrows;
   if (live)
-    for (int k = q; k < NF; k += SUR_L) sg[lrow * NF + k] = K.gG[(size_t)row * NF + k];
+    for (int k = q; k < NF; k += LN) sg[lrow * NF + k] = K.gG[(size_t)row * NF + k];
   if (live && q < 2) {
     float ac[NMON], ax[NMON];
     sur_back_coef(K.gG + (size_t)row * NF, q, K.M + ((size_t)row * 4 + q) * 36, K.M + ((size_t)row * 4 + 2 + q) * 36,
                   ac, ax);
-    float* sC = sc + (lrow * 2 + q) * CP;
-#pragma unroll
-    for (int t = 0; t < NMON; ++t) { sC[t] = ax[t]; sC[NMON + t] = ac[t]; }
+    SurCoefLds::store(sc + (lrow * 2 + q) * CP, ac, ax);
   }
   __syncthreads();
   if (!live) return;
@@ -589,79 +719,94 @@ __global__ void __launch_bounds__(256) k_sur_back(RowArgsS a, SurK K, const uint
   const Geo<R> Gm = sgeo<R>(a, i);
   const typename Geo<R>::P pi = Gm.at(i);
   double sf[3];
-  sur_back_walk<R>(K, Gm, pi, a.nbr + (size_t)row * a.stride, a.nnum[row], i, q, mask, sg + lrow * NF,
-                   SurCoefLds{sc + lrow * 2 * CP}, SurCoefLds{sc + (lrow * 2 + 1) * CP}, K.d + (size_t)row * K.stride0,
-                   sf);
+  sur_back_walk<R, LN>(K, Gm, pi, a.nbr + (size_t)row * a.stride, a.nnum[row], i, q, mask, sg + lrow * NF,
+                       SurCoefLds{sc + lrow * 2 * CP}, SurCoefLds{sc + (lrow * 2 + 1) * CP},
+                       K.d + (size_t)row * K.stride0, sf);
   if (q == 0) K.fself[row] = make_double4(sf[0], sf[1], sf[2], 0.0);
 }
 
-// The three row passes of a step in one kernel (inference): a workgroup's
-// 256 / SUR_L rows take their moments, their descriptors go to LDS, one
-// wavefront per 16 rows runs the network on them (weights staged in LDS),
-// and the rows walk again
-// for dE/d(dr), the monomial adjoints of their moments in LDS where the
-// weights were, each lane taking both etas of its entries.  The moments, descriptors and dE/dG never reach memory; the
-// results are those of k_sur_desc, k_sur_mlp and k_sur_back.
-// Three workgroups fit a CU by LDS; the bound of three waves per SIMD caps
-// the registers at 168 (a few spill around the moments walk).
 template <class R>
-__global__ void __launch_bounds__(256, 3) k_sur_fused(RowArgsS a, SurK K, const uint32_t* __restrict__ mask,
-                                                   int nb_real) {
-  constexpr int RB = 256 / SUR_L;  // rows of the workgroup
-  // adjoints of one row and eta: ax then ac; the odd pitch puts the 16
-  // row/eta blocks of a wavefront in distinct banks
-  constexpr int CP = 2 * NMON + 3;
-  static_assert(RB * 2 * CP * 4 <= SUR_LNW * 2, "adjoints exceed the weight tile");
-  __shared__ __align__(16) union {
-    uint16_t w[SUR_LNW];
-    float c[RB * 2 * CP];
-  } sWC;
-  uint16_t* sW = sWC.w;
-  __shared__ float sfp[SUR_NFP_];
-  __shared__ float sG[RB * NF], sgG[RB * NF];
-  const int lb = xcd_block(nb_real);
-  if (lb < 0) return;
+__global__ void __launch_bounds__(256) k_sur_back(RowArgsS a, SurK K, const uint32_t* __restrict__ mask, SurSplit S) {
+  constexpr int RB = 256 / SUR_L, RW = 256 / SUR_LW;
+  __shared__ __align__(16) float sc[RB * 2 * CP];
+  __shared__ float sg[RB * NF];
+  const int t = (int)blockIdx.x - ((S.nmain + 7) & ~7);
+  if (t >= 0) {
+    sur_back_rows<R, SUR_LW>(a, K, mask, S.nmain * RB + t * RW, sc, sg);
+  } else {
+    const int lb = sur_main_block(S);
+    if (lb >= 0) sur_back_rows<R, SUR_L>(a, K, mask, lb * RB, sc, sg);
+  }
+}
+
+// The three row passes of a step in one kernel (inference): a workgroup's
+// rows take their moments, their descriptors go to LDS, one wavefront per 16
+// rows runs the network on them (weights staged in LDS), and the rows walk
+// again for dE/d(dr), the monomial adjoints of their moments in LDS where the
+// weights were, each lane taking both etas of its entries.  The moments,
+// descriptors and dE/dG never reach memory; the results are those of
+// k_sur_desc, k_sur_mlp and k_sur_back.
+// Bound by the vector units (the walks' products; three wavefronts per SIMD
+// by registers and LDS) where the rows fill the card.
+template <class R, int LN>
+__device__ __forceinline__ void sur_fused_rows(const RowArgsS& a, const SurK& K, const uint32_t* __restrict__ mask,
+                                               int row0, uint16_t* sW, float* sC, float* sfp, float* sG, float* sgG) {
+  constexpr int RB = 256 / LN;  // rows of the workgroup
   stage_network(K, sW, sfp);
-  const int row = (lb * blockDim.x + threadIdx.x) / SUR_L, q = threadIdx.x & (SUR_L - 1), lrow = threadIdx.x / SUR_L;
+  const int lrow = threadIdx.x / LN, row = row0 + lrow, q = threadIdx.x & (LN - 1);
   const bool live = row < a.nrows;
   const int i = live ? a.rows[row] : a.rows[0];
   const Geo<R> Gm = sgeo<R>(a, i);
   const typename Geo<R>::P pi = Gm.at(i);
   const int n = live ? a.nnum[row] : 0;
   const int* nbrow = a.nbr + (size_t)(live ? row : 0) * a.stride;
-  const int ke = q & 1, eg = q >> 1;
-  const float eta = K.etaa[ke];
-  float e2k[6];
-#pragma unroll
-  for (int k = 0; k < 6; ++k) e2k[k] = K.eta2[6 * ke + k];
+  const int ke = q & 1;
+  const bool first = q < 2;  // entry group 0
   float mc[NMON], mx[NMON], dd, gc[6], gx[6];
-  sur_moments<R>(K, Gm, pi, nbrow, n, i, eg, eta, e2k, mask, mc, mx, dd, gc, gx);
-  if (eg == 0) sur_features(ke, mc, mx, dd, gc, gx, sG + lrow * NF);
+  sur_moments_of<R, LN>(K, Gm, pi, nbrow, n, i, q, mask, mc, mx, dd, gc, gx);
+  if (first) sur_features(ke, mc, mx, dd, gc, gx, sG + lrow * NF);
   __syncthreads();
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (w < RB / 16) {
+  if (w < (RB + 15) / 16) {
     const int lr = 16 * w + (lane & 15);
-    const int rr = lb * RB + lr;
-    const bool ok = rr < a.nrows;
-    sur_mlp16(lane, ok, sG + lr * NF, sfp, sW, K.e_row + (ok ? rr : 0), sgG + lr * NF);
+    const int rr = row0 + lr;
+    const bool ok = lr < RB && rr < a.nrows;
+    const int ls = lr < RB ? lr : 0;
+    sur_mlp16(lane, ok, sG + ls * NF, sfp, sW, K.e_row + (ok ? rr : 0), sgG + ls * NF);
   }
   __syncthreads();
   // the weights are no longer read: their tile takes the adjoints
-  float* sC = sWC.c + (lrow * 2 + ke) * CP;
   if (live) {
     float ac[NMON], ax[NMON];
     sur_back_coef(sgG + lrow * NF, ke, mc, mx, ac, ax);
-    if (eg == 0) {
-#pragma unroll
-      for (int t = 0; t < NMON; ++t) { sC[t] = ax[t]; sC[NMON + t] = ac[t]; }
-    }
+    if (first) SurCoefLds::store(sC + (lrow * 2 + ke) * CP, ac, ax);
   }
   __syncthreads();
   if (!live) return;
   double sf[3];
-  sur_back_walk<R>(K, Gm, pi, nbrow, n, i, q, mask, sgG + lrow * NF, SurCoefLds{sWC.c + lrow * 2 * CP},
-                   SurCoefLds{sWC.c + (lrow * 2 + 1) * CP}, K.d + (size_t)row * K.stride0, sf);
+  sur_back_walk<R, LN>(K, Gm, pi, nbrow, n, i, q, mask, sgG + lrow * NF, SurCoefLds{sC + lrow * 2 * CP},
+                       SurCoefLds{sC + (lrow * 2 + 1) * CP}, K.d + (size_t)row * K.stride0, sf);
   if (q == 0) K.fself[row] = make_double4(sf[0], sf[1], sf[2], 0.0);
+}
+
+template <class R>
+__global__ void __launch_bounds__(256, 3) k_sur_fused(RowArgsS a, SurK K, const uint32_t* __restrict__ mask,
+                                                      SurSplit S) {
+  constexpr int RB = 256 / SUR_L, RW = 256 / SUR_LW;
+  static_assert(RB * 2 * CP * 4 <= SUR_LNW * 2, "adjoints exceed the weight tile");
+  __shared__ __align__(16) union {
+    uint16_t w[SUR_LNW];
+    float c[RB * 2 * CP];
+  } sWC;
+  __shared__ float sfp[SUR_NFP_];
+  __shared__ float sG[RB * NF], sgG[RB * NF];
+  const int t = (int)blockIdx.x - ((S.nmain + 7) & ~7);
+  if (t >= 0) {
+    sur_fused_rows<R, SUR_LW>(a, K, mask, S.nmain * RB + t * RW, sWC.w, sWC.c, sfp, sG, sgG);
+  } else {
+    const int lb = sur_main_block(S);
+    if (lb >= 0) sur_fused_rows<R, SUR_L>(a, K, mask, lb * RB, sWC.w, sWC.c, sfp, sG, sgG);
+  }
 }
 
 // F_a = sum_{j in N(a)} d_aj - sum_{i: a in N(i)} d_ia over the rows of the
@@ -776,63 +921,122 @@ __global__ void __launch_bounds__(256) k_sur_resid(int N, const double4* __restr
   if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
-// tangent descriptors dG_i = sum_j dG_i/d(dr_ij) (res_j - res_i)
-template <class R>
-__global__ void __launch_bounds__(256) k_sur_tangent(RowArgsS a, SurK K, const uint32_t* __restrict__ mask,
-                                                     int nb_real) {
-  SUR_ROW_PROLOGUE
-  float dmc[NMON], dmx[NMON], ddd[1] = {0.0f}, dgc[6], dgx[6];
-#pragma unroll
-  for (int t = 0; t < NMON; ++t) { dmc[t] = 0.0f; dmx[t] = 0.0f; }
-#pragma unroll
-  for (int k = 0; k < 6; ++k) { dgc[k] = 0.0f; dgx[k] = 0.0f; }
-  const float4 ri = K.res[i];
-#define SUR_RES(j) K.res[j]
-  SUR_WALK_BEGIN(float4, SUR_RES)
-    float dx, dy, dz;
-    float r2 = sur_dr_rec<R>(Gm, pi, pj, dx, dy, dz);
-    if (!(r2 < K.rc2)) continue;
-    bool cj = (mj & K.bit1) != 0;
-    float r = __builtin_amdgcn_sqrtf(r2), ir = 1.0f / r;
-    float fc, fcp;
+// the terms of one entry in the tangent walk
+struct TangentTerms {
+  float r, ex, fc, fcp, w, wp, ud, u[3], du[3];
+  bool cj;
+  __device__ __forceinline__ TangentTerms(const SurK& K, float dx, float dy, float dz, float r2, float eta, bool cj,
+                                          const float4& ri, const float4& rj)
+      : cj(cj) {
+    r = __builtin_amdgcn_sqrtf(r2);
+    const float ir = 1.0f / r;
     sur_cut(K, r, fc, fcp);
-    float u[3] = {dx * ir, dy * ir, dz * ir};
-    const float4 rj = aj;
-    float de[3] = {rj.x - ri.x, rj.y - ri.y, rj.z - ri.z};
-    float ud = u[0] * de[0] + u[1] * de[1] + u[2] * de[2];
-    float ex = __expf(-eta * r2);
-    float w = ex * fc, wp = ex * (fcp - 2.0f * eta * r * fc);
-    float dw = wp * ud;
-    float du[3] = {(de[0] - u[0] * ud) * ir, (de[1] - u[1] * ud) * ir, (de[2] - u[2] * ud) * ir};
-    float mono[NMON], dmono[NMON];
+    u[0] = dx * ir; u[1] = dy * ir; u[2] = dz * ir;
+    const float de[3] = {rj.x - ri.x, rj.y - ri.y, rj.z - ri.z};
+    ud = fmaf(u[2], de[2], fmaf(u[1], de[1], u[0] * de[0]));
+    ex = __expf(-eta * r2);
+    w = ex * fc;
+    wp = ex * fmaf(-fc, 2.0f * eta * r, fcp);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) du[k] = fmaf(-u[k], ud, de[k]) * ir;
+  }
+  // weights among the carbon neighbours and the others, and their
+  // derivatives, rounded as MomentTerms rounds them
+  __device__ __forceinline__ float carbon() const { return cj ? w : 0.0f; }
+  __device__ __forceinline__ float other(float wc) const { return fmaf(ex, fc, -wc); }
+  __device__ __forceinline__ float dcarbon() const { return cj ? wp * ud : 0.0f; }
+  __device__ __forceinline__ float dother(float dwc) const { return fmaf(ud, wp, -dwc); }
+  __device__ __forceinline__ void monomials(float* mono, float* dmono) const {
     mono[0] = 1.0f;
     dmono[0] = 0.0f;
 #pragma unroll
     for (int t = 1; t < NMON; ++t) {
       mono[t] = mono[kPar[t]] * u[kCrd[t]];
-      dmono[t] = dmono[kPar[t]] * u[kCrd[t]] + mono[kPar[t]] * du[kCrd[t]];
+      dmono[t] = fmaf(dmono[kPar[t]], u[kCrd[t]], mono[kPar[t]] * du[kCrd[t]]);
     }
-    float wc = cj ? w : 0.0f, wx = w - wc, dwc = cj ? dw : 0.0f, dwx = dw - dwc;
+  }
+  __device__ __forceinline__ float radial(float e2, float r2) const {
+    return __expf(-e2 * r2) * fmaf(-fc, 2.0f * e2 * r, fcp) * ud;
+  }
+};
+
+// tangent descriptors dG_i = sum_j dG_i/d(dr_ij) (res_j - res_i), by the LN
+// lanes of a row: with SUR_LW lanes the entries' sums are split by species and
+// radial eta as in sur_moments_wide
+template <class R, int LN>
+__device__ __forceinline__ void sur_tangent_rows(const RowArgsS& a, const SurK& K, const uint32_t* __restrict__ mask,
+                                                 int row0) {
+  const int row = row0 + threadIdx.x / LN, q = threadIdx.x & (LN - 1);
+  if (row >= a.nrows) return;
+  const int i = a.rows[row], n = a.nnum[row];
+  const Geo<R> Gm = sgeo<R>(a, i);
+  const typename Geo<R>::P pi = Gm.at(i);
+  const int* nbrow = a.nbr + (size_t)row * a.stride;
+  const int ke = q & 1, eg = (q >> 1) & (SUR_EG - 1);
+  const float eta = K.etaa[ke];
+  float dmc[NMON], dmx[NMON], ddd[1] = {0.0f}, dgc[6], dgx[6];
+  const float4 ri = K.res[i];
+#define SUR_RES(j) K.res[j]
+  if constexpr (LN == SUR_L) {
 #pragma unroll
-    for (int t = 0; t < NMON; ++t) {
-      dmc[t] += dwc * mono[t] + wc * dmono[t];
-      dmx[t] += dwx * mono[t] + wx * dmono[t];
-    }
-    ddd[0] += 2.0f * wc * dw;
+    for (int t = 0; t < NMON; ++t) { dmc[t] = 0.0f; dmx[t] = 0.0f; }
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
-      float pk = __expf(-e2k[k] * r2) * (fcp - 2.0f * e2k[k] * r * fc) * ud;
-      dgc[k] += cj ? pk : 0.0f;
-      dgx[k] += cj ? 0.0f : pk;
-    }
-  SUR_WALK_END
+    for (int k = 0; k < 6; ++k) { dgc[k] = 0.0f; dgx[k] = 0.0f; }
+    SUR_WALK_BEGIN(float4, SUR_RES)
+      float dx, dy, dz;
+      float r2 = sur_dr_rec<R>(Gm, pi, pj, u_ == 0, dx, dy, dz);
+      if (!(r2 < K.rc2)) continue;
+      const TangentTerms T(K, dx, dy, dz, r2, eta, (mj & K.bit1) != 0, ri, aj);
+      float mono[NMON], dmono[NMON];
+      T.monomials(mono, dmono);
+      const float wc = T.carbon(), wx = T.other(wc), dwc = T.dcarbon(), dwx = T.dother(dwc);
+#pragma unroll
+      for (int t = 0; t < NMON; ++t) {
+        dmc[t] += fmaf(dwc, mono[t], wc * dmono[t]);
+        dmx[t] += fmaf(dwx, mono[t], wx * dmono[t]);
+      }
+      ddd[0] = fmaf(2.0f * wc, T.wp * T.ud, ddd[0]);
+#pragma unroll
+      for (int k = 0; k < 6; ++k) {
+        const float pk = T.radial(K.eta2[6 * ke + k], r2);
+        dgc[k] += T.cj ? pk : 0.0f;
+        dgx[k] += T.cj ? 0.0f : pk;
+      }
+    SUR_WALK_END
+    sum_groups<NMON>(dmc);
+    sum_groups<NMON>(dmx);
+    sum_groups<1>(ddd);
+    sum_groups<6>(dgc);
+    sum_groups<6>(dgx);
+  } else {
+    const bool metal = (q & 8) != 0, high = (q & 16) != 0;
+    float m[NMON], g[3] = {0.0f, 0.0f, 0.0f}, e2[3];
+#pragma unroll
+    for (int t = 0; t < NMON; ++t) m[t] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) e2[k] = K.eta2[6 * ke + (high ? 3 + k : k)];
+    SUR_WALK_BEGIN(float4, SUR_RES)
+      float dx, dy, dz;
+      float r2 = sur_dr_rec<R>(Gm, pi, pj, u_ == 0, dx, dy, dz);
+      if (!(r2 < K.rc2)) continue;
+      const TangentTerms T(K, dx, dy, dz, r2, eta, (mj & K.bit1) != 0, ri, aj);
+      float mono[NMON], dmono[NMON];
+      T.monomials(mono, dmono);
+      const float wc = T.carbon(), dwc = T.dcarbon();
+      const float ws = metal ? T.other(wc) : wc, dws = metal ? T.dother(dwc) : dwc;
+#pragma unroll
+      for (int t = 0; t < NMON; ++t) m[t] += fmaf(dws, mono[t], ws * dmono[t]);
+      ddd[0] = fmaf(2.0f * wc, T.wp * T.ud, ddd[0]);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) g[k] += T.cj != metal ? T.radial(e2[k], r2) : 0.0f;
+    SUR_WALK_END
+    sum_groups<NMON>(m);
+    sum_groups<1>(ddd);
+    sum_groups<3>(g);
+    both_species(m, g, metal, high, dmc, dmx, dgc, dgx);
+  }
 #undef SUR_RES
-  sum_groups<NMON>(dmc);
-  sum_groups<NMON>(dmx);
-  sum_groups<1>(ddd);
-  sum_groups<6>(dgc);
-  sum_groups<6>(dgx);
-  if (eg != 0) return;
+  if (q >= 2) return;
   float* dGr = K.dG + (size_t)row * NF;
 #pragma unroll
   for (int k = 0; k < 6; ++k) { dGr[6 * ke + k] = dgc[k]; dGr[12 + 6 * ke + k] = dgx[k]; }
@@ -854,6 +1058,18 @@ __global__ void __launch_bounds__(256) k_sur_tangent(RowArgsS a, SurK K, const u
   g5_of(Scx, o);
 #pragma unroll
   for (int m = 0; m < 4; ++m) dGr[32 + ke * 4 + m] = o[m];
+}
+
+template <class R>
+__global__ void __launch_bounds__(256) k_sur_tangent(RowArgsS a, SurK K, const uint32_t* __restrict__ mask,
+                                                     SurSplit S) {
+  const int t = (int)blockIdx.x - ((S.nmain + 7) & ~7);
+  if (t >= 0) {
+    sur_tangent_rows<R, SUR_LW>(a, K, mask, S.nmain * (256 / SUR_L) + t * (256 / SUR_LW));
+  } else {
+    const int lb = sur_main_block(S);
+    if (lb >= 0) sur_tangent_rows<R, SUR_L>(a, K, mask, lb * (256 / SUR_L));
+  }
 }
 
 // E = sum_i E_i, the loss terms and the seeds of the weight gradient:
@@ -1202,6 +1418,23 @@ void launch_sur_converse(pfm_ctx* h, Inter& it, int step) {
   PFM_LAUNCH(h, "list_conv", k_sur_clip, (L1.nrows + 255) / 256, 256, L1.nrows, L1.nnum, L1.nmax);
 }
 
+// The row passes hold three workgroups of 32 rows on a CU.  What full rounds
+// of those leave over would occupy a few CUs for a workgroup's whole time
+// (24,960 rows, 780 workgroups on 768 places: 94.5 us of k_sur_fused, about 35
+// of them for the last twelve), and few rows alone would leave most of the
+// card idle (1,560 rows, 49 workgroups: fused 41, back 20, descriptors 17.8,
+// tangent 28 us).  Where at most one round of workgroups of 8 rows is left,
+// they take it: 79.6 us, and 29, 11.5, 14.1 and 23.2.  More rows than that
+// keep 8 lanes each (6,240 rows, one round and 12 workgroups of the wide kind:
+// about 50 us against 40).
+static SurSplit sur_split(pfm_ctx* h, int nrows) {
+  constexpr int RB = 256 / SUR_L, RW = 256 / SUR_LW;
+  const int places = std::max(8, 3 * h->cus / 8 * 8);
+  const int full = nrows / (RB * places) * places, rest = nrows - full * RB;
+  if (rest <= RW * places) return SurSplit{full, (rest + RW - 1) / RW};
+  return SurSplit{(nrows + RB - 1) / RB, 0};
+}
+
 // keep (the training passes read the moments, descriptors and dE/dG) or
 // pfm_set_fusion(h, 0): three kernels; else the fused kernel
 template <class R>
@@ -1209,14 +1442,14 @@ static void sur_forces_T(pfm_ctx* h, Inter& it, int accumulate, double4* frc, bo
   SurK K = sur_k(h, it);
   RowArgsS a = sur_rows(h, it.nl[0]);
   if (a.nrows > 0) {
-    int nb = (int)(((long)a.nrows * SUR_L + 255) / 256);
+    const SurSplit S = sur_split(h, a.nrows);
     if (keep || !h->fuse) {
-      PFM_LAUNCH(h, "sur_desc", k_sur_desc<R>, pad8(nb), 256, a, K, h->mask, nb);
+      PFM_LAUNCH(h, "sur_desc", k_sur_desc<R>, S.grid(), 256, a, K, h->mask, S);
       int ng = (a.nrows + 15) / 16;
       PFM_LAUNCH(h, "sur_mlp", k_sur_mlp, (ng + 3) / 4, 256, a.nrows, K);
-      PFM_LAUNCH(h, "sur_back", k_sur_back<R>, pad8(nb), 256, a, K, h->mask, nb);
+      PFM_LAUNCH(h, "sur_back", k_sur_back<R>, S.grid(), 256, a, K, h->mask, S);
     } else {
-      PFM_LAUNCH(h, "sur_fused", k_sur_fused<R>, pad8(nb), 256, a, K, h->mask, nb);
+      PFM_LAUNCH(h, "sur_fused", k_sur_fused<R>, S.grid(), 256, a, K, h->mask, S);
     }
   }
   RowArgsS c = sur_rows(h, it.nl[1]);
@@ -1300,9 +1533,9 @@ int pfm_sur_descriptors(pfm_ctx* h, int inter, double* G) {
   SurK K = sur_k(h, it);
   RowArgsS a = sur_rows(h, L);
   if (a.nrows == 0) return PFM_OK;
-  int nb = (int)(((long)a.nrows * SUR_L + 255) / 256);
-  if (h->precision == PFM_MIXED) PFM_LAUNCH(h, "sur_desc", k_sur_desc<float>, pad8(nb), 256, a, K, h->mask, nb);
-  else PFM_LAUNCH(h, "sur_desc", k_sur_desc<double>, pad8(nb), 256, a, K, h->mask, nb);
+  const SurSplit S = sur_split(h, a.nrows);
+  if (h->precision == PFM_MIXED) PFM_LAUNCH(h, "sur_desc", k_sur_desc<float>, S.grid(), 256, a, K, h->mask, S);
+  else PFM_LAUNCH(h, "sur_desc", k_sur_desc<double>, S.grid(), 256, a, K, h->mask, S);
   std::vector<float> g((size_t)a.nrows * NF);
   std::vector<int> rows(a.nrows), o(h->N);
   HIPCHK(h, hipMemcpyAsync(g.data(), it.sur->G, g.size() * 4, hipMemcpyDeviceToHost, h->stream));
@@ -1339,9 +1572,9 @@ int pfm_sur_loss_grad(pfm_ctx* h, int inter, const double* f_ref, double e_ref, 
   SurK K = sur_k(h, it);
   RowArgsS a = sur_rows(h, it.nl[0]);
   if (nrows > 0) {
-    int nb = (int)(((long)nrows * SUR_L + 255) / 256);
-    if (h->precision == PFM_MIXED) PFM_LAUNCH(h, "sur_tangent", k_sur_tangent<float>, pad8(nb), 256, a, K, h->mask, nb);
-    else PFM_LAUNCH(h, "sur_tangent", k_sur_tangent<double>, pad8(nb), 256, a, K, h->mask, nb);
+    const SurSplit S = sur_split(h, nrows);
+    if (h->precision == PFM_MIXED) PFM_LAUNCH(h, "sur_tangent", k_sur_tangent<float>, S.grid(), 256, a, K, h->mask, S);
+    else PFM_LAUNCH(h, "sur_tangent", k_sur_tangent<double>, S.grid(), 256, a, K, h->mask, S);
   }
   PFM_LAUNCH(h, "sur_loss", k_sur_loss, 1, 256, nrows, it.e_row, nrp, B.rpart, e_ref, w_e, w_f,
              h->grp.n[it.nl[0].g2], B.scal);
