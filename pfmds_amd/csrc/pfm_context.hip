@@ -256,15 +256,31 @@ __global__ void __launch_bounds__(RED_THREADS) k_reduce_rows(int nq, int nb, con
   }
 }
 
-// zero_momentum: v -= sum(m v)/sum(m) over the group (md_general.f90:236-253)
-__global__ void k_sub_mcv(int N, double4* __restrict__ vel, const uint32_t* __restrict__ mask, uint32_t bit,
-                          const double* __restrict__ sums) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= N || !(mask[i] & bit)) return;
-  double tm = sums[3];
-  double4 v = vel[i];
-  v.x -= sums[0] / tm; v.y -= sums[1] / tm; v.z -= sums[2] / tm;
-  vel[i] = v;
+// zero_momentum: v -= sum(m v)/sum(m) over the group (md_general.f90:236-253);
+// every block adds the nb partials of k_mom_part up for itself, in the order of
+// reduce_part.  Grid-stride, so that the blocks stay few beside the atoms
+// (6,164 atoms: 5.1 us, 4.0 + 2.6 with the sums in a launch of their own).
+__global__ void __launch_bounds__(RED_THREADS) k_sub_mcv(int N, double4* __restrict__ vel,
+                                                         const uint32_t* __restrict__ mask, uint32_t bit,
+                                                         const double* __restrict__ part, int nb) {
+  __shared__ double sh[2 * RED_THREADS];
+  __shared__ double sums[4];
+  CSum a[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+  for (int b = threadIdx.x; b < nb; b += RED_THREADS)
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      a[q].add(CSum{part[(size_t)(2 * q) * nb + b], part[(size_t)(2 * q + 1) * nb + b]});
+  block_csum_n<4>(a, sh);
+  if (threadIdx.x == 0)
+    for (int q = 0; q < 4; ++q) sums[q] = a[q].value();
+  __syncthreads();
+  const double tm = sums[3], mx = sums[0] / tm, my = sums[1] / tm, mz = sums[2] / tm;
+  for (int i = blockIdx.x * RED_THREADS + threadIdx.x; i < N; i += gridDim.x * RED_THREADS) {
+    if (!(mask[i] & bit)) continue;
+    double4 v = vel[i];
+    v.x -= mx; v.y -= my; v.z -= mz;
+    vel[i] = v;
+  }
 }
 
 // ------------------------------------------------------------- records
@@ -1544,8 +1560,7 @@ static int zero_momentum(pfm_ctx* h) {
     return PFM_OK;
   }
   PFM_LAUNCH(h, "zero_momentum", k_mom_part, nb, RED_THREADS, h->N, h->vel4, h->mask, bit, h->red_part);
-  PFM_LAUNCH(h, "zero_momentum", k_reduce_rows, 1, RED_THREADS, 4, nb, h->red_part, h->red_out);
-  PFM_LAUNCH(h, "zero_momentum", k_sub_mcv, (h->N + 255) / 256, 256, h->N, h->vel4, h->mask, bit, h->red_out);
+  PFM_LAUNCH(h, "zero_momentum", k_sub_mcv, nb, RED_THREADS, h->N, h->vel4, h->mask, bit, h->red_part, nb);
   return PFM_OK;
 }
 

@@ -157,6 +157,86 @@ __global__ void k_scatter(int N, const int* __restrict__ atom_rank, const int* _
   if (valid) perm[cell_start[r] + slot] = i;
 }
 
+// k_cell_keys, the scan of the counts and k_scatter in one workgroup, the
+// counts in LDS: up to BIN_N atoms, whose ranks stay in registers, and BIN_C
+// cells.  Three launches of 2.6 to 3.2 us each took longer than one workgroup
+// takes for it all (6,312 atoms 7.2 us, 4,000 5.4, 500 3.6; 9.2, 8.4 and 8 in three).
+#define BIN_N 8192
+#define BIN_C 4096
+__global__ void __launch_bounds__(1024) k_bin_small(int N, int ncell, const double4* __restrict__ pos,
+                                                    const int* __restrict__ rep, const RepDev* __restrict__ rdev,
+                                                    const int* __restrict__ cell_rank, int* __restrict__ cell_start,
+                                                    int* __restrict__ cell_tmp, int* __restrict__ perm) {
+  __shared__ int cnt[BIN_C];
+  __shared__ int wsum[16];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  for (int c = t; c < ncell; c += 1024) cnt[c] = 0;
+  // each phase for all of a thread's atoms at once (those past the end repeat
+  // the last one): loads of one wait beside those of the others
+  constexpr int U = BIN_N / 1024;
+  int rank[U], slot[U];
+  double4 p[U];
+#pragma unroll
+  for (int u = 0; u < U && u * 1024 < N; ++u) p[u] = pos[min(u * 1024 + t, N - 1)];
+  auto cell_of = [](const double4& x, const RepDev& R) {
+    const int cx = cell_coord(x.x, R.inv_clen.x, R.nc[0]);
+    const int cy = cell_coord(x.y, R.inv_clen.y, R.nc[1]);
+    const int cz = cell_coord(x.z, R.inv_clen.z, R.nc[2]);
+    return R.cell_base + (cz * R.nc[1] + cy) * R.nc[0] + cx;
+  };
+  if (rep) {
+#pragma unroll
+    for (int u = 0; u < U && u * 1024 < N; ++u) rank[u] = rep[min(u * 1024 + t, N - 1)];
+#pragma unroll
+    for (int u = 0; u < U && u * 1024 < N; ++u) rank[u] = cell_of(p[u], rdev[rank[u]]);
+  } else {
+#pragma unroll
+    for (int u = 0; u < U && u * 1024 < N; ++u) rank[u] = cell_of(p[u], rdev[0]);
+  }
+#pragma unroll
+  for (int u = 0; u < U && u * 1024 < N; ++u) rank[u] = cell_rank[rank[u]];
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (u * 1024 >= N) break;
+    const bool valid = u * 1024 + t < N;
+    slot[u] = run_atomic_inc(cnt, valid ? rank[u] : -1, valid);
+  }
+  __syncthreads();
+  // exclusive scan: BIN_C / 1024 consecutive cells a thread
+  int x[BIN_C / 1024], sum = 0;
+#pragma unroll
+  for (int k = 0; k < BIN_C / 1024; ++k) {
+    const int c = t * (BIN_C / 1024) + k;
+    x[k] = c < ncell ? cnt[c] : 0;
+    sum += x[k];
+  }
+  int inc = sum;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(inc, o);
+    if (lane >= o) inc += v;
+  }
+  if (lane == 63) wsum[w] = inc;
+  __syncthreads();
+  int run = inc - sum;
+  for (int k = 0; k < w; ++k) run += wsum[k];
+#pragma unroll
+  for (int k = 0; k < BIN_C / 1024; ++k) {
+    const int c = t * (BIN_C / 1024) + k;
+    if (c < ncell) {
+      cell_start[c] = run;
+      cell_tmp[c] = x[k];
+      cnt[c] = run;
+    }
+    run += x[k];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (u * 1024 + t < N) perm[cnt[rank[u]] + slot[u]] = u * 1024 + t;
+}
+
 // the per-atom arrays in their current order (0) and in cell order (1)
 struct PermArgs {
   const double4 *p0, *v0, *f0;
@@ -196,9 +276,15 @@ __global__ void __launch_bounds__(64) k_cell_sort(int ncell, const int* __restri
   for (int k = threadIdx.x; k < n; k += 64) {
     int v = perm_in[s + k];
     g |= mask[v];
-    int kk = lds ? key[k] : orig[v];
     int rank = 0;
-    for (int m = 0; m < n; ++m) rank += ((lds ? key[m] : orig[perm_in[s + m]]) < kk) ? 1 : 0;
+    if (lds) {
+      const int kk = key[k];
+#pragma unroll 8
+      for (int m = 0; m < n; ++m) rank += key[m] < kk ? 1 : 0;
+    } else {
+      const int kk = orig[v];
+      for (int m = 0; m < n; ++m) rank += orig[perm_in[s + m]] < kk ? 1 : 0;
+    }
     if constexpr (PERM) {
       const int d = s + rank;
       const double4 p = P.p0[v];
@@ -230,10 +316,15 @@ __global__ void __launch_bounds__(64) k_cell_sort(int ncell, const int* __restri
 int launch_sort_and_bin(pfm_ctx* h, int step, bool permute) {
   (void)step;
   int N = h->N, nb = (N + 255) / 256;
-  PFM_LAUNCH(h, "cell_keys", k_cell_keys, nb, 256, N, h->pos4, h->rep, h->rdev, h->cell_rank, h->atom_rank,
-             h->cell_tmp);
-  scan_excl(h, h->ncell, h->cell_tmp, h->cell_start, h->scan_tmp);
-  PFM_LAUNCH(h, "scatter", k_scatter, nb, 256, N, h->atom_rank, h->cell_start, h->cell_fill, h->scan_tmp + N);
+  if (N <= BIN_N && h->ncell <= BIN_C) {
+    PFM_LAUNCH(h, "cell_keys", k_bin_small, 1, 1024, N, h->ncell, h->pos4, h->rep, h->rdev, h->cell_rank,
+               h->cell_start, h->cell_tmp, h->scan_tmp + N);
+  } else {
+    PFM_LAUNCH(h, "cell_keys", k_cell_keys, nb, 256, N, h->pos4, h->rep, h->rdev, h->cell_rank, h->atom_rank,
+               h->cell_tmp);
+    scan_excl(h, h->ncell, h->cell_tmp, h->cell_start, h->scan_tmp);
+    PFM_LAUNCH(h, "scatter", k_scatter, nb, 256, N, h->atom_rank, h->cell_start, h->cell_fill, h->scan_tmp + N);
+  }
   PermArgs P{h->pos4, h->vel4, h->frc4, h->mask, h->orig, h->rep, h->pos4b, h->vel4b, h->frc4b, h->maskb,
              h->origb, h->repb, h->qpos, h->rdev};
   if (!permute) {
@@ -259,7 +350,8 @@ int launch_sort_and_bin(pfm_ctx* h, int step, bool permute) {
 
 // --------------------------------------------------------------- group rows
 //
-// The rows of up to GR_MAX groups in three launches whatever their number:
+// The rows of up to GR_MAX groups in three launches (one on few atoms,
+// k_grp_rows_small) whatever their number:
 // per 256-atom block and group the member count (wave ballots), one
 // workgroup per group scanning its block counts, then every member's row
 // from its block's offset, its wave's offset and its rank in the wave.  Rows
@@ -319,6 +411,57 @@ __global__ void __launch_bounds__(256) k_grp_write(int N, const uint32_t* __rest
   }
 }
 
+// k_grp_count, k_grp_scan and k_grp_write in one launch: every block counts
+// the members in the masks before it for itself, which up to GR_SMALL blocks
+// costs less than two launches (6,312 atoms 4.8 us against 3.4 + 3.2 + 4.3)
+#define GR_SMALL 32
+__global__ void __launch_bounds__(256) k_grp_rows_small(int N, const uint32_t* __restrict__ mask, GroupRowsArgs G) {
+  __shared__ int wc[GR_MAX][4], before[GR_MAX][4];
+  const int i = blockIdx.x * 256 + threadIdx.x, w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const uint32_t m = i < N ? mask[i] : 0u;
+  int cnt[GR_MAX];
+#pragma unroll
+  for (int q = 0; q < GR_MAX; ++q) cnt[q] = 0;
+  for (int b0 = 0; b0 < (int)blockIdx.x; b0 += 8) {
+    uint32_t mb[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const uint32_t x = mask[min(b0 + u, (int)blockIdx.x - 1) * 256 + threadIdx.x];
+      mb[u] = b0 + u < (int)blockIdx.x ? x : 0u;
+    }
+#pragma unroll
+    for (int q = 0; q < GR_MAX; ++q) {
+      if (q >= G.ng) break;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) cnt[q] += __popcll(__ballot((mb[u] & G.bit[q]) != 0));
+    }
+  }
+  unsigned long long bal[GR_MAX];
+#pragma unroll
+  for (int q = 0; q < GR_MAX; ++q) {
+    if (q >= G.ng) break;
+    bal[q] = __ballot((m & G.bit[q]) != 0);
+    if (lane == 0) {
+      wc[q][w] = __popcll(bal[q]);
+      before[q][w] = cnt[q];
+    }
+  }
+  __syncthreads();
+  if (i >= N) return;
+  const unsigned long long below = (1ull << lane) - 1ull;
+#pragma unroll
+  for (int q = 0; q < GR_MAX; ++q) {
+    if (q >= G.ng) break;
+    int r = -1;
+    if (m & G.bit[q]) {
+      r = __popcll(bal[q] & below);
+      for (int v = 0; v < 4; ++v) r += before[q][v] + (v < w ? wc[q][v] : 0);
+      G.rows[q][r] = i;
+    }
+    G.row_of[q][i] = r;
+  }
+}
+
 __global__ void k_identity_rows(int N, int* __restrict__ rows, int* __restrict__ row_of) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < N) { rows[i] = i; row_of[i] = i; }
@@ -331,6 +474,11 @@ void launch_group_rows(pfm_ctx* h) {
   G.nb = nb;
   auto flush = [&]() {
     if (!G.ng) return;
+    if (nb <= GR_SMALL) {
+      PFM_LAUNCH(h, "group_rows", k_grp_rows_small, nb, 256, N, h->mask, G);
+      G.ng = 0;
+      return;
+    }
     int* cnt = h->scan_tmp;
     int* off = h->scan_tmp + (size_t)GR_MAX * nb;
     PFM_LAUNCH(h, "group_rows", k_grp_count, nb, 256, N, h->mask, G, cnt);
@@ -400,76 +548,87 @@ struct SearchArgs {
 };
 
 // slot of the row atom inside each neighbour's own row (Tersoff-Brenner's
-// `do l=1,nl%nnum(j); if(nl%nlist(l,j)==i) exit` and graphene's l1 search)
-__global__ void k_rev(int nrows, const int* __restrict__ rows, const int* __restrict__ row_of,
-                      const int* __restrict__ nnum, const int* __restrict__ nbr, int stride, int* __restrict__ rev,
-                      DevErr* err, const int* __restrict__ orig, int step) {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
+// `do l=1,nl%nnum(j); if(nl%nlist(l,j)==i) exit` and graphene's l1 search);
+// REV_T lanes a row, an entry each (bound by the chain of dependent loads of
+// one entry: 3.9 us at 1,664 rows, 6.3 with one lane taking them in turn)
+#define REV_T 4
+__global__ void __launch_bounds__(256) k_rev(int nrows, const int* __restrict__ rows, const int* __restrict__ row_of,
+                                             const int* __restrict__ nnum, const int* __restrict__ nbr, int stride,
+                                             int* __restrict__ rev, DevErr* err, const int* __restrict__ orig,
+                                             int step) {
+  const int gt = blockIdx.x * 256 + threadIdx.x, r = gt / REV_T;
   if (r >= nrows) return;
-  int i = rows[r], n = nnum[r];
-  for (int p = 0; p < n; ++p) {
-    int j = nbr[(size_t)r * stride + p];
-    int jr = row_of[j];
+  const int i = rows[r], n = nnum[r];
+  for (int p = gt & (REV_T - 1); p < n; p += REV_T) {
+    const int jr = row_of[nbr[(size_t)r * stride + p]];
     int l = -1;
     if (jr >= 0) {
-      int nj = nnum[jr];
-      for (int q = 0; q < nj; ++q)
-        if (nbr[(size_t)jr * stride + q] == i) { l = q; break; }
+      const int nj = nnum[jr];
+      const int* row = nbr + (size_t)jr * stride;
+#pragma unroll 4
+      for (int q = nj - 1; q >= 0; --q) l = row[q] == i ? q : l;  // the first match, without leaving early
     }
     rev[(size_t)r * stride + p] = l;
     if (l < 0) raise_err(err, PFM_E_GRAPHENE_NN, orig[i] + 1, -1, step);
   }
 }
 
-// lj1g: every atom's group-local index (the group of the list's second side)
-__global__ void k_lj1g_loc(int N, const int* __restrict__ orig, const int* __restrict__ loc, int2* __restrict__ lc) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < N) lc[i].x = loc[orig[i]];
-}
-
-// lj1g: group-local index of the first listed neighbour whose atom index is
-// larger than the row atom's (the reference's lessnnum boundary, in list
-// order = ascending group order); T lanes per row, the minimum over the
-// row's entries
+// lj1g: every row atom's group-local index, and that of the first listed
+// neighbour whose atom index is larger than the row atom's (the reference's
+// lessnnum boundary, in list order = ascending group order); T lanes per row,
+// the minimum over the row's entries
 template <int T>
 __global__ void __launch_bounds__(256) k_lj1g_cut(int nrows, const int* __restrict__ rows,
                                                   const int* __restrict__ nnum, const int* __restrict__ nbr, int stride,
-                                                  const int* __restrict__ orig, int2* __restrict__ lc) {
+                                                  const int* __restrict__ orig, const int* __restrict__ loc,
+                                                  int2* __restrict__ lc) {
   int gt = blockIdx.x * blockDim.x + threadIdx.x;
   int r = gt / T, t = threadIdx.x & (T - 1);
   if (r >= nrows) return;
   int i = rows[r], oi = orig[i], n = nnum[r], c = 0x7fffffff;
+#pragma unroll 4
   for (int p = t; p < n; p += T) {
-    int j = nbr[(size_t)r * stride + p];
-    if (orig[j] > oi) { int l = lc[j].x; c = l < c ? l : c; }
+    const int oj = orig[nbr[(size_t)r * stride + p]];
+    const int l = loc[oj];
+    c = oj > oi && l < c ? l : c;
   }
 #pragma unroll
   for (int o = T / 2; o > 0; o >>= 1) {
     int v = __shfl_xor(c, o, T);
     c = v < c ? v : c;
   }
-  if (t == 0) lc[i].y = c;
+  if (t == 0) lc[i] = make_int2(loc[oi], c);
 }
 
 // ljc/morsec metal rows (nl(2)) that have entries, appended in any order
 // (each row's force is summed on its own, so the order of the work list does
 // not change any result); the count goes after the rows.  One atomic per
 // 1024-thread workgroup: wave ballots, then the wave counts' prefix in LDS.
+// ONE: a single workgroup takes all the rows in turn and writes the count,
+// which needs no clearing launch before it.
+template <bool ONE>
 __global__ void __launch_bounds__(1024) k_mark_rows(int nrows, const int* __restrict__ nnum, int* __restrict__ mrows) {
   __shared__ int wc[17];
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  const bool keep = r < nrows && nnum[r] > 0;
-  const unsigned long long bal = __ballot(keep);
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  if (lane == 0) wc[w] = __popcll(bal);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int tot = 0;
-    for (int q = 0; q < nw; ++q) { const int c = wc[q]; wc[q] = tot; tot += c; }
-    wc[16] = tot ? atomicAdd(&mrows[nrows], tot) : 0;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int base = 0;
+  for (int r0 = ONE ? 0 : blockIdx.x * 1024; r0 < nrows; r0 += ONE ? 1024 : nrows) {
+    const int r = r0 + threadIdx.x;
+    const bool keep = r < nrows && nnum[r] > 0;
+    const unsigned long long bal = __ballot(keep);
+    if (lane == 0) wc[w] = __popcll(bal);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int tot = 0;
+      for (int q = 0; q < 16; ++q) { const int c = wc[q]; wc[q] = tot; tot += c; }
+      wc[16] = ONE ? tot : (tot ? atomicAdd(&mrows[nrows], tot) : 0);
+    }
+    __syncthreads();
+    const int at = ONE ? base : wc[16];
+    if (keep) mrows[at + wc[w] + __popcll(bal & ((1ull << lane) - 1ull))] = r;
+    if (ONE) base += wc[16];
+    __syncthreads();
   }
-  __syncthreads();
-  if (keep) mrows[wc[16] + wc[w] + __popcll(bal & ((1ull << lane) - 1ull))] = r;
+  if (ONE && threadIdx.x == 0) mrows[nrows] = base;
 }
 
 // lj1g: each entry's weight in the gather, [loc(j) < cut(i)] (the pair is in
@@ -1127,6 +1286,12 @@ static SearchArgs search_args(pfm_ctx* h, int ii, int k, int step) {
   return a;
 }
 
+static int rev_blocks(int nrows) { return (int)(((long)nrows * REV_T + 255) / 256); }
+
+// one workgroup marks this many rows faster than a clearing launch and the
+// blocks of 1,024 (4,648 rows: 4.5 us against 4.5 + 3.6)
+#define MARK_ONE 8192
+
 // what follows a list's search: tb reverse slots, the ljc/morsec metal work
 // list, lj1g half-list tags
 static void list_post(pfm_ctx* h, int ii, int k, int step) {
@@ -1136,19 +1301,21 @@ static void list_post(pfm_ctx* h, int ii, int k, int step) {
     L.built = true;
     return;
   }
-  int nb = (L.nrows + 255) / 256;
   if (it.kind == PFM_TB || it.kind == PFM_REBOSC || (k == 2 && !(int)it.p[it.kind == PFM_LJC ? 5 : 6])) {
-    PFM_LAUNCH(h, "list_rev", k_rev, nb, 256, L.nrows, h->grp.rows[L.g1], h->grp.row_of[L.g1], L.nnum, L.nbr,
+    PFM_LAUNCH(h, "list_rev", k_rev, rev_blocks(L.nrows), 256, L.nrows, h->grp.rows[L.g1], h->grp.row_of[L.g1], L.nnum, L.nbr,
                L.stride, L.rev, h->derr, h->orig, step - h->step_base);
   }
   if ((it.kind == PFM_LJC || it.kind == PFM_MORSEC) && k == 1) {
-    PFM_LAUNCH(h, "list_rows", k_fill_int, 1, 64, 1, it.mrows + L.nrows, 0);
-    PFM_LAUNCH(h, "list_rows", k_mark_rows, (L.nrows + 1023) / 1024, 1024, L.nrows, L.nnum, it.mrows);
+    if (L.nrows <= MARK_ONE) {
+      PFM_LAUNCH(h, "list_rows", k_mark_rows<true>, 1, 1024, L.nrows, L.nnum, it.mrows);
+    } else {
+      PFM_LAUNCH(h, "list_rows", k_fill_int, 1, 64, 1, it.mrows + L.nrows, 0);
+      PFM_LAUNCH(h, "list_rows", k_mark_rows<false>, (L.nrows + 1023) / 1024, 1024, L.nrows, L.nnum, it.mrows);
+    }
   }
   if (it.kind == PFM_LJ1G) {
-    PFM_LAUNCH(h, "list_cut", k_lj1g_loc, (h->N + 255) / 256, 256, h->N, h->orig, h->grp.loc[L.g2], it.lc);
     PFM_LAUNCH(h, "list_cut", k_lj1g_cut<8>, (int)(((long)L.nrows * 8 + 255) / 256), 256, L.nrows, h->grp.rows[L.g1],
-               L.nnum, L.nbr, L.stride, h->orig, it.lc);
+               L.nnum, L.nbr, L.stride, h->orig, h->grp.loc[L.g2], it.lc);
     PFM_LAUNCH(h, "list_cut", k_lj1g_tag, (int)(((long)L.nrows * 8 + 255) / 256), 256, L.nrows, h->grp.rows[L.g1],
                L.nnum, L.nbr, L.stride, it.lc);
   }
@@ -1225,12 +1392,12 @@ int launch_nn_from_tb(pfm_ctx* h, int ii, int step) {
   ListDev& L = it.nl[2];
   ListDev& T = tb.nl[0];
   if (L.nrows == 0) return PFM_OK;
-  int nb = (L.nrows + 255) / 256;
+  const int nb = (L.nrows + 255) / 256;
   PFM_LAUNCH(h, "nn_from_tb", k_nn_from_tb, nb, 256, L.nrows, h->grp.rows[L.g1], T.nnum, T.nbr, T.stride, h->pos4,
              h->rep, h->rdev, L.rcut, L.nnum, L.nbr, h->derr, h->orig, step - h->step_base);
   bool simplified = (int)it.p[it.kind == PFM_LJC ? 5 : 6];
   if (!simplified)
-    PFM_LAUNCH(h, "list_rev", k_rev, nb, 256, L.nrows, h->grp.rows[L.g1], h->grp.row_of[L.g1], L.nnum, L.nbr,
+    PFM_LAUNCH(h, "list_rev", k_rev, rev_blocks(L.nrows), 256, L.nrows, h->grp.rows[L.g1], h->grp.row_of[L.g1], L.nnum, L.nbr,
                L.stride, L.rev, h->derr, h->orig, step - h->step_base);
   L.built = true;
   return PFM_OK;
