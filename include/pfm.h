@@ -203,8 +203,10 @@ int pfm_set_timing(pfm_ctx* h, int on);
 int pfm_kernel_time(pfm_ctx* h, const char* name, int* count, double* mean_ms);
 
 /* Shape of the pair passes: lanes per atom row (1,2,4,8,16,32) and
- * workgroup size (64..1024); 0 keeps the current value.  No counterpart in
- * the reference (launch-shape control for tuning and benchmarks). */
+ * workgroup size (64..1024); 0 keeps the current value.  A handle starts
+ * with 8 lanes (16 up to 15,000 atoms in FP64 and 8,192 in the mixed path)
+ * and 256.  No counterpart in the reference (launch-shape control for tuning
+ * and benchmarks). */
 int pfm_set_tuning(pfm_ctx* h, int lanes_per_row, int block);
 
 /* Co-scheduled passes (default on).  For graphene on a metal -- exactly

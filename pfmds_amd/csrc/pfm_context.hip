@@ -831,6 +831,17 @@ static int growth_setup(pfm_ctx* h) {
 }
 
 // Allocate lists, cells and reductions once all interactions are known.
+// Lanes that share one list row until pfm_set_tuning says otherwise.  With 8,
+// a few thousand rows do not give every SIMD a wavefront and a step waits for
+// each lane's serial share of its row; 16 halve that share, until the card is
+// full and their longer sums cost more (us a step with 8 and 16 lanes): FP64
+// gas of 2,000 atoms 11.6 and 10.1, 8,000 12.5 and 11.6, 16,000 14.5 and 14.7,
+// 32,000 19.5 and 21.0, crystal of 2,048 21.4 and 16.7, 16,384 26.9 and 25.7,
+// 32,000 37.3 and 37.8, graphene/Cu of 5,088 48.1 and 44.8, 21,040 56.4 and
+// 55.8; mixed gas of 2,000 10.4 and 9.5, 8,000 11.0 and 10.6, 16,000 12.1 and
+// 12.5, crystal of 6,912 16.1 and 15.9, 16,384 18.1 and 18.9.
+static int row_lanes(int n, int precision) { return n <= (precision == PFM_MIXED ? 8192 : 15000) ? 16 : 8; }
+
 static int finalize(pfm_ctx* h) {
   if (h->sorted_once) return PFM_OK;
   int rc;
@@ -1907,6 +1918,7 @@ int pfm_create_batch(pfm_ctx** out, int nrep, const int* n_atoms, const double* 
   int dev = 0;
   HIPCHK(h, hipGetDevice(&dev));
   HIPCHK(h, hipDeviceGetAttribute(&h->cus, hipDeviceAttributeMultiprocessorCount, dev));
+  h->lanes = row_lanes(n, precision);
   h->red_blocks = std::max(1, std::min(1024, (n + RED_THREADS - 1) / RED_THREADS));
   // compensated partial rows: an (s, c) pair per block
   if ((rc = dalloc(h, &h->red_part, (size_t)2 * (PFM_MAXI + 1 + RED_MAXQ) * h->red_blocks))) return rc;

@@ -654,7 +654,7 @@ struct pfm_ctx {
   uint32_t* sp_mask = nullptr;
   int* sp_orig = nullptr;
   // tuning
-  int lanes = 8, block = 256;  // lanes per list row and workgroup size of the pair passes
+  int lanes = 8, block = 256;  // lanes per list row (row_lanes) and workgroup size of the pair passes
   // graphene on a metal (rjl on the metal, tb on the graphene, ljc/morsec
   // between them, no common atom): passes over disjoint atoms share launches
   struct GmPlan {
