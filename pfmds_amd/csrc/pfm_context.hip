@@ -77,104 +77,6 @@ __global__ void k_check(int N, const double4* __restrict__ pos, double bx, doubl
   }
 }
 
-#define RED_THREADS 256
-#define RED_MAXQ 8
-
-struct MaskQ {
-  int nq;
-  uint32_t bit[RED_MAXQ];
-};
-
-// compensated sum of one (s, c) pair per thread over the block, in a fixed
-// order: a butterfly over each wavefront's 64 lanes (cross-lane shuffles, no
-// barrier), then the four wavefront sums in LDS in wavefront order.  Every
-// thread returns the block's pair.  sh holds at least 8 doubles (callers
-// pass 2 * RED_THREADS).
-__device__ __forceinline__ CSum block_csum(CSum v, double* sh) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v.add(CSum{__shfl_xor(v.s, o), __shfl_xor(v.c, o)});
-  const int w = threadIdx.x >> 6, nw = RED_THREADS >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    sh[w] = v.s;
-    sh[nw + w] = v.c;
-  }
-  __syncthreads();
-  CSum r{sh[0], sh[nw]};
-  for (int k = 1; k < nw; ++k) r.add(CSum{sh[k], sh[nw + k]});
-  __syncthreads();
-  return r;
-}
-
-// The same sums of NQ pairs per thread at once: the exchanges of the NQ
-// butterflies overlap and the block meets once instead of NQ times.  Thread 0
-// returns the block's pairs, bit for bit those of block_csum.
-template <int NQ>
-__device__ __forceinline__ void block_csum_n(CSum (&v)[NQ], double* sh) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) v[q].add(CSum{__shfl_xor(v[q].s, o), __shfl_xor(v[q].c, o)});
-  constexpr int nw = RED_THREADS / 64;
-  const int w = threadIdx.x >> 6;
-  __syncthreads();  // sh may still be read by the last call
-  if ((threadIdx.x & 63) == 0) {
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      sh[(q * nw + w) * 2] = v[q].s;
-      sh[(q * nw + w) * 2 + 1] = v[q].c;
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      CSum r{sh[q * nw * 2], sh[q * nw * 2 + 1]};
-      for (int k = 1; k < nw; ++k) r.add(CSum{sh[(q * nw + k) * 2], sh[(q * nw + k) * 2 + 1]});
-      v[q] = r;
-    }
-  }
-}
-
-// Per-block partials of compensated sums: row q of a grid of nb blocks keeps
-// the s parts at part[2q nb + b] and the c parts at part[(2q+1) nb + b].
-__device__ __forceinline__ void put_part(double* part, int q, int nb, int b, const CSum& v) {
-  part[(size_t)(2 * q) * nb + b] = v.s;
-  part[(size_t)(2 * q + 1) * nb + b] = v.c;
-}
-// the compensated sum of row q's nb partials, in a fixed order
-__device__ __forceinline__ CSum reduce_part(const double* part, int q, int nb, double* sh) {
-  CSum a{0.0, 0.0};
-  for (int b = threadIdx.x; b < nb; b += RED_THREADS)
-    a.add(CSum{part[(size_t)(2 * q) * nb + b], part[(size_t)(2 * q + 1) * nb + b]});
-  return block_csum(a, sh);
-}
-
-// second half of one atom: kick xyz/z, then for nvms the projections
-// molecular_static_xyz/1D_velocities (md_integrators.f90:99-145).  Returns
-// whether the atom moves.
-// The fused multiply-adds are written out: what the compiler would
-// contract differs between the kernels that call this, and an nvms run has
-// to give the same bits through each of them.
-__device__ __forceinline__ bool kick2_atom(double4& v, const double4& f, double k, uint32_t m, const IntP& P,
-                                           bool nvms) {
-  const bool bx = (m & P.bxyz) != 0, bz = (m & P.bz) != 0;
-  if (!(bx || bz)) return false;
-  if (bx) { v.x = fma(f.x * k, P.ts1, v.x); v.y = fma(f.y * k, P.ts1, v.y); v.z = fma(f.z * k, P.ts1, v.z); }
-  if (bz) v.z = fma(f.z * k, P.ts1, v.z);
-  if (nvms) {
-    if (bx) {
-      const double fv = fma(f.z, v.z, fma(f.x, v.x, f.y * v.y)), ff = fma(f.z, f.z, fma(f.x, f.x, f.y * f.y));
-      if (fv > 0.0 && ff > 1e-12) { double c = fv / ff; v.x = c * f.x; v.y = c * f.y; v.z = c * f.z; }
-      else { v.x = 0; v.y = 0; v.z = 0; }
-    }
-    if (bz) {
-      const double fv = fma(f.z, v.z, fma(f.x, v.x, f.y * v.y));
-      if (!(fv > 0.0)) { v.x = 0; v.y = 0; v.z = 0; }
-    }
-  }
-  return true;
-}
-
 __global__ void k_kick2(int N, double4* __restrict__ vel, const double4* __restrict__ frc,
                         const uint32_t* __restrict__ mask, IntP P, int nvms) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -2107,6 +2009,9 @@ static int run_steps(pfm_ctx* h, int integ, double dt, int s0, int s1, int energ
   h->need_forces = false;
   const bool nvt = integ == PFM_NVT && !h->nhc.empty();
   bool nhc_pending = false;
+  // blocks whose partials hold a step's kinetic energies: the force launch's
+  // where it can form them, else k_kick2_ke's
+  const int ke_nb = nvt ? multi_ke_blocks(h) : 0, ke_parts = ke_nb ? ke_nb : h->red_blocks;
   bool kick_pending = false;  // second half kick deferred into the next kick_drift
   const int CONVERGED = -1;
   // nvms blocks: the steps from spec_base on record their energies and
@@ -2146,7 +2051,7 @@ static int run_steps(pfm_ctx* h, int integ, double dt, int s0, int s1, int energ
         Q.pre_kick = 1;
         PFM_LAUNCH(h, "kick_drift", k_kick_drift<true>, nb, RED_THREADS, N, h->pos4, h->vel4, h->frc4, h->mask, Q,
                    h->derr, h->orig, s - h->step_base, h->qpos, h->qscale, h->rep, h->rdev,
-                   chain_args(h, dt, h->nhc_state0), h->red_part, h->red_blocks);
+                   chain_args(h, dt, h->nhc_state0), h->red_part, ke_parts);
         nhc_pending = false;
       } else if (!drifted) {
         PFM_LAUNCH(h, "kick_drift", k_kick_drift<false>, nb, RED_THREADS, N, h->pos4, h->vel4, h->frc4, h->mask, Q,
@@ -2160,18 +2065,26 @@ static int run_steps(pfm_ctx* h, int integ, double dt, int s0, int s1, int energ
     h->rep_pe_prev = h->rep_pe;
     if ((rc = update_lists(h, s))) return rc;
     if (s % h->zm_period == 0 && (rc = zero_momentum(h))) return rc;
-    if ((rc = launch_forces(h, energy || re, first_writes))) return rc;
+    const bool in_pass = nvt && s != 0 && ke_nb > 0;  // the force launch forms the kinetic energies
+    if (nvt && s != 0) nhc_pending = !report && s < s1;
+    if (in_pass)
+      h->mp_ke = KeArgs{ke_nb, h->vel4, h->mask, P, chain_masks(h), h->red_part, h->nhc_state,
+                     nhc_pending ? h->nhc_state0 : nullptr, (int)(h->nhc.size() * sizeof(NhcDev) / sizeof(double))};
+    rc = launch_forces(h, energy || re, first_writes);
+    h->mp_ke.nb = 0;
+    if (rc) return rc;
     if (s != 0) {
       if (nvt) {
         // second half step; on steps with nothing to report, the next step's
         // first half takes it and both halves of the chain update with it
-        nhc_pending = !report && s < s1;
-        const MaskQ C = chain_masks(h);
-        PFM_LAUNCH(h, "kick2", k_kick2_ke, h->red_blocks, RED_THREADS, N, h->vel4, h->frc4, h->mask, P, C, h->red_part,
-                   (const NhcDev*)h->nhc_state, nhc_pending ? (NhcDev*)h->nhc_state0 : nullptr);
+        if (!in_pass)
+          PFM_LAUNCH(h, "kick2", k_kick2_ke, h->red_blocks, RED_THREADS, N, h->vel4, h->frc4, h->mask, P,
+                     chain_masks(h), h->red_part, (const NhcDev*)h->nhc_state,
+                     nhc_pending ? (NhcDev*)h->nhc_state0 : nullptr);
         if (!nhc_pending) {
-          PFM_LAUNCH(h, "nhc", k_nhc_chain, 1, RED_THREADS, C.nq, chain_args(h, dt, h->nhc_state), h->red_part,
-                     h->red_blocks);
+          if (in_pass) PFM_LAUNCH(h, "kick2", k_kick2, nb, 256, N, h->vel4, h->frc4, h->mask, P, 0);
+          PFM_LAUNCH(h, "nhc", k_nhc_chain, 1, RED_THREADS, (int)h->nhc.size(), chain_args(h, dt, h->nhc_state),
+                     h->red_part, ke_parts);
           PFM_LAUNCH(h, "nhc_scale", k_scale, nb, 256, N, h->vel4, h->mask, P);
         }
       } else if (integ != PFM_NVMS && !report && s < s1) {
@@ -2208,6 +2121,7 @@ static int run_steps(pfm_ctx* h, int integ, double dt, int s0, int s1, int energ
     int rc;
     std::vector<uint64_t> key = graph_key(h, integ, dt, nblk, first_writes, s);
     key.push_back((uint64_t)(spec_on ? h->spec_e : nullptr));
+    key.push_back((uint64_t)ke_nb);
     pfm_ctx::GraphEntry* g = nullptr;
     for (auto& e : h->graphs)
       if (e.key == key) g = &e;

@@ -65,12 +65,13 @@ template <> __device__ __forceinline__ void store_w<float>(const RowArgs& a, int
 }
 
 #define ROW_PROLOGUE(T) ROW_PROLOGUE_AT(T, xcd_block(nb_real))
-#define ROW_PROLOGUE_AT(T, LB)                            \
+#define ROW_PROLOGUE_AT(T, LB) ROW_PROLOGUE_RET(T, LB, )
+#define ROW_PROLOGUE_RET(T, LB, RET)                      \
   int lb = (LB);                                          \
-  if (lb < 0) return;                                     \
+  if (lb < 0) return RET;                                 \
   int gt = lb * blockDim.x + threadIdx.x;                 \
   int row = gt / (T), t = threadIdx.x & ((T)-1);          \
-  if (row >= a.nrows) return;                             \
+  if (row >= a.nrows) return RET;                         \
   int i = a.rows[row];                                    \
   const Geo<R> G = geo_of<R>(a, i);                       \
   const typename Geo<R>::P pi = G.at(i);                  \
@@ -238,6 +239,12 @@ __device__ __forceinline__ void write_force(const RowArgs& a, int i, double fx, 
   f.x += fx; f.y += fy; f.z += fz;
   a.frc[i] = f;
 }
+
+// the force a row's first lane wrote (i < 0: this lane wrote none)
+struct RowForce {
+  int i = -1;
+  double x = 0, y = 0, z = 0;
+};
 
 // ------------------------------------------------------------------- RGL
 
@@ -439,8 +446,8 @@ __device__ __forceinline__ void lj_walk(const LjP& P, const Geo<R>& G, const typ
 
 // (E with a.e_row null: the converse rows nl(2), which carry no energy)
 template <int T, class R, bool E>
-__device__ __forceinline__ void lj_rows(const RowArgs& a, const LjP& P, int blk) {
-  ROW_PROLOGUE_AT(T, blk)
+__device__ __forceinline__ RowForce lj_rows(const RowArgs& a, const LjP& P, int blk) {
+  ROW_PROLOGUE_RET(T, blk, RowForce{})
   RowAcc<R> acc;
   lj_walk<T, R, E>(P, G, pi, nbrow, n, t, i, acc);
   const double fx = group_sum<T>(acc.fx), fy = group_sum<T>(acc.fy), fz = group_sum<T>(acc.fz);
@@ -449,6 +456,7 @@ __device__ __forceinline__ void lj_rows(const RowArgs& a, const LjP& P, int blk)
     write_force(a, i, fx, fy, fz);
     if (E && a.e_row) a.e_row[row] = e;
   }
+  return t == 0 ? RowForce{i, fx, fy, fz} : RowForce{};
 }
 
 template <int T, class R, bool E>
@@ -506,8 +514,8 @@ __device__ __forceinline__ void lj1g_walk(const Lj1gP& P, const Geo<R>& G, const
 }
 
 template <int T, class R, bool E>
-__device__ __forceinline__ void lj1g_rows(const RowArgs& a, const Lj1gP& P, int blk) {
-  ROW_PROLOGUE_AT(T, blk)
+__device__ __forceinline__ RowForce lj1g_rows(const RowArgs& a, const Lj1gP& P, int blk) {
+  ROW_PROLOGUE_RET(T, blk, RowForce{})
   RowAcc<R> acc;
   lj1g_walk<T, R, E>(P, G, pi, nbrow, n, t, i, acc);
   const double fx = group_sum<T>(acc.fx), fy = group_sum<T>(acc.fy), fz = group_sum<T>(acc.fz);
@@ -516,6 +524,7 @@ __device__ __forceinline__ void lj1g_rows(const RowArgs& a, const Lj1gP& P, int 
     write_force(a, i, fx, fy, fz);
     if (E) a.e_row[row] = e;
   }
+  return t == 0 ? RowForce{i, fx, fy, fz} : RowForce{};
 }
 
 // lj1g rows and the lj rows of the same atoms (a species' own pairs, then its
@@ -530,8 +539,8 @@ struct LjRows {
   LjP p;
 };
 template <int T, class R, bool E>
-__device__ __forceinline__ void lj_both_rows(const RowArgs& a, const Lj1gP& P, const LjRows& b, int blk) {
-  ROW_PROLOGUE_AT(T, blk)
+__device__ __forceinline__ RowForce lj_both_rows(const RowArgs& a, const Lj1gP& P, const LjRows& b, int blk) {
+  ROW_PROLOGUE_RET(T, blk, RowForce{})
   const int n2 = b.nnum[row];
   RowAcc<R> acc;
   lj1g_walk<T, R, E>(P, G, pi, nbrow, n, t, i, acc);
@@ -547,6 +556,7 @@ __device__ __forceinline__ void lj_both_rows(const RowArgs& a, const Lj1gP& P, c
       if (b.e_row) b.e_row[row] = el;
     }
   }
+  return t == 0 ? RowForce{i, fx, fy, fz} : RowForce{};
 }
 
 template <int T, class R, bool E>
@@ -1089,7 +1099,30 @@ struct MultiPass {
 struct MultiArgs {
   int n;
   MultiPass s[MULTI_MAXP];
+  KeArgs ke;
 };
+
+// KeArgs: the block's kinetic-energy partials from the forces its rows wrote
+// (a mixed gas of 4,000 atoms: the launch 7.1 us for 5.7, in place of a
+// k_kick2_ke of 3.1 us that reads the forces again)
+__device__ __forceinline__ void ke_parts(const KeArgs& K, const RowForce& f) {
+  __shared__ double sh[2 * RED_THREADS];
+  double ke = 0.0;
+  uint32_t m = 0u;
+  if (f.i >= 0) {
+    m = K.mask[f.i];
+    double4 v = K.vel[f.i];
+    kick2_atom(v, make_double4(f.x, f.y, f.z, 0.0), kick_factor(v.w), m, K.P, false);
+    ke = v.w * (v.x * v.x + v.y * v.y + v.z * v.z) / 2 * PFM_MASS_COEF;
+  }
+#pragma unroll 1
+  for (int q = 0; q < K.Q.nq; ++q) {
+    const CSum s = block_csum(CSum{(m & K.Q.bit[q]) ? ke : 0.0, 0.0}, sh);
+    if (threadIdx.x == 0) put_part(K.part, q, K.nb, blockIdx.x, s);
+  }
+  if (K.C0 && blockIdx.x == 0)
+    for (int j = threadIdx.x; j < K.cw; j += RED_THREADS) K.C0[j] = K.C[j];
+}
 
 template <int T, class R, bool E>
 __global__ void __launch_bounds__(256) k_multi(MultiArgs A) {
@@ -1098,14 +1131,17 @@ __global__ void __launch_bounds__(256) k_multi(MultiArgs A) {
   while (k + 1 < A.n && b >= A.s[k + 1].start) ++k;
   const MultiPass& S = A.s[k];
   const int lb = xcd_local(b - S.start, S.np, S.nb);
-  if (lb < 0) return;
-  switch (S.kind) {
-    case MK_LJ1G: lj1g_rows<T, R, E>(S.a, S.p.lj1g, lb); break;
-    case MK_LJ: lj_rows<T, R, E>(S.a, S.p.lj, lb); break;
-    case MK_LJ_BOTH: lj_both_rows<T, R, E>(S.a, S.p.lj1g, S.lj, lb); break;
-    case MK_RJL_DENSITY: rjl_density_rows<T, R>(S.a, S.p.rjl, S.eb, lb); break;
-    default: rjl_force_rows<T, R, E>(S.a, S.p.rjl, S.eb, lb); break;
+  RowForce f;
+  if (lb >= 0) {
+    switch (S.kind) {
+      case MK_LJ1G: f = lj1g_rows<T, R, E>(S.a, S.p.lj1g, lb); break;
+      case MK_LJ: f = lj_rows<T, R, E>(S.a, S.p.lj, lb); break;
+      case MK_LJ_BOTH: f = lj_both_rows<T, R, E>(S.a, S.p.lj1g, S.lj, lb); break;
+      case MK_RJL_DENSITY: rjl_density_rows<T, R>(S.a, S.p.rjl, S.eb, lb); break;
+      default: rjl_force_rows<T, R, E>(S.a, S.p.rjl, S.eb, lb); break;
+    }
   }
+  if (A.ke.nb) ke_parts(A.ke, f);
 }
 
 // ------------------------------------------------- graphene on a metal
@@ -1369,6 +1405,26 @@ bool multi_first_writes(pfm_ctx* h) {
   return rows == h->N;
 }
 
+// Blocks of the shared launch when it alone completes every atom's force and
+// can form an nvt step's kinetic energies as well (KeArgs), else 0: one phase
+// of lj / lj1g passes, each the only writer of its atoms.  Up to 1,024 blocks,
+// whose partials every block of the next kick_drift adds up: with 8 lanes
+// 32,768 atoms, where that costs what the launch saves (us a step with and
+// without, FP64: 8,192 atoms 16.3 and 17.4, 16,000 18.8 and 20.0, 32,000 25.3
+// and 25.1; mixed 15.0 and 16.2, 16.8 and 18.0, 21.6 and 21.9).  And what
+// red_part holds.
+int multi_ke_blocks(pfm_ctx* h) {
+  if (h->gm.ok || !multi_first_writes(h) || h->mp.phases.size() != 1 || h->nhc.size() > RED_MAXQ) return 0;
+  int nb = 0;
+  for (const auto& ps : h->mp.phases[0]) {
+    if (!ps.first || (ps.kind != MK_LJ1G && ps.kind != MK_LJ && ps.kind != MK_LJ_BOTH)) return 0;
+    const int nrows = h->inter[ps.inter].nl[ps.list].nrows;
+    if (nrows) nb += pad8(row_blocks(nrows, h->lanes, 256));
+  }
+  const size_t room = (size_t)(PFM_MAXI + 1 + RED_MAXQ) * h->red_blocks;
+  return nb <= 1024 && h->nhc.size() * nb <= room ? nb : 0;
+}
+
 // the phases of h->mp, one launch each.  Every pass adds to forces the kick
 // cleared, or with `first` (multi_first_writes) the first writer of each atom
 // writes its force.  Returns 1 when the lane count has no variant here.
@@ -1404,6 +1460,10 @@ static int multi_forces(pfm_ctx* h, bool energy, bool first) {
       ++A.n;
     }
     if (A.n == 0) continue;
+    if (h->mp_ke.nb) {
+      if (h->mp_ke.nb != start) return PFM_E_INVALID;  // the launch multi_ke_blocks counted
+      A.ke = h->mp_ke;
+    }
     DISPATCH_T3(T, {
       if (energy) PFM_LAUNCH(h, "multi", (k_multi<T, R, true>), start, BS, A);
       else PFM_LAUNCH(h, "multi", (k_multi<T, R, false>), start, BS, A);

@@ -475,6 +475,119 @@ __device__ __forceinline__ void kick_drift_atom(int i, double4 p, double4 v, con
     raise_out_of_cell(err, orig[i] + 1, step + 1, p);
 }
 
+#define RED_THREADS 256
+#define RED_MAXQ 8
+
+struct MaskQ {
+  int nq;
+  uint32_t bit[RED_MAXQ];
+};
+
+// compensated sum of one (s, c) pair per thread over the block, in a fixed
+// order: a butterfly over each wavefront's 64 lanes (cross-lane shuffles, no
+// barrier), then the four wavefront sums in LDS in wavefront order.  Every
+// thread returns the block's pair.  sh holds at least 8 doubles (callers
+// pass 2 * RED_THREADS).
+__device__ __forceinline__ CSum block_csum(CSum v, double* sh) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v.add(CSum{__shfl_xor(v.s, o), __shfl_xor(v.c, o)});
+  const int w = threadIdx.x >> 6, nw = RED_THREADS >> 6;
+  if ((threadIdx.x & 63) == 0) {
+    sh[w] = v.s;
+    sh[nw + w] = v.c;
+  }
+  __syncthreads();
+  CSum r{sh[0], sh[nw]};
+  for (int k = 1; k < nw; ++k) r.add(CSum{sh[k], sh[nw + k]});
+  __syncthreads();
+  return r;
+}
+
+// The same sums of NQ pairs per thread at once: the exchanges of the NQ
+// butterflies overlap and the block meets once instead of NQ times.  Thread 0
+// returns the block's pairs, bit for bit those of block_csum.
+template <int NQ>
+__device__ __forceinline__ void block_csum_n(CSum (&v)[NQ], double* sh) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) v[q].add(CSum{__shfl_xor(v[q].s, o), __shfl_xor(v[q].c, o)});
+  constexpr int nw = RED_THREADS / 64;
+  const int w = threadIdx.x >> 6;
+  __syncthreads();  // sh may still be read by the last call
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      sh[(q * nw + w) * 2] = v[q].s;
+      sh[(q * nw + w) * 2 + 1] = v[q].c;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      CSum r{sh[q * nw * 2], sh[q * nw * 2 + 1]};
+      for (int k = 1; k < nw; ++k) r.add(CSum{sh[(q * nw + k) * 2], sh[(q * nw + k) * 2 + 1]});
+      v[q] = r;
+    }
+  }
+}
+
+// Per-block partials of compensated sums: row q of a grid of nb blocks keeps
+// the s parts at part[2q nb + b] and the c parts at part[(2q+1) nb + b].
+__device__ __forceinline__ void put_part(double* part, int q, int nb, int b, const CSum& v) {
+  part[(size_t)(2 * q) * nb + b] = v.s;
+  part[(size_t)(2 * q + 1) * nb + b] = v.c;
+}
+// the compensated sum of row q's nb partials, in a fixed order
+__device__ __forceinline__ CSum reduce_part(const double* part, int q, int nb, double* sh) {
+  CSum a{0.0, 0.0};
+  for (int b = threadIdx.x; b < nb; b += RED_THREADS)
+    a.add(CSum{part[(size_t)(2 * q) * nb + b], part[(size_t)(2 * q + 1) * nb + b]});
+  return block_csum(a, sh);
+}
+
+// second half of one atom: kick xyz/z, then for nvms the projections
+// molecular_static_xyz/1D_velocities (md_integrators.f90:99-145).  Returns
+// whether the atom moves.
+// The fused multiply-adds are written out: what the compiler would
+// contract differs between the kernels that call this, and an nvms run has
+// to give the same bits through each of them.
+__device__ __forceinline__ bool kick2_atom(double4& v, const double4& f, double k, uint32_t m, const IntP& P,
+                                           bool nvms) {
+  const bool bx = (m & P.bxyz) != 0, bz = (m & P.bz) != 0;
+  if (!(bx || bz)) return false;
+  if (bx) { v.x = fma(f.x * k, P.ts1, v.x); v.y = fma(f.y * k, P.ts1, v.y); v.z = fma(f.z * k, P.ts1, v.z); }
+  if (bz) v.z = fma(f.z * k, P.ts1, v.z);
+  if (nvms) {
+    if (bx) {
+      const double fv = fma(f.z, v.z, fma(f.x, v.x, f.y * v.y)), ff = fma(f.z, f.z, fma(f.x, f.x, f.y * f.y));
+      if (fv > 0.0 && ff > 1e-12) { double c = fv / ff; v.x = c * f.x; v.y = c * f.y; v.z = c * f.z; }
+      else { v.x = 0; v.y = 0; v.z = 0; }
+    }
+    if (bz) {
+      const double fv = fma(f.z, v.z, fma(f.x, v.x, f.y * v.y));
+      if (!(fv > 0.0)) { v.x = 0; v.y = 0; v.z = 0; }
+    }
+  }
+  return true;
+}
+
+// What a force launch that completes every atom's force adds for an nvt step:
+// the kinetic energies of the chain groups after the second half kick, which
+// the next step's k_kick_drift<true> repeats, per block of the launch.
+struct KeArgs {
+  int nb;  // blocks of the launch (0: nothing to add)
+  const double4* vel;
+  const uint32_t* mask;
+  IntP P;
+  MaskQ Q;
+  double* part;
+  const double* C;  // chain states, cw doubles copied to C0 (as k_kick2_ke), or C0 null
+  double* C0;
+  int cw;
+};
+
 // ------------------------------------------------------------------ host side
 
 struct ListDev {
@@ -679,6 +792,7 @@ struct pfm_ctx {
     };
     std::vector<std::vector<Pass>> phases;
   } mp;
+  KeArgs mp_ke{};  // asked of the next launch_forces (multi_ke_blocks)
   // captured steady-state blocks of steps (pfm_run)
   bool use_graphs = true;
   int step_base = 0;  // first step of the block being captured (kernel step arguments are relative to it)
@@ -769,6 +883,7 @@ int launch_forces(pfm_ctx* h, bool energy, bool first_writes);
 // the shared lj / lj1g / rjl launches can write every atom's force first
 // (no zeroing before them): see plan_multi
 bool multi_first_writes(pfm_ctx* h);
+int multi_ke_blocks(pfm_ctx* h);
 // the co-scheduled launches of graphene on a metal can write every atom's
 // force first: see gm_forces
 bool gm_first_writes(pfm_ctx* h);

@@ -40,3 +40,28 @@ def test_chains(n, chains):
         np.testing.assert_allclose(eg["e_nhc"], eo["e_nhc"], rtol=1e-10)
     for (xg, vg), (xo, vo) in zip(cg, co):
         assert rel_inf(xg, xo) < 1e-10 and rel_inf(vg, vo) < 1e-10
+
+
+@pytest.mark.parametrize("n", [300, 8193, 32752, 32784])
+@pytest.mark.parametrize("groups", [(3,), (1, 2)])
+def test_energies_in_the_force_launch(n, groups):
+    """The force launch of a gas forms the kinetic energies up to 1,024 blocks
+    (32,768 atoms of 8 lanes); with separate launches (pfm_set_fusion(h, 0))
+    k_kick2_ke forms them: the same run within 1e-10."""
+    s = configs.lj_gas_lattice(n, 0.02, 72, 150.0)
+    s.nhcs = [NHC(g, 100.0, 3, 3 * n * KB * 100.0 * 20.0 ** 2) for g in groups]
+    res = []
+    for fuse in (True, False):
+        c = gpu_ctx(s)
+        c.set_fusion(fuse)
+        c.run("nvt", 0.5, 0, 0, True)
+        c.run("nvt", 0.5, 1, 30, False)
+        c.run("nvt", 0.5, 31, 40, True)
+        res.append((c.state(), c.energies(), [c.get_chain(k + 1, 3) for k in range(len(groups))]))
+        c.close()
+    (sa, ea, ca), (sb, eb, cb) = res
+    for x, y in zip(sa, sb):
+        assert rel_inf(x, y) < 1e-10
+    np.testing.assert_allclose(ea["e_nhc"], eb["e_nhc"], rtol=1e-10)
+    for (xa, va), (xb, vb) in zip(ca, cb):
+        assert rel_inf(xa, xb) < 1e-10 and rel_inf(va, vb) < 1e-10
