@@ -1,8 +1,8 @@
 """Rebuilds of few atoms (binning in one workgroup, group rows in one launch)
 about their limits: lists, velocities after the zero-momentum step and a run
 over three rebuilds against the oracle (FP64: velocities 1e-12 after the one
-subtraction, positions and forces 1e-10 as elsewhere), for 1 to 8,193 atoms
-about the steps of 256, 1,024 and 8,192, and for two replicas."""
+subtraction, positions, forces and energies 1e-10 as elsewhere), for 1 to 8,193 atoms
+about the steps of 256, 1,024 and 8,192, and for replicas."""
 import numpy as np
 import pytest
 
@@ -31,19 +31,23 @@ def test_small_rebuild(n):
     c.close()
 
 
-@pytest.mark.parametrize("sizes", [(170, 855), (4096, 4096), (4096, 4097)])
+@pytest.mark.parametrize("sizes", [(170, 855), (4096, 4096), (4096, 4097), (2047, 2049, 257)])
 def test_small_rebuild_of_replicas(sizes):
     reps = [configs.lj_gas_lattice(n, 0.02, 20 + k, 100.0, period=4) for k, n in enumerate(sizes)]
     b = system.build_batch_context(system.merge_replicas(reps), capi.FP64)
     b.run("nve", 0.5, 0, 9, True)
     p, v, f = b.state()
+    e = b.replica_energies()
     at = 0
-    for s in reps:
+    for r, s in enumerate(reps):
         c = gpu_ctx(s)
         c.run("nve", 0.5, 0, 9, True)
         q, w, g = c.state()
         for x, y in ((p, q), (v, w), (f, g)):
             assert rel_inf(x[at:at + s.n], y) < 1e-10
+        one = c.energies()
+        for name in ("pe", "ke", "temp"):
+            np.testing.assert_allclose(e[name][r], one[name], rtol=1e-10)
         at += s.n
         c.close()
     b.close()
