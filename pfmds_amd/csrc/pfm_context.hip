@@ -2028,8 +2028,9 @@ static int run_steps(pfm_ctx* h, int integ, double dt, int s0, int s1, int energ
   const bool nvt = integ == PFM_NVT && !h->nhc.empty();
   bool nhc_pending = false;
   // blocks whose partials hold a step's kinetic energies: the force launch's
-  // where it can form them, else k_kick2_ke's
-  const int ke_nb = nvt ? multi_ke_blocks(h) : 0, ke_parts = ke_nb ? ke_nb : h->red_blocks;
+  // where it can form them (it writes the forces, so none are carried over
+  // from atoms outside all_atoms), else k_kick2_ke's
+  const int ke_nb = nvt && first_writes ? multi_ke_blocks(h) : 0, ke_parts = ke_nb ? ke_nb : h->red_blocks;
   bool kick_pending = false;  // second half kick deferred into the next kick_drift
   const int CONVERGED = -1;
   // nvms blocks: the steps from spec_base on record their energies and

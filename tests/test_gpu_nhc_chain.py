@@ -65,3 +65,25 @@ def test_energies_in_the_force_launch(n, groups):
     np.testing.assert_allclose(ea["e_nhc"], eb["e_nhc"], rtol=1e-10)
     for (xa, va), (xb, vb) in zip(ca, cb):
         assert rel_inf(xa, xb) < 1e-10 and rel_inf(va, vb) < 1e-10
+
+
+def test_forces_carried_over_outside_all_atoms():
+    """Atoms outside all_atoms keep their forces between steps (zero_forces
+    clears that group only): the kinetic energies then come from the whole
+    force, as in the oracle."""
+    s = configs.lj_gas_lattice(300, 0.02, 73, 150.0)
+    s.all_atoms = 1
+    s.nhcs = [NHC(3, 100.0, 3, 3 * 300 * KB * 100.0 * 20.0 ** 2)]
+    res = []
+    for make in (oracle_ctx, gpu_ctx):
+        c = make(s)
+        c.run("nvt", 0.2, 0, 0, True)
+        c.run("nvt", 0.2, 1, 8, False)
+        c.run("nvt", 0.2, 9, 10, True)
+        res.append((c.state(), c.get_chain(1, 3)))
+        c.close()
+    (so, co), (sg, cg) = res
+    for x, y in zip(sg, so):
+        assert rel_inf(x, y) < 1e-10
+    for x, y in zip(cg, co):
+        assert rel_inf(x, y) < 1e-10
