@@ -165,9 +165,10 @@ __device__ __forceinline__ void sum_groups(V* v) {
 }
 
 // separation of a gathered entry, in FP32 (dr in FP64 then rounded, or fixed
-// point).  The lead entry of a block and the other three round their squares
-// in another order: descriptors keep the bits they have had, since a last bit
-// can move a BF16 input of the network.
+// point).  The lead entry of a block and the other three (in the tangent walk
+// all four) round their squares in another order: descriptors and tangents keep
+// the bits they have had, since a last bit can move a BF16 input of the network
+// and with it a weight gradient by some 1e-5.
 template <class R>
 __device__ __forceinline__ float sur_dr_rec(const Geo<R>& Gm, const typename Geo<R>::P& pi,
                                             const typename Geo<R>::P& pj, bool lead, float& x, float& y, float& z) {
@@ -984,7 +985,7 @@ __device__ __forceinline__ void sur_tangent_rows(const RowArgsS& a, const SurK& 
     for (int k = 0; k < 6; ++k) { dgc[k] = 0.0f; dgx[k] = 0.0f; }
     SUR_WALK_BEGIN(float4, SUR_RES)
       float dx, dy, dz;
-      float r2 = sur_dr_rec<R>(Gm, pi, pj, u_ == 0, dx, dy, dz);
+      float r2 = sur_dr_rec<R>(Gm, pi, pj, false, dx, dy, dz);
       if (!(r2 < K.rc2)) continue;
       const TangentTerms T(K, dx, dy, dz, r2, eta, (mj & K.bit1) != 0, ri, aj);
       float mono[NMON], dmono[NMON];
@@ -1017,7 +1018,7 @@ __device__ __forceinline__ void sur_tangent_rows(const RowArgsS& a, const SurK& 
     for (int k = 0; k < 3; ++k) e2[k] = K.eta2[6 * ke + (high ? 3 + k : k)];
     SUR_WALK_BEGIN(float4, SUR_RES)
       float dx, dy, dz;
-      float r2 = sur_dr_rec<R>(Gm, pi, pj, u_ == 0, dx, dy, dz);
+      float r2 = sur_dr_rec<R>(Gm, pi, pj, false, dx, dy, dz);
       if (!(r2 < K.rc2)) continue;
       const TangentTerms T(K, dx, dy, dz, r2, eta, (mj & K.bit1) != 0, ri, aj);
       float mono[NMON], dmono[NMON];
@@ -1046,8 +1047,8 @@ __device__ __forceinline__ void sur_tangent_rows(const RowArgsS& a, const SurK& 
 #pragma unroll
   for (int t = 0; t < NMON; ++t) {
     float mc = Mc[t], mx = Mx[t];
-    Scc[kDeg[t]] += kMul[t] * 2.0f * mc * dmc[t];
-    Scx[kDeg[t]] += kMul[t] * (dmc[t] * mx + mc * dmx[t]);
+    Scc[kDeg[t]] = fmaf(dmc[t], kMul[t] * 2.0f * mc, Scc[kDeg[t]]);
+    Scx[kDeg[t]] = fmaf(kMul[t], fmaf(dmc[t], mx, mc * dmx[t]), Scx[kDeg[t]]);
   }
 #pragma unroll
   for (int m = 0; m < 5; ++m) Scc[m] -= ddd[0];
