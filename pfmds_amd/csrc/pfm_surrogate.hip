@@ -385,14 +385,17 @@ __device__ __forceinline__ void sur_features(int ke, const float* mc, const floa
                                              const float* gx, float* Gr) {
 #pragma unroll
   for (int k = 0; k < 6; ++k) { Gr[6 * ke + k] = gc[k]; Gr[12 + 6 * ke + k] = gx[k]; }
-  // the first term of a degree is added to the rounded second one
-  float Scc[5], Scx[5];
+  // the first term of a degree is added to the rounded second one; the mixed
+  // sums start from fma(., ., 0), which keeps degree 0 rounded in g5_of's sums
+  // (a plain product is contracted into them: 1e-7 of G, which moves a BF16
+  // input of the network in some 2 of 1,000 rows)
+  float Scc[5], Scx[5] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int t = 0; t < NMON; ++t) {
     const float k = kMul[t] * mc[t];
     const int d = kDeg[t];
     const bool head = t == 0 || kDeg[t - 1] != d, second = !head && (t == 1 || kDeg[t >= 2 ? t - 2 : 0] != d);
-    Scx[d] = head ? k * mx[t] : fmaf(k, mx[t], Scx[d]);
+    Scx[d] = fmaf(k, mx[t], Scx[d]);
     if (head) Scc[d] = mc[t];
     else if (second) Scc[d] = fmaf(Scc[d], Scc[d], k * mc[t]);
     else Scc[d] = fmaf(mc[t], k, Scc[d]);
