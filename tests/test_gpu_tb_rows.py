@@ -42,3 +42,18 @@ def test_rows_against_oracle(a, m):
     assert rel_inf(g.state()[2], fo) < 1e-11
     np.testing.assert_allclose(g.energies()["e_inter"], o.energies()["e_inter"], rtol=1e-11)
     assert rel_inf(x.state()[2], fo) < 1e-4
+
+
+@pytest.mark.parametrize("r1,r2", [(2.0, 2.0), (1.7, 1.7), (2.1, 2.0)])
+def test_cutoff_without_a_switching_zone(r1, r2):
+    """R1 = R2 (and R1 beyond R2, which the reference's branches also take):
+    the cutoff is 1 with derivative 0 below R1, against the oracle within the
+    same 1e-11."""
+    s = clusters(1.45, 0.06, 2)
+    s.interactions[0].params[8:10] = [r1, r2]
+    g, o = gpu_ctx(s), oracle_ctx(s)
+    for c in (g, o):
+        c.run("nve", 0.5, 0, 0, True)
+    assert np.abs(o.state()[2]).max() > 1.0
+    assert rel_inf(g.state()[2], o.state()[2]) < 1e-11
+    np.testing.assert_allclose(g.energies()["e_inter"], o.energies()["e_inter"], rtol=1e-11)
