@@ -598,9 +598,12 @@ struct TbBond {
       R ir;
       dist_and_inverse<R>(d2, r, ir);
       cutoff_bl<R>(r, P.R1, P.invw, -0.5 * PFM_PI * P.invw, fc, dfc);
+      // two atoms on one point are at distance 0, inside the cutoff: the bond
+      // has an energy, and a force that is not a number stops the run
+      r = d2 > R(0) ? r : d2;
       // the selects of cos_cutoff: below R1 nothing of 1/(R2 - R1), which is
       // infinite in a cutoff without a switching zone
-      const bool below = r < P.R1, in = inside<R>(r, P.R2);
+      const bool below = r < P.R1, in = r < P.R2;
       fc = below ? R(1) : in ? fc : R(0);
       dfc = !below && in ? dfc * ir : R(0);
     }

@@ -57,3 +57,20 @@ def test_cutoff_without_a_switching_zone(r1, r2):
     assert np.abs(o.state()[2]).max() > 1.0
     assert rel_inf(g.state()[2], o.state()[2]) < 1e-11
     np.testing.assert_allclose(g.energies()["e_inter"], o.energies()["e_inter"], rtol=1e-11)
+
+
+def test_coincident_carbons_stop_the_run():
+    """Two atoms on one point with no other neighbour: as in the oracle the
+    forces are not numbers, the energy is one, and the next step's position
+    check stops the run."""
+    s = clusters(1.8, 0.0, 1)
+    s.pos[1] = s.pos[0]
+    g, o = gpu_ctx(s), oracle_ctx(s)
+    for c in (g, o):
+        c.run("nve", 0.5, 0, 0, True)
+    np.testing.assert_array_equal(np.isnan(g.state()[2]), np.isnan(o.state()[2]))
+    assert np.isnan(g.state()[2][:2]).any()
+    np.testing.assert_allclose(g.energies()["e_inter"], o.energies()["e_inter"], rtol=1e-11)
+    with pytest.raises(capi.PfmError) as e:
+        g.run("nve", 0.5, 1, 2, False)
+    assert e.value.code == capi.E_OUT_OF_CELL
