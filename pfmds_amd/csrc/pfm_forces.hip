@@ -389,7 +389,7 @@ __device__ __forceinline__ void rjl_force_rows(const RowArgs& a, const RjlP& P, 
     const double ie = Geo<R>::w(pi);
     walk_row<T, R>(G, nbrow, n, t, i, [&](int, const typename Geo<R>::P& q, bool) {
       double dx, dy, dz, r, ir;
-      f64::sqrt_rsqrt(G.d2(pi, q, dx, dy, dz), r, ir);
+      dist_and_inverse<double, E>(G.d2(pi, q, dx, dy, dz), r, ir);
       const double y = cutoff_half(r, R1, invw);
       const double C = f64::cos_q1(y), S = f64::sin_q1(y);
       const double ep = f64::exp((r - r0) * kp), eq = f64::exp((r - r0) * kq);
@@ -429,7 +429,7 @@ __device__ __forceinline__ void lj_walk(const LjP& P, const Geo<R>& G, const typ
   walk_row<T, R>(G, nbrow, n, t, i, [&](int, const typename Geo<R>::P& q, bool valid) {
     R dx, dy, dz;
     R r, ir;
-    dist_and_inverse<R>(G.d2(pi, q, dx, dy, dz), r, ir);
+    dist_and_inverse<R, E>(G.d2(pi, q, dx, dy, dz), r, ir);
     R fc, dfr;
     cutoff_bl<R>(r, R1, invw, kdf, fc, dfr);
     R s = sig * ir, s2 = s * s, V = s2 * s2 * s2;
@@ -488,12 +488,13 @@ __device__ __forceinline__ void lj1g_walk(const Lj1gP& P, const Geo<R>& G, const
     // r and 1/r from one reciprocal square root
     R ir;
     const R d2 = G.d2(pi, q, dx, dy, dz);
-    dist_and_inverse<R>(d2, r, ir);
+    dist_and_inverse<R, E>(d2, r, ir);
     invr2 = ir * ir;
     if constexpr (sizeof(R) == 4) {
       tr = __builtin_amdgcn_fmed3f(r, R1, R2);  // the clamp to [R1, R2]
     } else {
-      invr2 = fma(fma(-d2, invr2, 1.0), invr2, invr2);  // its third power follows: to within half an ulp
+      const double c2 = fma(fma(-d2, invr2, 1.0), invr2, invr2);  // its third power follows: to within half an ulp
+      invr2 = !E || d2 > 0.0 ? c2 : invr2;
       tr = fmin(fmax(r, R1), R2);
     }
     // f_dfr_cut (cut_off_poly.f90:30-43), dfr without the 1/(R2-R1) factor

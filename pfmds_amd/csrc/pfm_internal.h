@@ -301,17 +301,21 @@ __device__ __forceinline__ void cutoff_bl<float>(float r, float R1, float inv_w,
 }
 
 // r = |dr| and 1/r from dr.dr: FP64 by f64::sqrt_rsqrt; the mixed path from
-// one v_rsq_f32 (r = d2 / sqrt(d2)).  Two atoms on one point give NaN in both.
-template <class R>
-__device__ __forceinline__ void dist_and_inverse(R d2, R& r, R& ir);
-template <>
-__device__ __forceinline__ void dist_and_inverse<double>(double d2, double& r, double& ir) {
-  f64::sqrt_rsqrt(d2, r, ir);
-}
-template <>
-__device__ __forceinline__ void dist_and_inverse<float>(float d2, float& r, float& ir) {
-  ir = __builtin_amdgcn_rsqf(d2);
-  r = d2 * ir;
+// one v_rsq_f32 (r = d2 / sqrt(d2)).  Two atoms on one point give NaN in both,
+// with E (FP64 passes that form energies) r = 0 and 1/r infinite: their force
+// is not a number either way, and their energy is that of the formula.
+template <class R, bool E = false>
+__device__ __forceinline__ void dist_and_inverse(R d2, R& r, R& ir) {
+  if constexpr (sizeof(R) == 8) {
+    f64::sqrt_rsqrt(d2, r, ir);
+    if (E) {
+      r = d2 > 0.0 ? r : d2;
+      ir = d2 > 0.0 ? ir : __builtin_amdgcn_rsq(d2);
+    }
+  } else {
+    ir = __builtin_amdgcn_rsqf(d2);
+    r = d2 * ir;
+  }
 }
 
 // Neumaier's compensated sum (Neumaier 1974, "Rundungsfehleranalyse einiger

@@ -120,3 +120,23 @@ def test_coincident_atoms_stop_the_run(name):
     with pytest.raises(capi.PfmError) as e:
         c.run("nve", 1.0, 1, 2, False)
     assert e.value.code == capi.E_OUT_OF_CELL
+
+
+@pytest.mark.parametrize("name", ["lj", "lj1g", "rjl"])
+def test_coincident_atoms_energy(name):
+    """Two atoms on one point: their rows' energies are those of the formulas,
+    infinite for the powers of 1/r (and the interaction's sum then is no
+    number, as its compensated sum cannot be) and finite for the exponentials
+    (the sum is the oracle's)."""
+    params = list(configs.RJL_CU) if name == "rjl" else [0.0104, 3.4, 6.5, 7.5]
+    s, _ = dimers(name, params, 2.6, 5.9, 6.5 if name == "rjl" else 8.5)
+    s.pos[1] = s.pos[0]
+    g, o = gpu_ctx(s), oracle_ctx(s)
+    for c in (g, o):
+        c.run("nve", 1.0, 0, 0, True)
+    np.testing.assert_array_equal(np.isnan(g.state()[2][:2]), np.isnan(o.state()[2][:2]))
+    if name == "rjl":
+        np.testing.assert_allclose(g.energies()["e_inter"], o.energies()["e_inter"], rtol=1e-12)
+    else:
+        e = g.row_energies(1)
+        assert not np.isnan(e).any() and np.isposinf(e).sum() == 1 and o.energies()["e_inter"][0] == np.inf
