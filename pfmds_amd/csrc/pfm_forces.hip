@@ -269,8 +269,15 @@ __device__ __forceinline__ float rjl_d2(const Geo<float>& G, const uint4& a, con
   }
 }
 
+// -pi/(2 (R2 - R1)) of a potential's parameters: in FP64 from one division
+template <class R, class P>
+__device__ __forceinline__ R cutoff_kdf(const P& p) {
+  if constexpr (sizeof(R) == 8) return -p.hw;
+  return -0.5 * PFM_PI * p.invw;
+}
+
 struct RjlP {
-  double A0, xi, p, q, r0, R1, R2, invw;
+  double A0, xi, p, q, r0, R1, R2, invw, hw;  // hw: pi/(2 (R2 - R1)), FP64 passes
 };
 
 // largest workgroup of the row passes: FP32 pair arithmetic fits 128 VGPRs
@@ -307,12 +314,11 @@ __device__ __forceinline__ void rjl_density_rows(const RowArgs& a, const RjlP& P
     // FP64: exp(-2q(r/r0 - 1)) with its argument as (r - r0) (-2q/r0), whose
     // rounding vanishes where the term is largest; two atoms on one point
     // count as at a vanishing distance
-    const double R1 = P.R1, R2 = P.R2, invw = P.invw, r0 = P.r0, kr = -2.0 * P.q / P.r0;
+    const double R1 = P.R1, R2 = P.R2, hw = P.hw, r0 = P.r0, kr = -2.0 * P.q / P.r0;
     walk_row<T, R>(G, nbrow, n, t, i, [&](int, const typename Geo<R>::P& q, bool) {
       double dx, dy, dz, r, ir;
       f64::sqrt_rsqrt(fmax(G.d2(pi, q, dx, dy, dz), 1e-300), r, ir);
-      const double c = f64::cos_q1(cutoff_half(r, R1, invw));
-      const double e = f64::exp((r - r0) * kr) * (c * c);
+      const double e = f64::exp((r - r0) * kr) * CutoffHalf(r, R1, R2, hw).f();
       rho += r <= R2 ? e : 0.0;
     });
   }
@@ -379,26 +385,24 @@ __device__ __forceinline__ void rjl_force_rows(const RowArgs& a, const RjlP& P, 
     if (hiso > 0.0f) body(std::true_type{});
     else body(std::false_type{});
   } else {
-    // FP64: with C = cos(pi x/2), S = sin(pi x/2) of the cutoff's x, fc = C^2
-    // and df r = 2 kdf S C, so the two brackets are C (Ac C + As S) and
-    // C (Bc C + Bs S).  Two atoms on one point give NaN.
-    const double R1 = P.R1, R2 = P.R2, invw = P.invw, kdf = -0.5 * PFM_PI * P.invw;
+    // FP64: df r = -2 hw times the cutoff's half_sine
+    const double R1 = P.R1, R2 = P.R2, hw = P.hw;
     const double r0 = P.r0, kp = -P.p / P.r0, kq = -2.0 * P.q / P.r0;
-    const double Ac = 2.0 * P.A0 * P.p / P.r0, As = -4.0 * P.A0 * kdf;
-    const double Bc = P.xi * P.q / P.r0, Bs = -P.xi * kdf;
+    const double Ac = 2.0 * P.A0 * P.p / P.r0, As = 4.0 * P.A0 * hw;
+    const double Bc = P.xi * P.q / P.r0, Bs = P.xi * hw;
     const double ie = Geo<R>::w(pi);
     walk_row<T, R>(G, nbrow, n, t, i, [&](int, const typename Geo<R>::P& q, bool) {
       double dx, dy, dz, r, ir;
       dist_and_inverse<double, E>(G.d2(pi, q, dx, dy, dz), r, ir);
-      const double y = cutoff_half(r, R1, invw);
-      const double C = f64::cos_q1(y), S = f64::sin_q1(y);
+      const CutoffHalf cut(r, R1, R2, hw);
+      const double fc = cut.f(), hs = cut.half_sine();
       const double ep = f64::exp((r - r0) * kp), eq = f64::exp((r - r0) * kq);
-      const double A = fma(As, S, Ac * C), B = fma(Bs, S, Bc * C);
-      double c = fma(A, ep, -(B * (ie + Geo<R>::w(q)) * eq)) * (C * ir);
+      const double A = fma(As, hs, Ac * fc), B = fma(Bs, hs, Bc * fc);
+      double c = fma(A, ep, -(B * (ie + Geo<R>::w(q)) * eq)) * ir;
       const bool in = !(r > R2);
       c = in ? c : 0.0;
       fx = fma(-c, dx, fx); fy = fma(-c, dy, fy); fz = fma(-c, dz, fz);
-      if (E) er += in ? ep * (C * C) : 0.0;
+      if (E) er += in ? ep * fc : 0.0;
     });
   }
   fx = group_sum<T>(fx); fy = group_sum<T>(fy); fz = group_sum<T>(fz);
@@ -418,20 +422,20 @@ __global__ void __launch_bounds__(PAIR_BLOCK) k_rjl_force(RowArgs a, RjlP P, con
 // -------------------------------------------------------------------- LJ
 
 struct LjP {
-  double eps4, sig, R1, R2, invw;
+  double eps4, sig, R1, R2, invw, hw;
 };
 
 // a row's lj entries into acc
 template <int T, class R, bool E>
 __device__ __forceinline__ void lj_walk(const LjP& P, const Geo<R>& G, const typename Geo<R>::P& pi,
                                         const int* __restrict__ nbrow, int n, int t, int i, RowAcc<R>& acc) {
-  const R R1 = P.R1, R2 = P.R2, invw = P.invw, sig = P.sig, e4 = P.eps4, kdf = -0.5 * PFM_PI * P.invw;
+  const R R1 = P.R1, R2 = P.R2, invw = P.invw, sig = P.sig, e4 = P.eps4, kdf = cutoff_kdf<R>(P);
   walk_row<T, R>(G, nbrow, n, t, i, [&](int, const typename Geo<R>::P& q, bool valid) {
     R dx, dy, dz;
     R r, ir;
     dist_and_inverse<R, E>(G.d2(pi, q, dx, dy, dz), r, ir);
     R fc, dfr;
-    cutoff_bl<R>(r, R1, invw, kdf, fc, dfr);
+    cutoff_bl<R>(r, R1, R2, invw, kdf, fc, dfr);
     R s = sig * ir, s2 = s * s, V = s2 * s2 * s2;
     R c = e4 * (V * (R(12) * V - R(6)) * fc * ir - V * (V - R(1)) * dfr) * ir;
     const bool in = valid && inside<R>(r, R2);
@@ -568,7 +572,7 @@ __global__ void __launch_bounds__(PAIR_BLOCK) k_lj1g(RowArgs a, Lj1gP P, int nb_
 // -------------------------------------------------------------------- TB
 
 struct TbP {
-  double D, S, beta, r0, delt, a0, c02, d02, R1, R2, invw;
+  double D, S, beta, r0, delt, a0, c02, d02, R1, R2, invw, hw;
 };
 
 // Tersoff-Brenner rows are short (three bonds in graphene): TB_T lanes share
@@ -598,7 +602,7 @@ struct TbBond {
       // no branch, and the polynomials instead of the library's sine and cosine
       R ir;
       dist_and_inverse<R>(d2, r, ir);
-      cutoff_bl<R>(r, P.R1, P.invw, -0.5 * PFM_PI * P.invw, fc, dfc);
+      cutoff_bl<R>(r, P.R1, P.R2, P.invw, cutoff_kdf<R>(P), fc, dfc);
       // two atoms on one point are at distance 0, inside the cutoff: the bond
       // has an energy, and a force that is not a number stops the run
       r = d2 > R(0) ? r : d2;
@@ -811,10 +815,11 @@ struct CosP {
   double pref, sig, a, r0, delt, R1, R2, invw, nn_coef;
   int morse;
   int whole;  // delt when it is 1, 2, 3 or 4, else 0
+  double hw;
 };
 
-// x**delt, x >= 0.  FP64: whole exponents up to 4 by products, at most two
-// roundings; the general power is 60 of the 190 instructions an entry takes
+// x**delt, x >= 0.  FP64: whole exponents up to 4 by products, the third and
+// fourth power from the square in two parts (0.50 ulp); the general power is 60 of the 190 instructions an entry takes
 // (graphene pass of 24,960 rows 20.0 -> 16.5 us, metal rows 25.6 -> 19.6 with
 // 1/|n| kept beside the normal; with the library's functions 30.1 and 38.5).
 // The mixed path's power is two transcendental instructions for any exponent.
@@ -822,8 +827,8 @@ template <class R>
 __device__ __forceinline__ R cos_power(const CosP& P, R x) {
   if constexpr (sizeof(R) == 8) {
     if (P.whole) {  // uniform
-      const R x2 = x * x;
-      return P.whole == 1 ? x : P.whole == 2 ? x2 : x2 * (P.whole == 3 ? x : x2);
+      const R x2 = x * x, l = fma(x, x, -x2);
+      return P.whole == 1 ? x : P.whole == 2 ? x2 : P.whole == 3 ? fma(x2, x, l * x) : fma(x2, x2, (l + l) * x2);
     }
   }
   return PM<R>::pow_(x, R(P.delt));
@@ -832,9 +837,9 @@ __device__ __forceinline__ R cos_power(const CosP& P, R x) {
 template <class R>
 __device__ __forceinline__ void cos_pair(const CosP& P, R r, R ir, R nd, R nnorm_r, R& A, R& Bc, R& S_coef,
                                          R& epair) {
-  const R R1 = P.R1, invw = P.invw, delt = P.delt, kdf = -0.5 * PFM_PI * P.invw;
+  const R R1 = P.R1, R2 = P.R2, invw = P.invw, delt = P.delt, kdf = cutoff_kdf<R>(P);
   R fc, dfr;
-  cutoff_bl<R>(r, R1, invw, kdf, fc, dfr);
+  cutoff_bl<R>(r, R1, R2, invw, kdf, fc, dfr);
   R dfc = dfr * ir;
   R V2;
   if (P.morse) V2 = PM<R>::exp_(-R(P.a) * (r - R(P.r0)));
@@ -1259,12 +1264,15 @@ static int pass_lanes(const pfm_ctx* h, const Inter& it) { return it.lanes ? it.
     default: { constexpr int T = 8; __VA_ARGS__; } break;  \
   }
 
+// pi/(2 (R2 - R1)) of a cosine cutoff (hw of the parameters)
+static double half_width(double R1, double R2) { return 0.5 * PFM_PI / (R2 - R1); }
 static TbP tb_params(const Inter& it) {
   return TbP{it.p[0], it.p[1], it.p[2], it.p[3], it.p[4], it.p[5], it.p[6] * it.p[6], it.p[7] * it.p[7],
-             it.p[8], it.p[9], 1.0 / (it.p[9] - it.p[8])};
+             it.p[8], it.p[9], 1.0 / (it.p[9] - it.p[8]), half_width(it.p[8], it.p[9])};
 }
 static RjlP rjl_params(const Inter& it) {
-  return RjlP{it.p[0], it.p[1], it.p[2], it.p[3], it.p[4], it.p[5], it.p[6], 1.0 / (it.p[6] - it.p[5])};
+  return RjlP{it.p[0], it.p[1], it.p[2], it.p[3], it.p[4], it.p[5], it.p[6], 1.0 / (it.p[6] - it.p[5]),
+              half_width(it.p[5], it.p[6])};
 }
 static CosP cos_params(const Inter& it) {
   const bool morse = it.kind == PFM_MORSEC;
@@ -1272,13 +1280,13 @@ static CosP cos_params(const Inter& it) {
   const int whole = delt == 1.0 || delt == 2.0 || delt == 3.0 || delt == 4.0 ? (int)delt : 0;
   if (morse)
     return CosP{it.p[0], 0.0, it.p[2], it.p[1], delt, it.p[4], it.p[5], 1.0 / (it.p[5] - it.p[4]),
-                2.0 * it.p[0] * delt, 1, whole};
+                2.0 * it.p[0] * delt, 1, whole, half_width(it.p[4], it.p[5])};
   return CosP{4.0 * it.p[0], it.p[1], 0.0, 0.0, delt, it.p[3], it.p[4], 1.0 / (it.p[4] - it.p[3]),
-              4.0 * it.p[0] * delt, 0, whole};
+              4.0 * it.p[0] * delt, 0, whole, half_width(it.p[3], it.p[4])};
 }
 
 static LjP lj_params(const Inter& it) {
-  return LjP{4.0 * it.p[0], it.p[1], it.p[2], it.p[3], 1.0 / (it.p[3] - it.p[2])};
+  return LjP{4.0 * it.p[0], it.p[1], it.p[2], it.p[3], 1.0 / (it.p[3] - it.p[2]), half_width(it.p[2], it.p[3])};
 }
 static Lj1gP lj1g_params(const Inter& it) {
   double eps = it.p[0], sig = it.p[1], s6 = sig * sig * sig * sig * sig * sig;
@@ -1573,7 +1581,7 @@ static int forces_T(pfm_ctx* h, bool energy, bool first_writes) {
       case PFM_RJL: {
         RowArgs a = row_args(h, it, 0, written ? 1 : 0);
         if (a.nrows == 0) break;
-        RjlP P{it.p[0], it.p[1], it.p[2], it.p[3], it.p[4], it.p[5], it.p[6], 1.0 / (it.p[6] - it.p[5])};
+        const RjlP P = rjl_params(it);
         int T = pass_lanes(h, it);
         DISPATCH_T(T, {
           int nb = row_blocks(a.nrows, T, BS);
@@ -1585,7 +1593,7 @@ static int forces_T(pfm_ctx* h, bool energy, bool first_writes) {
         break;
       }
       case PFM_LJ: {
-        LjP P{4.0 * it.p[0], it.p[1], it.p[2], it.p[3], 1.0 / (it.p[3] - it.p[2])};
+        const LjP P = lj_params(it);
         for (int k = 0; k < 2; ++k) {
           RowArgs a = row_args(h, it, k, written ? 1 : 0);
           if (a.nrows == 0) continue;
@@ -1603,9 +1611,7 @@ static int forces_T(pfm_ctx* h, bool energy, bool first_writes) {
       case PFM_LJ1G: {
         RowArgs a = row_args(h, it, 0, written ? 1 : 0);
         if (a.nrows == 0) break;
-        double eps = it.p[0], sig = it.p[1], s6 = sig * sig * sig * sig * sig * sig;
-        Lj1gP P{4.0 * eps * s6, 4.0 * eps * s6 * s6, 6.0 * 4.0 * eps * s6, 12.0 * 4.0 * eps * s6 * s6,
-                it.p[2], it.p[3], 1.0 / (it.p[3] - it.p[2])};
+        const Lj1gP P = lj1g_params(it);
         int T = pass_lanes(h, it);
         DISPATCH_T(T, {
           int nb = row_blocks(a.nrows, T, BS);
@@ -1618,8 +1624,7 @@ static int forces_T(pfm_ctx* h, bool energy, bool first_writes) {
       case PFM_TB: {
         RowArgs a = row_args(h, it, 0, written ? 1 : 0);
         if (a.nrows == 0) break;
-        TbP P{it.p[0], it.p[1], it.p[2], it.p[3], it.p[4], it.p[5], it.p[6] * it.p[6], it.p[7] * it.p[7],
-              it.p[8], it.p[9], 1.0 / (it.p[9] - it.p[8])};
+        const TbP P = tb_params(it);
         int nb = row_blocks(a.nrows, TB_T, BS1);
         double* BT = it.Bp + (size_t)it.nl[0].nrows * it.nl[0].stride;
         PFM_LAUNCH(h, "tb_bond", (k_tb_bond<R>), pad8(nb), BS1, a, P, it.B, it.Bp, BT, nb);

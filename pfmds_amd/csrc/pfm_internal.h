@@ -103,14 +103,16 @@ template <> struct Geo<float> {
 // versions carry the special cases of their whole domains (denormals,
 // large-argument reduction, division fix-up) into every list entry: the RGL
 // force pass took about 230 vector instructions an entry with them and takes
-// 112 with these, 60.7 -> 43.9 us a launch on 97,092 atoms (density pass
-// 50.7 -> 34.2 us).  These take the arguments the passes produce, without
-// branches; polynomials are interpolations at Chebyshev nodes (their own
-// error below 4e-17 relative), the last operation of each is the one that
-// rounds.  Largest errors in ulps: rcp 0.50, sqrt 0.50, 1/sqrt 0.99, exp
-// 1.13, sin 1.9, cos 1.3 below 1.4 (absolute 1.7e-16 at pi/2), pow 2.0; the
-// forces of a Cu crystal and of a gas against long double are no further off
-// than before (3.25e-15 -> 3.23e-15, 3.15e-15 -> 2.88e-15).
+// 126 with these, 59.4 -> 43.6 us a launch on 97,556 atoms (density pass
+// 49.6 -> 33.5 us).  These take the arguments the passes produce, without
+// branches; polynomials are interpolations at Chebyshev nodes, the last
+// operation of each is the one that rounds.  None is less accurate than what
+// it stands for; largest errors over 4 million arguments, here and the
+// library's, in ulps: exp 0.83 and 0.87, pow 0.83 and 1.34, 1/sqrt 1.00 and
+// (with its division) 1.49, rcp and sqrt 0.50 both, third and fourth power
+// 0.50 and 1.34; the cosine cutoff's f 2.3 and 2.7 x 2^-53 (RMS 0.39 and
+// 0.51), its derivative 3.9 and 6.4 (0.76 and 1.07).  Forms with fewer
+// instructions (exp 1.13, pow 1.57, cutoff 3.2 and 8.7) took 40.9 and 32.1 us.
 namespace f64 {
 // a constant in scalar registers: left to itself the compiler keeps the
 // polynomials' coefficients in vector registers and copies each one before
@@ -142,8 +144,12 @@ __device__ __forceinline__ double sqrt(double d2) {
   sqrt_rsqrt(d2, r, ir);
   return r;
 }
-// 2^n (1 + r + r^2 ...): e**r for |r| <= ln2/2 by degree 11, scaled
-__device__ __forceinline__ double exp_tail(double r, double n) {
+// 2^n e**(x - n ln2) with ln2 in two parts, the first with 21 zero bits at its
+// end so that rh = x - n ln2_hi is exact (the split of fdlibm's e_exp.c): the
+// sum 1 + rh in two parts, so that the last addition is the only one that
+// rounds at the result's size, and degree 11 in r = x - n ln2, |r| <= ln2/2
+__device__ __forceinline__ double exp_tail(double rh, double nl, double lo, double n) {
+  const double r = fma(nl, lo, rh);  // nl lo = -n ln2_lo (+ xl)
   double q = sc(0x1.af2391d7f5e6cp-26);
   q = fma(q, r, sc(0x1.288060f149570p-22));
   q = fma(q, r, sc(0x1.71de17d5ef6f3p-19));
@@ -154,44 +160,42 @@ __device__ __forceinline__ double exp_tail(double r, double n) {
   q = fma(q, r, sc(0x1.5555555554cb0p-5));
   q = fma(q, r, sc(0x1.5555555555555p-3));
   q = fma(q, r, 0.5);
-  return __builtin_amdgcn_ldexp(1.0 + fma(r * r, q, r), (int)n);
+  const double s = 1.0 + rh, e = fma(nl, lo, (1.0 - s) + rh);
+  return __builtin_amdgcn_ldexp(s + fma(r * r, q, e), (int)n);
 }
-// exp(x), x = n ln2 + r, for |x| < 1e15; underflow to 0 and overflow to
-// infinity come from the scaling
+// exp(x) for |x| < 1e15; underflow to 0 and overflow to infinity come from the
+// scaling
 __device__ __forceinline__ double exp(double x) {
   const double n = rint(x * 0x1.71547652b82fep+0);
-  return exp_tail(fma(-n, 0x1.a39ef35793c76p-33, fma(-n, 0x1.62e42fee00000p-1, x)), n);
+  return exp_tail(fma(-n, 0x1.62e42fee00000p-1, x), -n, 0x1.a39ef35793c76p-33, n);
 }
-// exp(x + xl), |xl| << |x|
+// exp(x + xl), |xl| << 1
 __device__ __forceinline__ double exp(double x, double xl) {
-  const double n = rint(x * 0x1.71547652b82fep+0);
-  return exp_tail(fma(-n, 0x1.62e42fee00000p-1, x) + fma(-n, 0x1.a39ef35793c76p-33, xl), n);
+  const double n = rint((x + xl) * 0x1.71547652b82fep+0);
+  return exp_tail(fma(-n, 0x1.62e42fee00000p-1, x), fma(-n, 0x1.a39ef35793c76p-33, xl), 1.0, n);
 }
-// sine and cosine of y in [0, pi/2]
-__device__ __forceinline__ double cos_q1(double y) {
-  const double z = y * y;
-  double p = sc(-0x1.5eeafc14774b8p-53);
-  p = fma(p, z, sc(0x1.ae5a5d377edf5p-45));
-  p = fma(p, z, sc(-0x1.9396fdb46f278p-37));
-  p = fma(p, z, sc(0x1.1eed8ea6c7954p-29));
-  p = fma(p, z, sc(-0x1.27e4fb771a86dp-22));
-  p = fma(p, z, sc(0x1.a01a01a019783p-16));
-  p = fma(p, z, sc(-0x1.6c16c16c16c13p-10));
+// sine and cosine of t in [0, pi/4]
+__device__ __forceinline__ double sin_q1(double t) {
+  const double z = t * t;
+  double p = sc(-0x1.ab16f5caa198ap-41);
+  p = fma(p, z, sc(0x1.61217d9252c03p-33));
+  p = fma(p, z, sc(-0x1.ae645410e937bp-26));
+  p = fma(p, z, sc(0x1.71de3a545f836p-19));
+  p = fma(p, z, sc(-0x1.a01a01a01992fp-13));
+  p = fma(p, z, sc(0x1.1111111111110p-7));
+  p = fma(p, z, sc(-0x1.5555555555555p-3));
+  return fma(t * z, p, t);
+}
+__device__ __forceinline__ double cos_q1(double t) {
+  const double z = t * t;
+  double p = sc(-0x1.907cd8ff5ed8fp-37);
+  p = fma(p, z, sc(0x1.1eeb67d026ec6p-29));
+  p = fma(p, z, sc(-0x1.27e4fa16cc2d1p-22));
+  p = fma(p, z, sc(0x1.a01a019f4ddfdp-16));
+  p = fma(p, z, sc(-0x1.6c16c16c16963p-10));
   p = fma(p, z, sc(0x1.5555555555555p-5));
   p = fma(p, z, -0.5);
   return fma(p, z, 1.0);
-}
-__device__ __forceinline__ double sin_q1(double y) {
-  const double z = y * y;
-  double p = sc(0x1.89a4866f527ebp-49);
-  p = fma(p, z, sc(-0x1.ae5138c1216b3p-41));
-  p = fma(p, z, sc(0x1.6124015b5ee3ap-33));
-  p = fma(p, z, sc(-0x1.ae6455a1d7087p-26));
-  p = fma(p, z, sc(0x1.71de3a5456716p-19));
-  p = fma(p, z, sc(-0x1.a01a01a018aadp-13));
-  p = fma(p, z, sc(0x1.1111111111107p-7));
-  p = fma(p, z, sc(-0x1.5555555555555p-3));
-  return fma(y * z, p, y);
 }
 // x**y for finite x > 0: log x = 2 atanh((m-1)/(m+1)) + e ln2 as a two-part
 // sum (its second part holds the quotient's remainder and the cubic and
@@ -275,25 +279,37 @@ __device__ __forceinline__ void cos_cutoff(R r, R R1, R R2, R inv_w, R& f, R& df
 // or beyond R2 are masked by the caller.  Returns f and dfr = f'(r)
 // (= df_cut * r of the reference, whose df_cut is f'/r), kdf = -pi/(2 (R2-R1)).
 template <class R>
-__device__ __forceinline__ void cutoff_bl(R r, R R1, R inv_w, R kdf, R& f, R& dfr);
-// FP64: through the half angle y = pi x / 2 in [0, pi/2], f = cos(y)^2 and
-// sin(pi x) = 2 sin(y) cos(y); f is exactly 1 and dfr exactly 0 at x = 0
-__device__ __forceinline__ double cutoff_half(double r, double R1, double inv_w) {
-  return fmin(fmax((r - R1) * (0.5 * PFM_PI * inv_w), 0.0), 0.5 * PFM_PI);
-}
+__device__ __forceinline__ void cutoff_bl(R r, R R1, R R2, R inv_w, R kdf, R& f, R& dfr);
+// FP64: through the half angle of the nearer edge, t = hw (r - R1) or
+// hw (R2 - r), hw = pi/(2 (R2 - R1)), in [0, pi/4]: with s = sin t, f =
+// cos^2(pi x/2) is 1 - s^2 in the lower half of the zone and s^2 in the upper
+// one, and sin(pi x) = 2 s cos t in both.  f is exactly 1 and dfr exactly 0 at
+// x = 0.  (The last term: pi is the reference's literal, short of pi by twice it.)
+struct CutoffHalf {
+  double s, t;
+  bool lower;
+  __device__ __forceinline__ CutoffHalf(double r, double R1, double R2, double hw) {
+    const double a = fmax((r - R1) * hw, 0.0), b = fma(R2 - r, hw, 0x1.d1a62633145c0p-50);
+    lower = a < b;
+    t = fmin(a, b);
+    s = f64::sin_q1(t);
+  }
+  __device__ __forceinline__ double f() const { return lower ? fma(-s, s, 1.0) : s * s; }
+  __device__ __forceinline__ double half_sine() const { return s * f64::cos_q1(t); }  // sin(pi x) / 2
+};
 template <>
-__device__ __forceinline__ void cutoff_bl<double>(double r, double R1, double inv_w, double kdf, double& f,
-                                                  double& dfr) {
-  const double y = cutoff_half(r, R1, inv_w);
-  const double c = f64::cos_q1(y);
-  f = c * c;
-  dfr = (kdf + kdf) * (f64::sin_q1(y) * c);
+__device__ __forceinline__ void cutoff_bl<double>(double r, double R1, double R2, double inv_w, double kdf,
+                                                  double& f, double& dfr) {
+  const CutoffHalf c(r, R1, R2, -kdf);
+  f = c.f();
+  dfr = (kdf + kdf) * c.half_sine();
 }
 // Mixed path: the argument in revolutions t = (r - R1) / (2 (R2 - R1)) is one
 // fused multiply-add (its constants are loop invariants), clamped to [0, 1/2]
 // by one v_med3_f32, then v_sin_f32 / v_cos_f32 of 2 pi t = pi x.
 template <>
-__device__ __forceinline__ void cutoff_bl<float>(float r, float R1, float inv_w, float kdf, float& f, float& dfr) {
+__device__ __forceinline__ void cutoff_bl<float>(float r, float R1, float R2, float inv_w, float kdf, float& f,
+                                                 float& dfr) {
   const float a = 0.5f * inv_w, b = -0.5f * R1 * inv_w;
   const float t = __builtin_amdgcn_fmed3f(__builtin_fmaf(r, a, b), 0.0f, 0.5f);
   f = 0.5f + 0.5f * __builtin_amdgcn_cosf(t);

@@ -140,3 +140,57 @@ def test_coincident_atoms_energy(name):
     else:
         e = g.row_energies(1)
         assert not np.isnan(e).any() and np.isposinf(e).sum() == 1 and o.energies()["e_inter"][0] == np.inf
+
+
+def rjl_row_energies(r, p, r0, R1, R2):
+    """Energies of isolated rjl dimers along x with A0 = 1 and xi = 0, so that
+    each of a dimer's two rows holds exp(-(r - r0) p/r0) f(r), in ascending
+    order; separations r are multiples of 2^-40."""
+    m = int(np.ceil(len(r) ** (1 / 3)))
+    step = float(2 ** np.ceil(np.log2(2.2 * R2 + 4.0)))
+    g = np.stack(np.meshgrid(np.arange(m), np.arange(m), np.arange(m), indexing="ij"), -1).reshape(-1, 3)[:len(r)]
+    a = g * step + 1.0
+    b = a.copy()
+    b[:, 0] += r
+    assert (b[:, 0] - a[:, 0] == r).all()
+    pos = np.stack([a, b], 1).reshape(-1, 3)
+    n = len(pos)
+    s = System(box=np.full(3, m * step), pos=pos, vel=np.zeros((n, 3)), mass=np.full(n, 63.546), species=["Cu"] * n,
+               groups=[["Cu"], ["#"]],
+               interactions=[Interaction("rjl", [1.0, 0.0, p, 0.0, r0, R1, R2], [(1, 1, 4, R2 + 0.25, 10)])],
+               integrators=[Integrator("nve", 1.0, 10, 10**9, 10**9)], z_moving=2)
+    c = gpu_ctx(s)
+    c.run("nve", 1.0, 0, 0, True)
+    e = np.sort(c.row_energies(1)).reshape(-1, 2)
+    np.testing.assert_array_equal(e[:, 0], e[:, 1])
+    return e[:, 0]
+
+
+def separations(lo, hi, k, seed):
+    return np.round(np.random.default_rng(seed).uniform(lo, hi, k) * 2.0 ** 40) / 2.0 ** 40
+
+
+def test_exponential_is_no_less_accurate_than_the_library():
+    """The argument r0 - r is exact for p = r0 = 1, so the rows hold the
+    exponential alone: within the 0.87 ulp that the library's has over
+    [-25, 12] (4 million arguments)."""
+    r = separations(0.1, 20.0, 8000, 1)
+    e = rjl_row_energies(r, 1.0, 1.0, 20.5, 21.0)
+    want = np.sort(np.exp(1 - r.astype(LD)))
+    err = np.abs(e - want) / np.spacing(want.astype(float))
+    print(f"[exp] max {float(err.max()):.3f} ulp", flush=True)
+    assert float(err.max()) < 0.87
+
+
+@pytest.mark.parametrize("R1,R2", [(1.7, 2.0), (5.5, 6.0), (6.1, 7.3), (6.5, 7.5)])
+def test_cutoff_is_no_less_accurate_than_the_library(R1, R2):
+    """p = 0 leaves the cutoff alone: its RMS error over the switching zone
+    within 0.51 u, that of (1 + cos(pi x))/2 with the library's cosine over
+    random zones."""
+    r = separations(R1, R2, 8000, 2)
+    r = r[(r > R1) & (r < R2)]
+    e = rjl_row_energies(r, 0.0, 1.0, R1, R2)
+    want = np.sort(switch(r.astype(LD), LD(R1), LD(R2))[0])
+    err = ((e - want) / U).astype(float)
+    print(f"[cutoff] max {np.abs(err).max():.3f} u, rms {np.sqrt((err ** 2).mean()):.3f} u", flush=True)
+    assert np.sqrt((err ** 2).mean()) < 0.51
