@@ -451,6 +451,10 @@ struct NhcLane {
   __device__ __forceinline__ void set(int j, double a) {
     if ((int)threadIdx.x == j) v = a;
   }
+  // e**x for every x: a thermostat light beside its group takes x to any size
+  static __device__ __forceinline__ double expo(double x) {
+    return f64::exp(x > 1e4 ? 1e4 : x < -1e4 ? -1e4 : x);
+  }
   // n / q[j], correctly rounded from the rounded reciprocal (Markstein)
   __device__ __forceinline__ double over_q(double n, int j) const {
     const double r = at(rq, j), d = at(q, j), y = n * r;
@@ -471,15 +475,15 @@ struct NhcLane {
       double vn = at(v, M - 1) + push(M - 1, ts2);
       set(M - 1, vn);
       for (int j = M - 2; j >= 1; --j) {
-        b = f64::exp(-vn * ts3);
+        b = expo(-vn * ts3);
         if ((int)threadIdx.x == j) bj = b;
         vn = fma(push(j, ts2), b, at(v, j) * (b * b));
         set(j, vn);
       }
-      b = f64::exp(-vn * ts3);
+      b = expo(-vn * ts3);
     }
     const double v0 = fma(over_q(fma(2.0, ke, -g), 0) * ts2, b, at(v, 0) * (b * b));
-    const double s = f64::exp(-v0 * ts1);
+    const double s = expo(-v0 * ts1);
     set(0, v0);
     x = fma(v, ts1, x);
     set(0, fma(over_q(fma(2.0 * ke, s * s, -g), 0) * ts2, b, v0 * (b * b)));

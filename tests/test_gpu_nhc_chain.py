@@ -87,3 +87,24 @@ def test_forces_carried_over_outside_all_atoms():
         assert rel_inf(x, y) < 1e-10
     for x, y in zip(cg, co):
         assert rel_inf(x, y) < 1e-10
+
+
+@pytest.mark.parametrize("q,M", [(1e-3, 1), (1e-12, 3), (1e-30, 1), (1e-30, 3), (1e-300, 1)])
+def test_small_masses_at_zero_temperature(q, M):
+    """A light thermostat at T = 0: its velocity takes the scale's exponent far
+    past the exponential's range, where the scale is 0 as in the oracle."""
+    s = configs.lj_gas_lattice(300, 0.02, 73, 150.0)
+    s.nhcs = [NHC(3, 0.0, M, q)]
+    res = []
+    for make in (oracle_ctx, gpu_ctx):
+        c = make(s)
+        c.run("nvt", 0.5, 0, 0, True)
+        c.run("nvt", 0.5, 1, 2, True)
+        c.run("nvt", 0.5, 3, 8, False)
+        res.append((c.state(), c.get_chain(1, M)))
+        c.close()
+    (so, co), (sg, cg) = res
+    for x, y in zip(sg, so):
+        np.testing.assert_allclose(x, y, rtol=0, atol=1e-10 * max(np.abs(y).max(), 1.0))
+    for x, y in zip(cg, co):
+        np.testing.assert_allclose(x, y, rtol=1e-9)
