@@ -797,9 +797,8 @@ static int finalize(pfm_ctx* h) {
   }
   // grids, Morton ranks offset by each replica's first cell
   h->hrep.assign(nrep, RepDev());
-  std::vector<int> rank_all, xyz_all, crep_all;
+  std::vector<int> rank_all, xyz_all, crep_all, narrow;
   h->ncell = 0;
-  h->any_narrow = false;
   for (int r = 0; r < nrep; ++r) {
     RepDev& R = h->hrep[r];
     memset(&R, 0, sizeof R);
@@ -826,7 +825,6 @@ static int finalize(pfm_ctx* h) {
     R.clen = make_double3(cl[0], cl[1], cl[2]);
     R.inv_clen = make_double3(1.0 / cl[0], 1.0 / cl[1], 1.0 / cl[2]);
     R.cell_base = h->ncell;
-    h->any_narrow = h->any_narrow || nc[0] < 3 || nc[1] < 3 || nc[2] < 3;
     R.zlo = 0.8 * bx[2];
     R.zhi = 0.9 * bx[2];
     const int ncr = nc[0] * nc[1] * nc[2];
@@ -846,6 +844,7 @@ static int finalize(pfm_ctx* h) {
       rank_all[h->ncell + lin] = h->ncell + k;
       xyz_all[h->ncell + k] = x | (y << 10) | (z << 20);
       crep_all[h->ncell + k] = r;
+      if (narrow_grid(R)) narrow.push_back(h->ncell + k);
     }
     h->ncell += ncr;
   }
@@ -862,6 +861,11 @@ static int finalize(pfm_ctx* h) {
   if (nrep > 1) {
     if ((rc = dalloc(h, &h->cell_rep, h->ncell))) return rc;
     HIPCHK(h, hipMemcpyAsync(h->cell_rep, crep_all.data(), sizeof(int) * h->ncell, hipMemcpyHostToDevice, h->stream));
+  }
+  h->n_narrow = (int)narrow.size();
+  if (h->n_narrow) {
+    if ((rc = dalloc(h, &h->narrow_cells, narrow.size()))) return rc;
+    HIPCHK(h, hipMemcpyAsync(h->narrow_cells, narrow.data(), sizeof(int) * narrow.size(), hipMemcpyHostToDevice, h->stream));
   }
   // rows of every group: replica r owns rows [row0[r], row0[r+1])
   std::vector<int> row0((size_t)(PFM_MAXG + 1) * (nrep + 1), 0);
@@ -891,14 +895,15 @@ static int finalize(pfm_ctx* h) {
       ListDev& L = it.nl[k];
       {
         // One wave per cell only for many cells of few atoms (over the
-        // replicas that hold rows of the list): four lists of a binary gas,
+        // replicas that hold rows of the list, grids under three cells wide
+        // apart, whose cells always take a workgroup each): four lists of a binary gas,
         // wave against workgroup: 3.4 atoms in each of 29,791 cells 71 and
         // 112 us, 7.3 in 2,744 14 and 17, 9.1 in 21,952 103 and 116, 11.4 in
         // 17,576 142 and 123, 13 in 4,913 105 and 44, 5.8 in 343 26 and 9
         // (few waves, each a long chain of dependent steps).
         double atoms = 0.0, cells = 0.0;
         for (int r = 0; r < nrep; ++r) {
-          if (gcnt[L.g1][r] == 0) continue;
+          if (gcnt[L.g1][r] == 0 || narrow_grid(h->hrep[r])) continue;
           atoms += h->rep_n[r];
           cells += (double)h->hrep[r].nc[0] * h->hrep[r].nc[1] * h->hrep[r].nc[2];
         }
@@ -3019,7 +3024,7 @@ int pfm_destroy(pfm_ctx* h) {
   for (auto e : h->rec.free_ev) (void)hipEventDestroy(e);
   auto F = [](void* p) { if (p) (void)hipFree(p); };
   F(h->pos4); F(h->vel4); F(h->frc4); F(h->pos4b); F(h->vel4b); F(h->frc4b); F(h->mask); F(h->maskb);
-  F(h->orig); F(h->origb); F(h->perm); F(h->atom_rank); F(h->scan_tmp); F(h->eb); F(h->qpos); F(h->rdev); F(h->rep); F(h->repb); F(h->cell_rep); F(h->d_rep_row0); F(h->d_rep_out);
+  F(h->orig); F(h->origb); F(h->perm); F(h->atom_rank); F(h->scan_tmp); F(h->eb); F(h->qpos); F(h->rdev); F(h->rep); F(h->repb); F(h->cell_rep); F(h->narrow_cells); F(h->d_rep_row0); F(h->d_rep_out);
   F(h->red_part); F(h->red_out); F(h->derr); F(h->cell_rank); F(h->cell_count); F(h->cell_start); F(h->cell_xyz);
   F(h->nhc_state); F(h->nhc_state0);
   F(h->xfer);

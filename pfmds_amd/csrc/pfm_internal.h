@@ -413,6 +413,8 @@ struct RepDev {
   int cell_base;        // global rank (and linear index) of the grid's first cell
   double zlo, zhi;      // invert_z_velocities band
 };
+// a grid under three cells wide in some direction
+__host__ __device__ __forceinline__ bool narrow_grid(const RepDev& R) { return R.nc[0] < 3 || R.nc[1] < 3 || R.nc[2] < 3; }
 
 // ------------------------------------------------------------- integration
 
@@ -717,7 +719,9 @@ struct pfm_ctx {
   RepDev* rdev = nullptr;             // [nrep]
   int *rep = nullptr, *repb = nullptr;  // [N] replica of every internal atom (batches only)
   int* cell_rep = nullptr;            // [ncell] replica of every cell (batches only)
-  bool any_narrow = false;  // some replica's grid is under three cells wide in some direction
+  // the cells of grids under three cells wide in some direction, and their number
+  int* narrow_cells = nullptr;
+  int n_narrow = 0;
   // per replica and group: first row of the replica in the group's rows
   std::vector<int> rep_row0[PFM_MAXG + 1];
   int* d_rep_row0 = nullptr;  // [(PFM_MAXG + 1) * (nrep + 1)]; slot 0: first internal atom of every replica

@@ -518,6 +518,7 @@ struct SearchArgs {
   const RepDev* rdev;   // replica geometry
   const int* rep;       // replica of every internal atom (null: one replica)
   const int* cell_rep;  // replica of every cell (null: one replica)
+  const int* cells;     // the cells to search (null: all of them)
   const int* bin;       // atoms of the cells in cell order (null: atoms are stored in cell order)
   double rc2, rc2_lo, rc2_hi;
   const int* cell_rank;
@@ -699,10 +700,9 @@ __global__ void k_nn_from_tb(int nrows, const int* __restrict__ rows, const int*
 // image (TileImage), nine more instructions a candidate.  A row-by-row search
 // of such grids, whose candidates wait on two dependent loads each, took 45 us
 // for a 256-atom Cu replica's list.
-// Handles with such a grid take the IMG kernels, which hold both scans and
-// choose by cell (launches of their own for the narrow cells waited on 28 us
+// Handles with such a grid take the IMG kernel, which holds both scans and
+// chooses by cell (launches of their own for the narrow cells waited on 28 us
 // of dependent steps each: a 12-replica batch's step 37.2 -> 33.6 us without).
-__device__ __forceinline__ bool narrow_grid(const RepDev& R) { return R.nc[0] < 3 || R.nc[1] < 3 || R.nc[2] < 3; }
 struct TileImage {
   float3 L, iL;  // box and its inverse in the directions under three cells wide, 0 in the others
   // a value equal on all lanes, in a scalar register
@@ -931,6 +931,7 @@ __global__ void __launch_bounds__(256, CMP || PAIR ? 5 : 6) k_build_tile(SearchA
   __shared__ TileCells tc;
   int c = xcd_block(nblocks_real);
   if (c < 0) return;
+  if (IMG && a.cells) c = a.cells[c];
   const int ncen = a.cell_count[c];
   if (ncen == 0 || !(a.cell_grp[c] & a.g1mem)) return;  // no member of group 1 in the cell
   const RepDev& RG = a.rdev[a.cell_rep ? a.cell_rep[c] : 0];
@@ -1074,7 +1075,7 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int T, bool CMP, bool PAIR, bool QUAD>
+template <int T, bool CMP, bool PAIR, bool QUAD, bool SKIP>
 __global__ void __launch_bounds__(256, 5) k_build_tile_wave(SearchArgs a, const int* __restrict__ rank_xyz,
                                                          const int* __restrict__ row_of, int ncell,
                                                          int nblocks_real) {
@@ -1089,6 +1090,7 @@ __global__ void __launch_bounds__(256, 5) k_build_tile_wave(SearchArgs a, const 
   const int ncen = a.cell_count[c];
   if (ncen == 0 || !(a.cell_grp[c] & a.g1mem)) return;  // no member of group 1 in the cell
   const RepDev& RG = a.rdev[a.cell_rep ? a.cell_rep[c] : 0];
+  if (SKIP && narrow_grid(RG)) return;  // searched by k_build_tile<..., IMG>
   const int cs = a.cell_start[c];
   float4* st = stw[wv];
   const int pk = rank_xyz[c];
@@ -1215,27 +1217,34 @@ __global__ void __launch_bounds__(256, 5) k_build_tile_wave(SearchArgs a, const 
   }
 }
 
-// one list (or with PAIR / QUAD the lists of a pair or two) by the kernel the
-// list takes: one wave per cell (ListDev::wave_cells) or one workgroup, the
-// latter with the nearest-image scan when some grid is under three cells wide
+// One list (or with PAIR / QUAD the lists of a pair or two) by the kernel the
+// list takes: one wave per cell (ListDev::wave_cells) or one workgroup.  With
+// grids under three cells wide among others (a batch), the workgroup kernel
+// searches all cells by its IMG form, and one wave per cell leaves it their
+// cells in a launch of their own: four lists of 27,000 cells of 3.7 atoms
+// beside one box of 256 atoms 81 us a rebuild (118 all one workgroup per cell,
+// 89 all one wave per cell), beside one of 600 dense atoms 103 (141 and 250).
 template <bool PAIR, bool QUAD>
 static void launch_build(pfm_ctx* h, SearchArgs& a, const int* row_of, bool sparse, bool wave_cells) {
   const int nc = h->ncell, nbw = (nc + 3) / 4;
-  const bool narrow = !PAIR && a.nmax <= 8;  // four lanes a row
-#define BUILD_AS(T, CMP)                                                                                           \
-  do {                                                                                                             \
-    if (h->any_narrow)                                                                                             \
-      PFM_LAUNCH(h, "build_list", (k_build_tile<T, CMP, PAIR, QUAD, true>), pad8(nc), 256, a, h->cell_xyz, row_of, \
-                 nc);                                                                                              \
-    else if (wave_cells)                                                                                           \
-      PFM_LAUNCH(h, "build_list", (k_build_tile_wave<T, CMP, PAIR, QUAD>), pad8(nbw), 256, a, h->cell_xyz, row_of, \
-                 nc, nbw);                                                                                         \
-    else                                                                                                           \
-      PFM_LAUNCH(h, "build_list", (k_build_tile<T, CMP, PAIR, QUAD, false>), pad8(nc), 256, a, h->cell_xyz,        \
-                 row_of, nc);                                                                                      \
+  const bool few = !PAIR && a.nmax <= 8;  // four lanes a row
+#define BUILD_TILE(T, CMP, IMG, N)                                                                                  \
+  PFM_LAUNCH(h, "build_list", (k_build_tile<T, CMP, PAIR, QUAD, IMG>), pad8(N), 256, a, h->cell_xyz, row_of, N)
+#define BUILD_WAVE(T, CMP, SKIP)                                                                                    \
+  PFM_LAUNCH(h, "build_list", (k_build_tile_wave<T, CMP, PAIR, QUAD, SKIP>), pad8(nbw), 256, a, h->cell_xyz,       \
+             row_of, nc, nbw)
+#define BUILD_AS(T, CMP)                              \
+  do {                                                \
+    if (wave_cells && h->n_narrow) {                  \
+      BUILD_WAVE(T, CMP, true);                       \
+      a.cells = h->narrow_cells;                      \
+      BUILD_TILE(T, CMP, true, h->n_narrow);          \
+    } else if (wave_cells) BUILD_WAVE(T, CMP, false); \
+    else if (h->n_narrow) BUILD_TILE(T, CMP, true, nc); \
+    else BUILD_TILE(T, CMP, false, nc);               \
   } while (0)
   if constexpr (!PAIR) {
-    if (narrow) {
+    if (few) {
       if (sparse) BUILD_AS(4, true);
       else BUILD_AS(4, false);
       return;
@@ -1244,6 +1253,8 @@ static void launch_build(pfm_ctx* h, SearchArgs& a, const int* row_of, bool spar
   if (sparse) BUILD_AS(8, true);
   else BUILD_AS(8, false);
 #undef BUILD_AS
+#undef BUILD_WAVE
+#undef BUILD_TILE
 }
 
 // Build list k (0-based) of interaction ii.  For lj/ljc/morsec, list 1 is the
