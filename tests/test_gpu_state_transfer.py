@@ -82,3 +82,16 @@ def test_copy_state_around_nvms_blocks():
         np.testing.assert_array_equal(p, q)
         np.testing.assert_array_equal(v, w)
         b.run("nvms", 1.0, 0, 25, True, 1e-30)
+
+
+@pytest.mark.parametrize("n", [64, 5000])
+def test_state_arrays_own_their_memory(n):
+    """A program that keeps the positions of many frames holds no more than
+    those: the three arrays share no block."""
+    s = configs.lj_gas_lattice(n, 0.02, 7, 100.0)
+    c = gpu_ctx(s)
+    a, b = c.state(), c.state()
+    for x in (*a, *b):
+        assert x.flags.owndata and x.base is None and x.shape == (n, 3) and x.flags.c_contiguous
+    for i, x in enumerate((*a, *b)):
+        assert not any(np.shares_memory(x, y) for y in (*a, *b)[i + 1:])
