@@ -2569,8 +2569,10 @@ static const size_t STAGE_CHUNK = 512u << 10;
 static int stage_ready(pfm_ctx* h) {
   if (h->stage) return PFM_OK;
   h->stage_chunk = std::min(STAGE_CHUNK, (72 * (size_t)h->N + 255) / 256 * 256);
+  // the chunks last: a handle that has them has their events too
+  for (auto& e : h->stage_ev)
+    if (!e) HIPCHK(h, hipEventCreateWithFlags(&e, hipEventDisableTiming));
   HIPCHK(h, hipHostMalloc((void**)&h->stage, 2 * h->stage_chunk));
-  for (int k = 0; k < 2; ++k) HIPCHK(h, hipEventCreateWithFlags(&h->stage_ev[k], hipEventDisableTiming));
   return PFM_OK;
 }
 
