@@ -46,7 +46,7 @@ void tim_end(pfm_ctx* h, hipEvent_t a, hipEvent_t b, const char* name) {
 
 struct NhcDev {
   double x[16], v[16], q[16];
-  double s, e, kt, L, T;
+  double e, kt, L, T;
   int M;
   uint32_t bit;
 };
@@ -1098,7 +1098,6 @@ static int finalize(pfm_ctx* h) {
       d.kt = PFM_KB * h->nhc[c].T;
       d.q[0] = h->nhc[c].q1;
       for (int i = 1; i < d.M; ++i) d.q[i] = d.q[0] / (3.0 * h->nhc[c].L);
-      d.s = 1.0;
       d.bit = 1u << (h->nhc[c].group - 1);
     }
     if ((rc = dalloc(h, (NhcDev**)&h->nhc_state, cs.size())) ||
@@ -1844,9 +1843,7 @@ int pfm_create_batch(pfm_ctx** out, int nrep, const int* n_atoms, const double* 
     return rc;
   for (int d = 0; d < 3; ++d) (&h->qscale.x)[d] = 4294967296.0 / boxes[d];
   if (precision == PFM_MIXED && (rc = dalloc(h, &h->qpos, n))) return rc;
-  int dev = 0;
-  HIPCHK(h, hipGetDevice(&dev));
-  HIPCHK(h, hipDeviceGetAttribute(&h->cus, hipDeviceAttributeMultiprocessorCount, dev));
+  h->cus = prop.multiProcessorCount;
   h->lanes = row_lanes(n, precision);
   h->red_blocks = std::max(1, std::min(1024, (n + RED_THREADS - 1) / RED_THREADS));
   // compensated partial rows: an (s, c) pair per block

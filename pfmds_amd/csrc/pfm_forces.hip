@@ -1451,7 +1451,7 @@ static int multi_forces(pfm_ctx* h, bool energy, bool first) {
     MultiArgs A;
     memset(&A, 0, sizeof A);
     int start = 0;
-      for (const auto& ps : ph) {
+    for (const auto& ps : ph) {
       Inter& it = h->inter[ps.inter];
       MultiPass& S = A.s[A.n];
       S.kind = ps.kind;
