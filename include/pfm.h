@@ -88,7 +88,11 @@ int pfm_create(pfm_ctx** h, int n_atoms, const double box[3], const double* pos,
  * are refused in batches (a chain's group would span replicas).  No
  * counterpart in the reference, which runs one system per md() call and farms
  * systems over MPI ranks (run_md_simulation_mpi.f90:68-88); pfm_create is the
- * batch of one. */
+ * batch of one.
+ * A replica's results are those of its own run within rounding, not bit for
+ * bit: the order of its sums follows the handle's lanes per row, which start
+ * by the atoms of the whole handle (pfm_set_tuning), and the order of its list
+ * entries the search that the whole handle's cells lead to. */
 int pfm_create_batch(pfm_ctx** h, int n_rep, const int* n_atoms, const double* boxes,
                      const double* pos, const double* vel, const double* mass, int precision);
 

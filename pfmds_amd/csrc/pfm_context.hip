@@ -764,6 +764,9 @@ static int growth_setup(pfm_ctx* h) {
 // 32,000 37.3 and 37.8, graphene/Cu of 5,088 48.1 and 44.8, 21,040 56.4 and
 // 55.8; mixed gas of 2,000 10.4 and 9.5, 8,000 11.0 and 10.6, 16,000 12.1 and
 // 12.5, crystal of 6,912 16.1 and 15.9, 16,384 18.1 and 18.9.
+// By the handle's atoms, not the replicas': a batch fills the card as one
+// system of its size does.  The sums of a replica of a large batch are then in
+// another order than in its own run unless both are told the same lanes.
 static int row_lanes(int n, int precision) { return n <= (precision == PFM_MIXED ? 8192 : 15000) ? 16 : 8; }
 
 static int finalize(pfm_ctx* h) {

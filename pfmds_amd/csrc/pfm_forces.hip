@@ -253,8 +253,9 @@ struct RowForce {
 // cube, h = L / 2^32 on every axis): the unscaled differences and
 // h^2 (ux^2 + uy^2 + uz^2), two multiplies fewer; dr = h (ux, uy, uz), so
 // a pass that sums c dr sums c u and multiplies the row's sum by h.  The
-// choice is the replica's own, so a replica takes the same arithmetic in a
-// batch as alone.
+// choice is the replica's own, so with the same lanes per row (pfm_set_tuning;
+// row_lanes starts a handle by its atoms) a replica takes the same arithmetic
+// in a batch as alone.
 __device__ __forceinline__ float hiso_of(const RowArgs& a, int i) { return a.rep ? a.rdev[a.rep[i]].hiso : a.hiso; }
 template <bool ISO>
 __device__ __forceinline__ float rjl_d2(const Geo<float>& G, const uint4& a, const uint4& b, float h2, float& dx,
