@@ -103,8 +103,8 @@ template <> struct Geo<float> {
 // versions carry the special cases of their whole domains (denormals,
 // large-argument reduction, division fix-up) into every list entry: the RGL
 // force pass took about 230 vector instructions an entry with them and takes
-// 126 with these, 59.4 -> 43.6 us a launch on 97,556 atoms (density pass
-// 49.6 -> 33.5 us).  These take the arguments the passes produce, without
+// 124 with these, 59.4 -> 42.4 us a launch on 97,556 atoms (density pass
+// 49.6 -> 33.3 us).  These take the arguments the passes produce, without
 // branches; polynomials are interpolations at Chebyshev nodes, the last
 // operation of each is the one that rounds.  None is less accurate than what
 // it stands for; largest errors over 4 million arguments, here and the
@@ -112,7 +112,7 @@ template <> struct Geo<float> {
 // (with its division) 1.49, rcp and sqrt 0.50 both, third and fourth power
 // 0.50 and 1.34; the cosine cutoff's f 2.3 and 2.7 x 2^-53 (RMS 0.39 and
 // 0.51), its derivative 3.9 and 6.4 (0.76 and 1.07).  Forms with fewer
-// instructions (exp 1.13, pow 1.57, cutoff 3.2 and 8.7) took 40.9 and 32.1 us.
+// instructions (exp 1.13, pow 1.57, cutoff 3.2 and 8.7) took 40.1 and 32.0 us.
 namespace f64 {
 // a constant in scalar registers: left to itself the compiler keeps the
 // polynomials' coefficients in vector registers and copies each one before
@@ -288,8 +288,10 @@ __device__ __forceinline__ void cutoff_bl(R r, R R1, R R2, R inv_w, R kdf, R& f,
 struct CutoffHalf {
   double s, t;
   bool lower;
+  // into [0, 1], the instructions' own clamp: 0 on the far sides of both edges
+  static __device__ __forceinline__ double unit(double x) { return fmin(fmax(x, 0.0), 1.0); }
   __device__ __forceinline__ CutoffHalf(double r, double R1, double R2, double hw) {
-    const double a = fmax((r - R1) * hw, 0.0), b = fma(R2 - r, hw, 0x1.d1a62633145c0p-50);
+    const double a = unit((r - R1) * hw), b = unit(fma(R2 - r, hw, 0x1.d1a62633145c0p-50));
     lower = a < b;
     t = fmin(a, b);
     s = f64::sin_q1(t);
