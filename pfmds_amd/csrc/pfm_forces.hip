@@ -583,7 +583,7 @@ struct TbP {
 // A row's time is its chain of dependent loads and functions.  Registers for
 // one bond a lane instead of arrays for four, loads ahead of the arithmetic
 // and the branch-free functions took the force pass of 24,960 atoms from 10.6
-// to 7.7 us in FP64 (205 -> 139 VGPRs) and 8.1 to 6.4 mixed.  Eight and
+// to 7.9 us in FP64 (205 -> 139 VGPRs) and 8.1 to 6.4 mixed.  Eight and
 // sixteen lanes a row (two and four for each bond's sums) shortened small
 // systems (1,664 atoms, FP64: 13.4 -> 10.4 and 8.6 us) but cost more work on
 // large ones, where these rows share a launch (30.0 -> 32.6 and 36.3 us).
@@ -820,10 +820,11 @@ struct CosP {
 };
 
 // x**delt, x >= 0.  FP64: whole exponents up to 4 by products, the third and
-// fourth power from the square in two parts (0.50 ulp); the general power is 60 of the 190 instructions an entry takes
-// (graphene pass of 24,960 rows 20.0 -> 16.5 us, metal rows 25.6 -> 19.6 with
-// 1/|n| kept beside the normal; with the library's functions 30.1 and 38.5).
-// The mixed path's power is two transcendental instructions for any exponent.
+// fourth power from the square in two parts (0.50 ulp); the general power is
+// about a third of an entry's instructions (the graphene pass of 24,960 rows
+// takes 17.3 us and the metal rows 19.2, some 3.5 and 6 more with it; with the
+// library's functions 30.1 and 38.2).  The mixed path's power is two
+// transcendental instructions for any exponent.
 template <class R>
 __device__ __forceinline__ R cos_power(const CosP& P, R x) {
   if constexpr (sizeof(R) == 8) {
